@@ -440,8 +440,7 @@ int upload_mat(const HostCsr &h, int prec, int index_mode, Mat &M) {
 // in the matrix precision; inv_diag is taken from A (not owned).  Each row's list is
 // padded to a multiple of KB entries (at least KB) with column = the block's end and
 // value +0: the sweep kernel reads a zero x there, so a pad subtracts +0 * +0 = +0 from
-// the row sum, which leaves every value (-0 included) unchanged.  KB (3 or 4) is the width
-// that needs fewer pads.
+// the row sum, which leaves every value (-0 included) unchanged.
 // The entries of each row i outside its core block [lo, lo + B), lo = (i / B) * B, in
 // stored order: b - (this matrix) x sums the products of the off-block residual of hybrid
 // GS (csr_gs.inl:75-130, the columns outside the calling core's rows) in their order.
@@ -474,12 +473,19 @@ int upload_core(const HostCsr &h, int64_t B, int prec, const Mat &A, Mat &M) {
         nreal += cnt[i];
     }
     auto padded = [](int64_t c, int kb) { return std::max<int64_t>(kb, (c + kb - 1) / kb * kb); };
-    int64_t tot3 = 0, tot4 = 0;
-    for (int64_t i = 0; i < n; ++i) {
-        tot3 += padded(cnt[i], 3);
-        tot4 += padded(cnt[i], 4);
+    // KB: the width whose rows take the least time in the sweep's serial chain, a batch
+    // costing one LDS round trip (about as long as 12 subtractions) and its KB subtractions
+    int KB = 3;
+    int64_t best = -1;
+    for (int kb : {3, 4, 6, 8}) {
+        int64_t cost = 0;
+        for (int64_t i = 0; i < n; ++i)
+            cost += padded(cnt[i], kb) / kb * (12 + kb);
+        if (best < 0 || cost < best) {
+            best = cost;
+            KB = kb;
+        }
     }
-    const int KB = tot3 < tot4 ? 3 : 4;
     std::vector<uint32_t> row(n + 1, 0), col;
     std::vector<double> val;
     for (int64_t i = 0; i < n; ++i) {

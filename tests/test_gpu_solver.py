@@ -239,6 +239,28 @@ def test_hsgs_core_path_bit_exact(gpu, O, mg_prec):
     assert f"k_hsgs_core<{'double' if mg_prec == 0 else 'float'},{nv}>" in names, names
 
 
+@pytest.mark.parametrize("N,nv,mg_prec,block_rows", [
+    (32, 4, 0, 64),   # 64 lanes' worth of blocks does not fit in LDS: fewer blocks per wave
+    (9, 1, 2, 64),    # a last block of a few rows, one lane per block
+    (48, 2, 0, 8),    # 6912 blocks: several per wave, the last wave part filled
+    (24, 64, 2, 40),  # one block per wave
+    (20, 16, 0, 8),   # blocks shorter than a prefetch of 16 rows
+])
+def test_hsgs_blocks_per_wave_bit_exact(gpu, O, N, nv, mg_prec, block_rows):
+    X = gpu
+    levels = levels_for(X, N)
+    prm = X.default_params(method="MergedPBiCGStab", smoother="HSGS", sweeps=1, mg_prec=mg_prec)
+    prm.hsgs_block_rows = block_rows
+    S = X.Solver(X.Hier(levels), prm, nv)
+    b = X.rhs_uniform(11, N ** 3, nv)
+    db, dx = X.DeviceArray.from_host(b), X.DeviceArray(N ** 3 * nv)
+    S.precond_apply(db, dx)
+    assert np.array_equal(dx.to_host(), O.mg_apply(O.Hier(levels), O.params_from(prm), nv, b))
+    dx.zero()
+    names = {k["kernel"] for k in S.profile(db, dx, 1)}
+    assert f"k_hsgs_core<{'double' if mg_prec == 0 else 'float'},{nv}>" in names, names
+
+
 def test_graph_and_eager_are_identical(gpu):
     X = gpu
     N, nv = 24, 8
