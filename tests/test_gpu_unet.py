@@ -65,6 +65,34 @@ def test_loss_and_gradients_match_oracle(gpu, channels, size, batch):
         assert np.linalg.norm(gg - rr) <= 3e-2 * np.linalg.norm(rr) + 1e-9, sl
 
 
+@pytest.mark.parametrize("channels,dims", [
+    ((16, 32, 48, 64), (3, 8, 16, 24)),  # levels down to 1 x 2 x 3 voxels, several samples
+    ((64,), (1, 5, 3, 7)),               # one level, no edge a power of two
+    ((48, 16), (2, 6, 10, 34)),          # lines just over a box edge, 16 -> 48 upsampling
+    ((32, 64), (1, 2, 2, 66)),
+])
+def test_gradients_on_ragged_volumes(gpu, channels, dims):
+    # the weight gradient's boxes overhang these volumes.  Bound: bf16 operands (2^-9 each,
+    # two per product) and activations rounded once per layer give about 1e-2 per tensor,
+    # the bar of the test above
+    X = gpu
+    net = X.UNet(channels, seed=3)
+    rng = np.random.default_rng(2)
+    p = net.get_params()
+    for sl in layer_slices(channels)[1::2]:
+        p[sl] = rng.standard_normal(sl.stop - sl.start).astype(np.float32) * 0.1
+    net.set_params(p)
+    x = rng.standard_normal(dims).astype(np.float32)
+    t = rng.standard_normal(dims).astype(np.float32)
+    loss, g, y = net.loss_grad(x, t)
+    ref = UO.UNet(channels, p.astype(np.float64))
+    rloss, rg, ry = ref.loss_grad(x.astype(np.float64), t.astype(np.float64), use_bf16=True)
+    assert abs(loss - rloss) <= 1e-3 * rloss
+    assert np.linalg.norm(y - ry) <= 1e-2 * np.linalg.norm(ry)
+    for sl in layer_slices(channels):
+        assert np.linalg.norm(g[sl] - rg[sl]) <= 3e-2 * np.linalg.norm(rg[sl]) + 1e-9, sl
+
+
 def test_training_and_solver_from_learned_x0(gpu):
     X = gpu
     N, nv = 32, 8
