@@ -481,7 +481,8 @@ void jacobi_update(int64_t n, int nv, int prec, void *x, const void *b, const vo
 void hsgs_sweeps(const Mat &A, int nv, const void *t, void *x, int x_zero, double relax,
                  int64_t blk_rows, const int *done, hipStream_t s);
 int64_t hsgs_block_rows(int64_t n, int nblocks);
-void dense_matvec(int64_t n, int nv, int prec, const void *D, const void *x, void *y,
+// y = D x; prec: precision of D and of the sums, xprec: of x and y (F64, or prec)
+void dense_matvec(int64_t n, int nv, int prec, int xprec, const void *D, const void *x, void *y,
                   const int *done, hipStream_t s);
 void convert(int64_t count, int from_prec, const void *src, void *dst, const int *done,
              hipStream_t s);

@@ -686,7 +686,6 @@ struct Level {
     void *sr = nullptr, *su1 = nullptr, *su2 = nullptr;
     void *dinv = nullptr;
     int dinv_prec = F64;
-    void *cb64 = nullptr, *cx64 = nullptr; // fp64 coarse solve in an fp32 hierarchy
     std::vector<double> cheb_pre, cheb_post, cheb_coarse;
 };
 
@@ -837,13 +836,7 @@ void smooth(xh_solver_s *S, const xh_role &role, Level &L, const std::vector<dou
         return;
     }
     case XH_DIRECT: {
-        if (L.cb64) {
-            convert(L.n * nv, F32, b, L.cb64, S->dflag, st);
-            dense_matvec(L.n, nv, F64, L.dinv, L.cb64, L.cx64, S->dflag, st);
-            convert(L.n * nv, F64, L.cx64, x, S->dflag, st);
-        } else {
-            dense_matvec(L.n, nv, L.dinv_prec, L.dinv, b, x, S->dflag, st);
-        }
+        dense_matvec(L.n, nv, L.dinv_prec, L.prec, L.dinv, b, x, S->dflag, st);
         return;
     }
     case XH_IDENTITY:
@@ -1452,7 +1445,7 @@ int xh_spmv_timed(xh_matrix A, int nv, const void *dx, void *dy, int accumulate,
 int xh_dense_matvec(int64_t n, int nv, int prec, const void *dD, const void *dx, void *dy) {
     if (n <= 0 || !nv_ok(nv) || !dD || !dx || !dy)
         return fail(XH_EINVAL, "xh_dense_matvec: bad arguments");
-    dense_matvec(n, nv, prec, dD, dx, dy, nullptr, g_stream);
+    dense_matvec(n, nv, prec, prec, dD, dx, dy, nullptr, g_stream);
     XH_HIP(hipGetLastError());
     XH_HIP(hipStreamSynchronize(g_stream));
     return 0;
@@ -1657,12 +1650,8 @@ int xh_solver_create(xh_hier H, const xh_params *prm, int nv, xh_solver *out) {
             if (nc > 8192)
                 return bail(fail(XH_EINVAL, "Direct coarse solve on a level larger than 8192"));
             C.dinv_prec = C.prec;
-            if (mg && mp == 2 && prm->coarse_fp64) {
+            if (mg && mp == 2 && prm->coarse_fp64)
                 C.dinv_prec = F64;
-                if ((rc = alloc_vec(S, (double **)&C.cb64, (size_t)nc * nv)) ||
-                    (rc = alloc_vec(S, (double **)&C.cx64, (size_t)nc * nv)))
-                    return bail(rc);
-            }
             if (C.dinv_prec == F64) {
                 std::vector<double> dense((size_t)nc * nc, 0.0), inv;
                 for (int64_t i = 0; i < nc; ++i)
@@ -1884,7 +1873,7 @@ int xh_solver_destroy(xh_solver S) {
         free_mat(L.off);
         free_mat(L.P);
         free_mat(L.R);
-        for (void *q : {L.tmp, L.tmp_t, L.b, L.x, L.sr, L.su1, L.su2, L.dinv, L.cb64, L.cx64})
+        for (void *q : {L.tmp, L.tmp_t, L.b, L.x, L.sr, L.su1, L.su2, L.dinv})
             if (q)
                 (void)hipFree(q);
     }

@@ -278,24 +278,98 @@ __global__ __launch_bounds__(kBlock) void k_jacobi(int64_t count, int nv, VT *__
     }
 }
 
-template <typename VT>
-__global__ __launch_bounds__(kBlock) void k_dense(int64_t n, int nv, const VT *__restrict__ D,
-                                                  const VT *__restrict__ x,
-                                                  VT *__restrict__ y,
-                                                  const int *__restrict__ done) {
+// y = D x, D dense n x n (the coarsest level's inverse, n of a few hundred): every output is
+// a sum of n terms added one by one in column order (the rounding of dense_Ax_y), so the
+// time cannot go below n dependent adds; what is left to hide is memory.  A workgroup owns
+// RB rows and all NV right-hand sides (one output per thread) and walks the columns in
+// tiles of TJ: D and x tiles go through double-buffered LDS, loaded NS tiles ahead into
+// registers, all threads loading contiguous rows.  A small product runs two waves per
+// workgroup, spread over the CUs; a large one shares each x tile among four.  One output
+// per thread reading memory itself waited for a load round trip every 16 terms: n = 500,
+// nv = 32, fp64: 23.7 us; here 12.8 (four waves and two tiles ahead: 13.8), of which the 500
+// dependent adds behind their LDS reads take about 5.  XT: type of x and y in memory
+// (float with a double D: the fp64 coarse solve of an fp32 hierarchy, each value converted
+// once as a separate pass would).
+template <int NV, int WV>
+struct DenseShape {
+    static constexpr int T = 64 * WV; // threads
+    static constexpr int RB = T / NV < 32 ? T / NV : 32; // rows
+};
+template <typename VT, typename XT, int NV, int WV>
+__global__ __launch_bounds__(64 * WV) void k_dense(int64_t n, const VT *__restrict__ D,
+                                                   const XT *__restrict__ x, XT *__restrict__ y,
+                                                   const int *__restrict__ done) {
     if (done != nullptr && *done)
         return;
-    const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (e >= n * nv)
-        return;
-    const int64_t i = e / nv;
-    const int k = (int)(e % nv);
+    constexpr int RB = DenseShape<NV, WV>::RB, T = 64 * WV, TJ = 64, NS = 4;
+    constexpr int DS = TJ + 16 / (int)sizeof(VT); // padded D row: 16-byte aligned, spread banks
+    constexpr int PX = (TJ * NV + T - 1) / T, PD = (RB * TJ + T - 1) / T;
+    __shared__ __align__(16) VT sx[2][TJ * NV];
+    __shared__ __align__(16) VT sd[2][RB * DS];
+    const int tid = threadIdx.x;
+    const int64_t i0 = (int64_t)blockIdx.x * RB;
+    const int r = tid / NV, k = tid % NV; // the thread's output (threads past RB rows have none)
+    VT rx[NS][PX], rd[NS][PD];
+    // tile loads, clamped into the arrays: entries past column n - 1 or row n - 1 are
+    // never used
+    auto load = [&](int64_t j0, VT (&ax)[PX], VT (&ad)[PD]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < PX; ++u) {
+            const int64_t e = j0 * NV + tid + u * T;
+            ax[u] = (VT)x[e < n * NV ? e : n * NV - 1];
+        }
+#pragma unroll
+        for (int u = 0; u < PD; ++u) {
+            const int e = tid + u * T, row = e / TJ, c = e % TJ;
+            const int64_t i = i0 + row < n ? i0 + row : n - 1;
+            const int64_t j = j0 + c < n ? j0 + c : n - 1;
+            ad[u] = D[i * n + j];
+        }
+    };
+    auto store = [&](int b, const VT (&ax)[PX], const VT (&ad)[PD]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < PX; ++u)
+            if (TJ * NV % T == 0 || tid + u * T < TJ * NV)
+                sx[b][tid + u * T] = ax[u];
+#pragma unroll
+        for (int u = 0; u < PD; ++u) {
+            const int e = tid + u * T;
+            if (RB * TJ % T == 0 || e < RB * TJ)
+                sd[b][(e / TJ) * DS + e % TJ] = ad[u];
+        }
+    };
     VT acc = VT(0);
-    // j order as dense_Ax_y; unrolled so that many loads are in flight
+    const bool mine = r < RB && i0 + r < n;
+    auto tile = [&](int b, int64_t j0) __attribute__((always_inline)) {
+        const VT *px = sx[b] + k, *pd = sd[b] + (r < RB ? r : 0) * DS;
+        const int m = (int)(n - j0 < TJ ? n - j0 : TJ);
+        if (m == TJ) {
 #pragma unroll 16
-    for (int64_t j = 0; j < n; ++j)
-        acc = acc + D[i * n + j] * x[j * nv + k];
-    y[e] = acc;
+            for (int j = 0; j < TJ; ++j)
+                acc = acc + pd[j] * px[j * NV];
+        } else {
+            for (int j = 0; j < m; ++j)
+                acc = acc + pd[j] * px[j * NV];
+        }
+    };
+#pragma unroll
+    for (int q = 0; q < NS; ++q)
+        load((int64_t)q * TJ, rx[q], rd[q]);
+    for (int64_t j0 = 0; j0 < n; j0 += NS * TJ) {
+#pragma unroll
+        for (int q = 0; q < NS; ++q) {
+            // an LDS buffer is written two tiles after its last reads, which the barrier
+            // of the tile between them has ordered
+            if (j0 + q * TJ < n) { // uniform
+                store(q & 1, rx[q], rd[q]);
+                load(j0 + (int64_t)(q + NS) * TJ, rx[q], rd[q]);
+                __syncthreads();
+                tile(q & 1, j0 + (int64_t)q * TJ);
+            }
+        }
+    }
+    if (mine)
+        y[(i0 + r) * NV + k] = (XT)acc;
 }
 
 template <typename T1, typename T2>
@@ -488,22 +562,53 @@ void jacobi_update(int64_t n, int nv, int prec, void *x, const void *b, const vo
                            (const float *)inv_diag, (float)relax, x_zero, done);
 }
 
-void dense_matvec(int64_t n, int nv, int prec, const void *D, const void *x, void *y,
+template <typename VT, typename XT, int NV>
+void dense_t(int64_t n, const void *D, const void *x, void *y, const int *done, hipStream_t s) {
+    // two waves per workgroup while that gives at most 2 workgroups per CU
+    constexpr int R1 = DenseShape<NV, 2>::RB, R4 = DenseShape<NV, 4>::RB;
+    if (R1 == R4 || (n + R1 - 1) / R1 <= 512)
+        hipLaunchKernelGGL((k_dense<VT, XT, NV, 2>), dim3((unsigned)((n + R1 - 1) / R1)), dim3(128),
+                           0, s, n, (const VT *)D, (const XT *)x, (XT *)y, done);
+    else
+        hipLaunchKernelGGL((k_dense<VT, XT, NV, 4>), dim3((unsigned)((n + R4 - 1) / R4)), dim3(256),
+                           0, s, n, (const VT *)D, (const XT *)x, (XT *)y, done);
+}
+
+template <typename VT, typename XT>
+void dense_nv(int64_t n, int nv, const void *D, const void *x, void *y, const int *done,
+              hipStream_t s) {
+    switch (nv) {
+    case 1:
+        return dense_t<VT, XT, 1>(n, D, x, y, done, s);
+    case 2:
+        return dense_t<VT, XT, 2>(n, D, x, y, done, s);
+    case 4:
+        return dense_t<VT, XT, 4>(n, D, x, y, done, s);
+    case 8:
+        return dense_t<VT, XT, 8>(n, D, x, y, done, s);
+    case 16:
+        return dense_t<VT, XT, 16>(n, D, x, y, done, s);
+    case 32:
+        return dense_t<VT, XT, 32>(n, D, x, y, done, s);
+    default:
+        return dense_t<VT, XT, 64>(n, D, x, y, done, s);
+    }
+}
+
+void dense_matvec(int64_t n, int nv, int prec, int xprec, const void *D, const void *x, void *y,
                   const int *done, hipStream_t s) {
-    const int64_t count = n * nv;
-    const int grid = (int)((count + kBlock - 1) / kBlock);
     LedgerScope led(s);
     if (led.on) {
-        const double sv = prec == F64 ? 8.0 : 4.0;
-        led.kernel = std::string("k_dense<") + prec_name(prec) + ">";
-        led.bytes = sv * (double)(n * n + 2 * count); // D, x, y
+        const double sv = prec == F64 ? 8.0 : 4.0, sx = xprec == F64 ? 8.0 : 4.0;
+        led.kernel = std::string("k_dense<") + prec_name(prec) + "," + prec_name(xprec) + ">";
+        led.bytes = sv * (double)(n * n) + 2.0 * sx * (double)(n * nv); // D, x, y
     }
-    if (prec == F64)
-        hipLaunchKernelGGL(k_dense<double>, dim3(grid), dim3(kBlock), 0, s, n, nv,
-                           (const double *)D, (const double *)x, (double *)y, done);
+    if (prec == F64 && xprec == F64)
+        dense_nv<double, double>(n, nv, D, x, y, done, s);
+    else if (prec == F64)
+        dense_nv<double, float>(n, nv, D, x, y, done, s);
     else
-        hipLaunchKernelGGL(k_dense<float>, dim3(grid), dim3(kBlock), 0, s, n, nv,
-                           (const float *)D, (const float *)x, (float *)y, done);
+        dense_nv<float, float>(n, nv, D, x, y, done, s);
 }
 
 void convert(int64_t count, int from_prec, const void *src, void *dst, const int *done,

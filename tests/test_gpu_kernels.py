@@ -160,6 +160,26 @@ def test_dense_matvec_bit_exact(gpu, O):
     assert np.array_equal(dy.to_host(), y)
 
 
+@pytest.mark.parametrize("n,nv", [(1, 1), (33, 1), (63, 2), (64, 4), (65, 8), (129, 16),
+                                  (200, 32), (7, 64), (191, 64),
+                                  (1100, 32), (530, 64), (700, 1)])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_dense_matvec_tile_edges_bit_exact(gpu, n, nv, prec):
+    # sums in column order with separate multiply and add, at the edges of the row blocks
+    # (1 to 32 rows), of the 64-column tiles (one, even and odd tile counts) and of the
+    # two-wave and four-wave variants
+    X = gpu
+    rng = np.random.default_rng(n + nv)
+    dt = np.float64 if prec == 0 else np.float32
+    D, x = rng.standard_normal((n, n)).astype(dt), rng.standard_normal((n, nv)).astype(dt)
+    y = np.zeros((n, nv), dt)
+    for j in range(n):
+        y = y + D[:, j:j + 1] * x[j]
+    dD, dx, dy = (X.DeviceArray.from_host(a.ravel()) for a in (D, x, np.zeros((n, nv), dt)))
+    X.check(X.hip().xh_dense_matvec(n, nv, prec, dD.ptr, dx.ptr, dy.ptr), "xh_dense_matvec")
+    assert np.array_equal(dy.to_host(), y.ravel())
+
+
 def test_spmv_full_size_cube_128(gpu, O):
     # the benchmark operator at full size: 2,097,152 rows, u16 panel columns, nv = 32
     X = gpu
