@@ -161,10 +161,15 @@ int xh_spmv_schedule(int64_t nrows, int64_t nnz, int64_t fold, int prec, int nv,
  * setup: a hybrid GS level also keeps the entries outside each row's core block as a
  * matrix of their own and computes the off-block residual as b - (that matrix) x,
  * bit-identical to skipping the in-block columns of A), "spmv_wide_batches" (0/1,
- * default 1: SpMVs at nv 8 and 32 over matrices of few rows and 32 or more entries per row
- * on average, at most 512 workgroups, issue 16 x loads per batch instead of 8; the sums
- * and their order are unchanged),
- * "spmv_grid_min_seg" (default 32), "unet_fuse_up" (0/1, default 1: U-Net inference reads
+ * default 1: SpMVs over few rows of many entries load more than 8 entries of a row at
+ * once: a whole row, see "spmv_wave_enable", or, at nv 8 and 32 where that is not the faster
+ * one, 32 or more entries per row on average and at most 512 workgroups, 16; the sums and
+ * their order are unchanged),
+ * "spmv_wave_enable" (SpMVs over few rows of many entries, the coarse levels of a
+ * hierarchy, load a whole row at once over the lanes of a wave: 0 never, 1
+ * wherever the kernel can run, 2 = default: where it is the faster one; sums and their
+ * order unchanged),
+ * "spmv_grid_min_seg" (default 32), "unet_fuse_up" (0/1, default 1: the U-Net reads
  * the decoder's upsampled inputs through the convolution instead of writing them),
  * "unet_conv_tile" (0/1, default 1: forward convolutions with 16 or 32 output channels
  * on volumes of w % 64 == h % 4 == d % 2 == 0, and with 48 on w % 32 == 0, read their

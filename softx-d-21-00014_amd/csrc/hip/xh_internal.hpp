@@ -199,8 +199,12 @@ struct Tuning {
     // their own (built at setup) and run the off-block residual as an OP_RESID over it
     // (grid path for 27-point operators); 0: OP_OFFBLOCK over A, skipping in-block columns
     int hsgs_off_csr = 1;
-    // 1: few-row, long-row SpMVs (nv 8 and 32) issue 16 x loads per batch (k_spmv<..., 16>)
+    // 1: few-row, long-row SpMVs load more than 8 entries of a row at once: k_spmv_wave by its
+    // rule, and k_spmv<..., 16> (nv 8 and 32) where that does not apply
     int wide_batches = 1;
+    // the kernel for few, long rows (k_spmv_wave): 0 never, 1 wherever it can run, 2 (default)
+    // by the rule at takes_wave
+    int wave_enable = 2;
     int grid_items = 2048;          // target work items (tile x segment) per launch
     int grid_min_seg = 32;          // shortest x segment of a work item
     // 1: matrices with a complete 7-point stencil view run the register-window line
@@ -307,6 +311,11 @@ struct SpmvArgs {
     int grid_cap = 0;           // 0: default
 };
 
+// the kernel for few, long rows (xh_spmv_wave.hip) and whether op on A takes it
+bool takes_wave(const Mat &A, SpmvOp op, int nv);
+int wave_entries(const Mat &A, int nv); // entries of a row it loads side by side
+void spmv_wave(const Mat &A, int nv, const void *x, void *y, SpmvOp op, const SpmvArgs &a,
+               hipStream_t s);
 // returns the number of partial blocks written (DOT ops) or 0
 int spmv(const Mat &A, int nv, const void *x, void *y, SpmvOp op, const SpmvArgs &a,
          hipStream_t s);

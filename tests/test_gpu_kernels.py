@@ -180,6 +180,59 @@ def test_dense_matvec_tile_edges_bit_exact(gpu, n, nv, prec):
     assert np.array_equal(dy.to_host(), y.ravel())
 
 
+@pytest.mark.parametrize("nv", NVS)
+@pytest.mark.parametrize("prec", [0, 1])
+def test_spmv_long_row_kernel_bit_exact(gpu, O, nv, prec):
+    # the kernel that loads a whole row at once, at row lengths around its batches of 8, its
+    # passes of 32 and 64 entries and an empty row, u32 and u16 columns, set and add
+    X = gpu
+    rng = np.random.default_rng(nv)
+    lens = [0, 1, 7, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65, 129, 200, 0, 5]
+    n, m = len(lens), 700
+    row = np.concatenate(([0], np.cumsum(lens))).astype(np.uint32)
+    col = np.concatenate([rng.choice(m, k, replace=False) for k in lens]).astype(np.uint32)
+    val = rng.standard_normal(len(col))
+    dt = np.float64 if prec == 0 else np.float32
+    x, y0 = rng.standard_normal(m * nv).astype(dt), rng.standard_normal(n * nv).astype(dt)
+    dx = X.DeviceArray.from_host(x)
+    X.set_option("spmv_wave_enable", 1)
+    try:
+        for index_mode in (1, 2):
+            A = X.Matrix(row, col, val, prec=prec, index_mode=index_mode, ncols=m)
+            for add in (False, True):
+                dy = X.DeviceArray.from_host(y0)
+                A.spmv(nv, dx, dy, accumulate=add)
+                ref = O.spmv(row, col, val, x, nv, y=y0 if add else None, ncols=m, f32=prec == 1)
+                assert np.array_equal(dy.to_host(), ref), (index_mode, add)
+    finally:
+        X.set_option("spmv_wave_enable", 2)
+
+
+@pytest.mark.parametrize("smoother,nv,mg_prec", [("Chebyshev", 1, 0), ("Chebyshev", 8, 2),
+                                                 ("Chebyshev", 32, 1), ("Jacobi", 4, 0),
+                                                 ("HSGS", 2, 2), ("Chebyshev", 64, 0)])
+def test_long_row_kernel_in_a_vcycle_is_identical(gpu, smoother, nv, mg_prec):
+    # every V-cycle operation that can take it (residuals stored in fp32, Chebyshev steps
+    # from zero and non-zero x, prolongation), against the row-parallel kernel
+    X = gpu
+    N = 20
+    row, col, val = X.cube(N)
+    levels = X.Amg(row, col, val, agg_num_levels=1, num_paths=2, coarse_size=60).export()
+    prm = X.default_params(smoother=smoother, poly_order=4, mg_prec=mg_prec)
+    S = X.Solver(X.Hier(levels), prm, nv)
+    db = X.DeviceArray.from_host(X.rhs_uniform(3, N ** 3, nv))
+    out = {}
+    try:
+        for on in (0, 1, 2):
+            X.set_option("spmv_wave_enable", on)
+            dx = X.DeviceArray(N ** 3 * nv)
+            S.precond_apply(db, dx)
+            out[on] = dx.to_host()
+    finally:
+        X.set_option("spmv_wave_enable", 2)
+    assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
+
+
 def test_spmv_full_size_cube_128(gpu, O):
     # the benchmark operator at full size: 2,097,152 rows, u16 panel columns, nv = 32
     X = gpu
