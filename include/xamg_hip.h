@@ -115,8 +115,9 @@ int xh_matrix_fold(xh_matrix A, int64_t set, int64_t *fold);
 /* Structured-grid view of a square matrix (set at upload when it applies): rows are the
  * points of an nx x ny x nz grid in natural order (row = (z*ny + y)*nx + x) and every
  * entry couples grid neighbours (|dx|, |dy|, |dz| <= 1; 7- and 27-point operators).  Such
- * a matrix runs the SpMV as a sweep along x over tiles of grid lines with the x rows of
- * the tile and its halo lines staged in LDS.  No reference counterpart (the reference's csr_Ax_y is row-parallel, src/blas2/
+ * a matrix can run the SpMV on 1-byte neighbour codes instead of column indices, or as a
+ * sweep along x over tiles of grid lines with the x rows of the tile and its halo lines
+ * staged in LDS ("spmv_grid_enable").  No reference counterpart (the reference's csr_Ax_y is row-parallel, src/blas2/
  * detail/csr_matvec.inl:149-260); the arithmetic is that of the row-parallel kernel.
  * xh_matrix_grid: dims = {nx, ny, nz}, zeros when the matrix has no grid view.
  * xh_csr_grid: the same detection on a host CSR; code
@@ -152,9 +153,11 @@ int xh_spmv_schedule(int64_t nrows, int64_t nnz, int64_t fold, int prec, int nv,
  * of a launch that writes dot-product partials), "grid_dot_groups" (default 2048: the same
  * for the structured-grid SpMV), "vec_dot_groups" (default 2048: the same for the fused
  * vector updates), "spmv_fold_enable" (0/1), "spmv_fold_min_bytes" (default 2 MiB: fold only
- * when 2*fold*nv*sizeof(value) exceeds it), "spmv_grid_enable" (the
- * structured-grid SpMV of matrices with a grid view: 0 never, 1 always, 2 = default: when
- * the rows average 12 or more entries, e.g. 27-point operators), "spmv_grid_items" (default 2048),
+ * when 2*fold*nv*sizeof(value) exceeds it), "spmv_grid_enable" (matrices
+ * with a grid view: 1 always the LDS-window line sweep; 2 = default: when the rows average
+ * 12 or more entries, e.g. 27-point operators, the row-parallel kernel reads 1-byte
+ * neighbour codes instead of columns, and the largest fp64 SpMMs with dot partials run the
+ * sweep; 0 neither), "spmv_grid_items" (default 2048),
  * "cheb_fuse_zero" (0/1, default 1: a Chebyshev smoother from a zero x runs its first two
  * steps as one SpMV that gathers b and forms the first step's values per entry,
  * bit-identical to two launches), "hsgs_offblock_csr" (0/1, default 1, read at solver

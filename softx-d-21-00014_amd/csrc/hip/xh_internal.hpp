@@ -168,7 +168,8 @@ int64_t csr_fold(int64_t nrows, int64_t ncols, const uint32_t *row, const uint32
                  int64_t min_fold);
 
 // Launch-shape knobs (xh_set_option)
-// rows of at least this many entries on average take the structured-grid SpMV by default
+// rows of at least this many entries on average make a matrix with a grid view read its
+// neighbour codes
 constexpr int64_t kGridMinRowNnz = 12;
 
 struct Tuning {
@@ -186,10 +187,8 @@ struct Tuning {
     int vec_dot_groups = 2048;
     int fold_enable = 1;            // 0: always contiguous order
     int64_t fold_min_bytes = 2 << 20; // fold only when 2*fold*nv*sizeof(value) exceeds this
-    // structured-grid matrices run the LDS-window line sweep (k_spmv_grid): 0 never, 1
-    // always, 2 (default) when rows average at least kGridMinRowNnz entries.  The 7-point
-    // cube at 128^3 only matches the row-parallel kernel at nv = 32 (slower at other nv
-    // and in fp32); the 27-point operator at 96^3 gains 10-20 %
+    // structured-grid matrices: 0 columns, 1 the LDS-window line sweep always, 2 (default) by
+    // the rules at takes_codes and takes_sweep
     int grid_enable = 2;
     int grid_dot_groups = 2048;     // work items of a grid-path launch that writes partials
     // 1: a Chebyshev smoother from a zero x runs its first two steps as one SpMV
@@ -214,12 +213,6 @@ struct Tuning {
     int st7_min_seg = 32;           // shortest x segment of a work item
 };
 extern Tuning g_tune;
-
-// whether the structured-grid SpMV takes a matrix that has a grid view (spmv_grid_enable)
-inline bool grid_on(const Mat &A) {
-    return g_tune.grid_enable == 1 ||
-           (g_tune.grid_enable == 2 && A.nnz >= kGridMinRowNnz * A.nrows);
-}
 
 // ---- launch accounting (xh_solver_profile) ----
 // While a profile solve runs, every launch helper of the solve path brackets its kernel

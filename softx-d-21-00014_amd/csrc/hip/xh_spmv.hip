@@ -55,12 +55,25 @@ struct Chunk {
     VT d[E];       // SCALE loads: the scale of the entry's column (sd[base + c])
 };
 
+// Column of an entry relative to the row's base: the stored index, or for a grid code
+// (GridCol: 9(dz+1) + 3(dy+1) + (dx+1), base = the row) the offset dz*F + dy*nx + dx,
+// modulo 2^32.  The divisions by 9 and 3 are exact for codes below 27.
+template <typename IT>
+__device__ __forceinline__ uint32_t column(IT v, int nx, int F) {
+    if constexpr (std::is_same<IT, GridCol>::value) {
+        const int cd = v.code, a = (cd * 57) >> 9, r = cd - 9 * a, b = (r * 11) >> 5, d = r - 3 * b;
+        return (uint32_t)((a - 1) * F + (b - 1) * nx + (d - 1));
+    } else {
+        return (uint32_t)v;
+    }
+}
+
 // SCALE: also the column's scale sd[base + c] of each loaded entry (a load that depends on
 // the column's), broadcast with the column and value
 template <typename VT, typename IT, int NV, int W, bool SCALE = false, int BX = 8>
 __device__ __forceinline__ void load_chunk(uint32_t j, uint32_t e, const IT *__restrict__ col,
                                            const VT *__restrict__ val,
-                                           Chunk<VT, NV, W, BX> &ch, uint32_t base = 0,
+                                           Chunk<VT, NV, W, BX> &ch, uint32_t base, int nx, int F,
                                            const VT *__restrict__ sd = nullptr) {
     // Entries past the row end repeat the row's last entry (its x row exists), so the
     // x loads of a batch need no select; their products are never added.
@@ -71,7 +84,7 @@ __device__ __forceinline__ void load_chunk(uint32_t j, uint32_t e, const IT *__r
     for (int q = 0; q < C::E; ++q) {
         const uint32_t jj = j + (C::L >= 2 ? (uint32_t)(q * C::LL + gl) : (uint32_t)q);
         const uint32_t jc = jj < e ? jj : e - 1;
-        ch.c[q] = live ? (uint32_t)col[jc] : 0u;
+        ch.c[q] = live ? column(col[jc], nx, F) : 0u;
         ch.v[q] = live ? val[jc] : VT(0);
     }
     if constexpr (SCALE) {
@@ -167,8 +180,9 @@ __device__ __forceinline__ void row_acc(uint32_t j, const uint32_t e,
                                         const Chunk<VT, NV, W, BX> &first,
                                         const IT *__restrict__ col, const VT *__restrict__ val,
                                         uint32_t base, const VT *__restrict__ x, int k0,
-                                        VT (&acc)[W], uint32_t slo = 0, uint32_t sn = 0,
-                                        const VT *__restrict__ sd = nullptr, VT cz = VT(0)) {
+                                        VT (&acc)[W], int nx, int F, uint32_t slo = 0,
+                                        uint32_t sn = 0, const VT *__restrict__ sd = nullptr,
+                                        VT cz = VT(0)) {
     using C = Chunk<VT, NV, W, BX>;
     // a longer row loads its next chunk before the x loads of the current one, so the
     // chunk's latency overlaps them
@@ -177,7 +191,7 @@ __device__ __forceinline__ void row_acc(uint32_t j, const uint32_t e,
         const bool more = j + C::CH < e; // the same for all lanes of the row
         C nxt;
         if (more)
-            load_chunk<VT, IT, NV, W, SCALE, BX>(j + C::CH, e, col, val, nxt, base, sd);
+            load_chunk<VT, IT, NV, W, SCALE, BX>(j + C::CH, e, col, val, nxt, base, nx, F, sd);
         consume_chunk<VT, NV, W, SKIP, SCALE, BX>(j, e, cur, base, x, k0, acc, slo, sn, cz);
         if (!more)
             break;
@@ -249,6 +263,9 @@ __global__ __launch_bounds__(kBlock) void k_spmv(
     using P = Pack<VT, W>;
     if (done != nullptr && *done)
         return;
+    // grid codes: the grid's nx and nx*ny come in the place of the panel shift and the
+    // hybrid GS block size
+    const int gnx = shift, gF = (int)blk_rows;
     const int64_t lb = logical_block();
     const int tr = threadIdx.x / L, k0 = (threadIdx.x % L) * W;
     double part[ND > 0 ? ND : 1][W];
@@ -282,7 +299,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv(
     }
     constexpr bool SC = OP == OP_CHEBZ; // chunks carry their columns' isd
     Chunk<VT, NV, W, BX> ch;
-    load_chunk<VT, IT, NV, W, SC, BX>(jb, je, col, val, ch, bs, isd);
+    load_chunk<VT, IT, NV, W, SC, BX>(jb, je, col, val, ch, bs, gnx, gF, isd);
     // Drain the prologue loads once per tile: the row loop's head then merges only its
     // own back edge, where the last y store may stay in flight.
     __builtin_amdgcn_s_waitcnt(0);
@@ -290,7 +307,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv(
         const size_t o = (size_t)i * NV + k0;
         const uint32_t base = bs;
         Chunk<VT, NV, W, BX> nch;
-        load_chunk<VT, IT, NV, W, SC, BX>(nb, ne, col, val, nch, nbs, isd);
+        load_chunk<VT, IT, NV, W, SC, BX>(nb, ne, col, val, nch, nbs, gnx, gF, isd);
         uint32_t nnb = 0, nne = 0, nnbs = 0;
         if (i + 2 * RPB < end) {
             nnb = row[i + 2 * RPB];
@@ -323,14 +340,14 @@ __global__ __launch_bounds__(kBlock) void k_spmv(
         if constexpr (OP == OP_OFFBLOCK) {
             // t = b - sum over off-block columns (old x), HSGS core blocks of blk_rows
             const uint32_t lo = (uint32_t)((i / blk_rows) * blk_rows);
-            row_acc<VT, IT, NV, W, true, false, BX>(jb, je, ch, col, val, base, x, k0, acc, lo,
+            row_acc<VT, IT, NV, W, true, false, BX>(jb, je, ch, col, val, base, x, k0, acc, gnx, gF, lo,
                                          (uint32_t)blk_rows);
         } else if constexpr (OP == OP_CHEBZ) {
             // the operand is b; each gathered entry enters as the zero-x first step's u
-            row_acc<VT, IT, NV, W, false, true, BX>(jb, je, ch, col, val, base, x, k0, acc, 0u, 0u,
+            row_acc<VT, IT, NV, W, false, true, BX>(jb, je, ch, col, val, base, x, k0, acc, gnx, gF, 0u, 0u,
                                                 isd, c2);
         } else {
-            row_acc<VT, IT, NV, W, false, false, BX>(jb, je, ch, col, val, base, x, k0, acc);
+            row_acc<VT, IT, NV, W, false, false, BX>(jb, je, ch, col, val, base, x, k0, acc, gnx, gF);
         }
         if constexpr (ND > 0)
             epi_load<VT, NV, W, OP>(i, o, oy, k0, in, yv, b, o1, isd, rr, out2, xupdv, last,
@@ -457,7 +474,7 @@ __device__ __forceinline__ void consume_gchunk(uint32_t j, uint32_t e, const GCh
 }
 
 template <typename VT, int NV, int OP>
-__global__ __launch_bounds__(kBlock) void k_spmv_grid(
+__global__ __launch_bounds__(kBlock) void k_spmv_sweep(
     const uint32_t *__restrict__ row, const VT *__restrict__ val,
     const uint8_t *__restrict__ gcode, const GridSched g, const VT *__restrict__ x, void *__restrict__ yv, const VT *__restrict__ b,
     const VT *__restrict__ o1, const VT *__restrict__ isd, const VT *__restrict__ rr,
@@ -946,6 +963,31 @@ bool spmv_wide_batches(const Mat &A, int rpb) {
            (A.nrows + rpb - 1) / rpb <= 512;
 }
 
+// Whether the row-parallel kernel reads the grid codes of A (1 byte per entry) instead of
+// its columns (2 or 4): matrices with a grid view whose rows are long enough for the index
+// bytes to show.  27-point operator at 96^3, y = A x, us (columns / codes): fp64 nv = 4
+// 106 / 76, 8 123 / 99, 32 312 / 296; fp32 nv = 4 119 / 80, 32 149 / 128; equal at 48^3 and
+// below, where the matrix stays in cache.
+bool takes_codes(const Mat &A, SpmvOp op) {
+    return op != OP_OFFBLOCK && op != OP_PROLONG32 && A.gcode != nullptr && A.row_ind == nullptr &&
+           g_tune.grid_enable == 2 && A.nnz >= kGridMinRowNnz * A.nrows;
+}
+
+// Whether op on A runs as the LDS-window line sweep (k_spmv_sweep).  By default only the
+// Krylov SpMMs with dot partials of a large fp64 long-row operator with 32 right-hand
+// sides: 340 against 385 us at 96^3 (x of 226 MB); everywhere else the row-parallel kernel
+// is the faster one (y = A x at 64^3, nv = 32: 118 against 72 us; fp32 at 96^3: 194 against
+// 128; nv = 8 at 24^3: 67 against 6, the sweep's lines being too few to fill the chip).
+bool takes_sweep(const Mat &A, SpmvOp op, int nv) {
+    if (A.idx == IDX_U8 || op == OP_OFFBLOCK || op == OP_PROLONG32 || op == OP_CHEBZ ||
+        op == OP_CHEBR || A.gcode == nullptr || A.row_ind != nullptr || g_tune.grid_enable == 0)
+        return false;
+    return g_tune.grid_enable == 1 ||
+           (A.prec == F64 && nv == 32 && A.nnz >= kGridMinRowNnz * A.nrows &&
+            (op == OP_DOT1 || op == OP_DOT3 || op == OP_RDOT4 || op == OP_RESID0) &&
+            A.nrows * nv * 8 >= ((int64_t)192 << 20));
+}
+
 namespace {
 
 template <typename VT, typename IT, int NV, int OP>
@@ -968,17 +1010,14 @@ int launch_t(const Mat &A, const void *x, void *y, const SpmvArgs &a, hipStream_
             return ND > 0 ? S.grid : 0;
         }
     }
-    // the off-block residual of hybrid GS stays on the row path: decoding each entry's
-    // column to skip the row's own block made the grid sweep slower (466 against 369 us on
-    // the 96^3 27-point operator)
     if constexpr (sizeof(IT) != 1 && OP != OP_OFFBLOCK && OP != OP_PROLONG32 &&
                   OP != OP_CHEBZ && OP != OP_CHEBR) {
-        if (A.gcode != nullptr && grid_on(A) && A.row_ind == nullptr) {
+        if (takes_sweep(A, (SpmvOp)OP, NV)) {
             // the grid sweep's dot launches take their own partial count: more work items
             // pay there (27-point, 96^3: 409 -> 336 us with 2048), unlike the row path
             const GridLaunch G = grid_plan(A.gx, A.gy, A.gz, RPB,
                                            ND > 0 ? g_tune.grid_dot_groups : cap);
-            hipLaunchKernelGGL((k_spmv_grid<VT, NV, OP>), dim3(G.grid), dim3(kBlock), 0, s,
+            hipLaunchKernelGGL((k_spmv_sweep<VT, NV, OP>), dim3(G.grid), dim3(kBlock), 0, s,
                                A.row, (const VT *)A.val, A.gcode, G.g,
                                (const VT *)x, y,
                                (const VT *)a.b, (const VT *)a.o1, (const VT *)a.isd,
@@ -999,6 +1038,18 @@ int launch_t(const Mat &A, const void *x, void *y, const SpmvArgs &a, hipStream_
                                (VT *)a.out2, (VT *)a.out3, a.xupd, (VT)a.c, a.last, a.x_zero,
                                a.out_f32, a.partials, a.done, a.blk_rows, A.row_ind,
                                (VT)a.c2);
+            return ND > 0 ? L.grid : 0;
+        }
+    }
+    if constexpr (sizeof(IT) != 1 && OP != OP_OFFBLOCK && OP != OP_PROLONG32) {
+        if (takes_codes(A, (SpmvOp)OP)) {
+            hipLaunchKernelGGL((k_spmv<VT, GridCol, NV, OP>), dim3(L.grid), dim3(kBlock), 0, s,
+                               A.row, (const GridCol *)A.gcode, (const VT *)A.val,
+                               (const uint32_t *)nullptr, A.gx, L.sc, (const VT *)x, y,
+                               (const VT *)a.b, (const VT *)a.o1, (const VT *)a.isd,
+                               (const VT *)a.r, (VT *)a.out2, (VT *)a.out3, a.xupd, (VT)a.c,
+                               a.last, a.x_zero, a.out_f32, a.partials, a.done,
+                               (int64_t)A.gx * A.gy, (const uint32_t *)nullptr, (VT)a.c2);
             return ND > 0 ? L.grid : 0;
         }
     }
@@ -1108,11 +1159,6 @@ bool takes_st7(const Mat &A, SpmvOp op, int nv) {
            op != OP_CHEBR && nv >= 8 &&
            A.st7 != nullptr && g_tune.st7_enable && A.row_ind == nullptr;
 }
-bool takes_grid(const Mat &A, SpmvOp op) {
-    return A.idx != IDX_U8 && op != OP_OFFBLOCK && op != OP_PROLONG32 && op != OP_CHEBZ &&
-           op != OP_CHEBR && A.gcode != nullptr && grid_on(A) && A.row_ind == nullptr;
-}
-
 // Algorithmic HBM bytes of one SpMV launch: the matrix streams once (values, column
 // indices or grid codes, row pointers, panel bases, row map), x once (ncols rows), and
 // the epilogue's vector operands and results once each; dot partials are added by the
@@ -1179,7 +1225,7 @@ double spmv_bytes(const Mat &A, int nv, SpmvOp op, const SpmvArgs &a, bool grid,
 
 int spmv_dispatch(const Mat &A, int nv, const void *x, void *y, SpmvOp op, const SpmvArgs &a,
                   hipStream_t s) {
-    if (takes_wave(A, op, nv) && !takes_st7(A, op, nv) && !takes_grid(A, op)) {
+    if (takes_wave(A, op, nv) && !takes_st7(A, op, nv) && !takes_sweep(A, op, nv)) {
         spmv_wave(A, nv, x, y, op, a, s);
         return 0;
     }
@@ -1204,7 +1250,7 @@ const char *idx_name(int idx) {
 
 // whether op on A runs on the row-parallel kernel (neither the stencil nor the grid path)
 bool spmv_row_parallel(const Mat &A, SpmvOp op, int nv) {
-    return !takes_st7(A, op, nv) && !takes_grid(A, op);
+    return !takes_st7(A, op, nv) && !takes_sweep(A, op, nv);
 }
 
 int spmv(const Mat &A, int nv, const void *x, void *y, SpmvOp op, const SpmvArgs &a,
@@ -1215,9 +1261,10 @@ int spmv(const Mat &A, int nv, const void *x, void *y, SpmvOp op, const SpmvArgs
     const int np = spmv_dispatch(A, nv, x, y, op, a, s);
     if (led.on) {
         const bool st7 = takes_st7(A, op, nv);
-        const bool grid = !st7 && takes_grid(A, op);
-        const bool wave = !st7 && !grid && takes_wave(A, op, nv);
-        const bool wide = !st7 && !grid && !wave && (nv == 8 || nv == 32) && A.idx != IDX_U8 &&
+        const bool sweep = !st7 && takes_sweep(A, op, nv);
+        const bool wave = !st7 && !sweep && takes_wave(A, op, nv);
+        const bool grid = !st7 && !sweep && !wave && takes_codes(A, op);
+        const bool wide = !st7 && !sweep && !grid && !wave && (nv == 8 || nv == 32) && A.idx != IDX_U8 &&
                           (op == OP_SET || op == OP_ADD || op == OP_RESID || op == OP_CHEB0 ||
                            op == OP_CHEB || op == OP_CHEBZ || op == OP_CHEBR) &&
                           spmv_wide_batches(A, kBlock / (nv / std::min(nv, A.prec == F64 ? 2 : 4)));
@@ -1226,10 +1273,11 @@ int spmv(const Mat &A, int nv, const void *x, void *y, SpmvOp op, const SpmvArgs
                                   : wave ? "," + std::to_string(wave_entries(A, nv)) + ">"
                                          : std::string(">"));
         led.kernel = st7    ? std::string("k_spmv_st7<") + prec_name(A.prec) + "," + tail
+                     : sweep ? std::string("k_spmv_sweep<") + prec_name(A.prec) + "," + tail
                      : grid ? std::string("k_spmv_grid<") + prec_name(A.prec) + "," + tail
                             : std::string(wave ? "k_spmv_wave<" : "k_spmv<") + prec_name(A.prec) + "," +
                                   idx_name(A.idx) + "," + tail;
-        led.bytes = spmv_bytes(A, nv, op, a, grid, st7) +
+        led.bytes = spmv_bytes(A, nv, op, a, grid || sweep, st7) +
                     (np > 0 ? (double)np * op_ndots(op) * nv * 8.0 : 0.0);
     }
     return np;

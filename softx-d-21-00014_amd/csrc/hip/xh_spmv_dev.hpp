@@ -29,10 +29,17 @@ __device__ __forceinline__ void st(T *__restrict__ p, const Pack<T, W> &v) {
     __builtin_nontemporal_store(t, reinterpret_cast<vec *>(p));
 }
 
+// the code of a grid neighbour (Mat::gcode) in the place of a column index
+struct GridCol {
+    uint8_t code;
+};
+
 template <typename IT>
 __device__ __forceinline__ uint32_t panel_base(const uint32_t *__restrict__ pb, int shift,
                                                int64_t i) {
-    if constexpr (sizeof(IT) == 4)
+    if constexpr (std::is_same<IT, GridCol>::value)
+        return (uint32_t)i;
+    else if constexpr (sizeof(IT) == 4)
         return 0u;
     else
         return pb[i >> shift];

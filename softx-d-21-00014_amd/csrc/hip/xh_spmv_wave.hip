@@ -228,9 +228,11 @@ bool takes_wave(const Mat &A, SpmvOp op, int nv) {
     if (g_tune.wide_batches == 0 || A.nnz < 4 * A.nrows)
         return false;
     const bool longrows = A.nnz >= 12 * A.nrows;
-    if (nv == 1 && longrows)
+    if (nv <= 2 && longrows)
         return true;
     const int L = nv / std::min(nv, A.prec == F64 ? 2 : 4);
+    if (A.gcode != nullptr && L > 1)
+        return false;
     const int64_t waves = L >= 4 ? A.nrows : A.nrows * L / 4;
     const int64_t cap = L == 1 ? 8192 : L == 2 ? 10240 : L == 4 ? 8192 : L == 8 ? 4096
                         : L == 16 ? 1536 : 0;

@@ -48,6 +48,39 @@ def test_grid_spmv_bit_identical(grid_on, prec):
             assert np.array_equal(out[0][1], out[1][1]), (name, nv)
 
 
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("dims", [(10, 9, 7), (33, 5, 4)])
+def test_grid_codes_bit_identical(gpu, prec, dims):
+    # the row-parallel kernel on 1-byte neighbour codes against its column indices: products
+    # of a random x, and a V-cycle with Chebyshev smoothing (from zero and non-zero x)
+    X = gpu
+    row, col, val = X.q1fem27(*dims)[:3]
+    n = len(row) - 1
+    A = X.Matrix(row, col, val, prec=prec)
+    assert A.grid() == dims
+    dt = np.float64 if prec == 0 else np.float32
+    levels = X.Amg(row, col, val, coarse_size=40).export()
+    prm = X.default_params(smoother="Chebyshev", poly_order=4, mg_prec=2 * prec)
+    try:
+        for nv in (1, 2, 4, 8, 16, 32, 64):
+            x = X.DeviceArray.from_host(np.random.default_rng(nv).standard_normal(n * nv).astype(dt))
+            S = X.Solver(X.Hier(levels), prm, nv)
+            db = X.DeviceArray.from_host(X.rhs_uniform(nv, n, nv))
+            out = []
+            for ge in (0, 2):
+                X.set_option("spmv_grid_enable", ge)
+                y, dx = X.DeviceArray(n * nv, dt), X.DeviceArray(n * nv)
+                y2 = X.DeviceArray.from_host(np.linspace(-1, 1, n * nv).astype(dt))
+                A.spmv(nv, x, y)
+                A.spmv(nv, x, y2, accumulate=True)
+                S.precond_apply(db, dx)
+                out.append((y.to_host(), y2.to_host(), dx.to_host()))
+            for a, b in zip(*out):
+                assert np.array_equal(a, b), nv
+    finally:
+        X.set_option("spmv_grid_enable", 2)
+
+
 def test_grid_path_by_row_length(gpu):
     # the default takes the grid path for the 27-point operator (27 entries per interior
     # row) and the row-parallel kernel for the 7-point cube: the launches of a solve show it
