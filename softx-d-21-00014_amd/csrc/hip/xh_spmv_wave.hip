@@ -2,7 +2,7 @@
 //
 // Such a launch leaves most of the GPU idle; its time is the chain of memory round trips of
 // one row.  The row-parallel kernel (xh_spmv.hip) gives a row L = NV/W lanes, which walk its
-// entries in batches of 8: a 93-entry row waits 12 times.  Here a group of GL >= 4 L lanes
+// entries in batches of 8: a 93-entry row waits 12 times.  Here a group of GL > L lanes
 // owns the row: its lanes load the columns and values of up to CH entries at once, then
 // all their x rows at once, round every product, and put the products in LDS by entry.  The
 // first L lanes then add them one by one in stored order, so each RHS gets the sum of
@@ -17,28 +17,29 @@
 namespace xh {
 namespace {
 
-template <typename VT, int NV>
+// EPX: entries of a row loaded side by side (at most; 64 lanes hold 64 / L)
+template <typename VT, int NV, int EPX>
 struct WaveShape {
     static constexpr int W = Width<VT, NV>::value;
     static constexpr int L = NV / W;                       // lanes per entry and per sum
-    static constexpr int GL = L >= 4 ? 64 : 16 * L;        // lanes per row
+    static constexpr int EP = EPX * L > 64 ? 64 / L : EPX; // entries loaded side by side
+    static constexpr int GL = EP * L;                      // lanes per row
     static constexpr int G = 64 / GL;                      // rows per wave
-    static constexpr int EP = GL / L;                      // entries loaded side by side
-    static constexpr int CH = EP >= 4 ? 64 : 32;           // entries per pass
+    static constexpr int CH = EPX == 16 && EP >= 4 ? 64 : 32; // entries per pass
     static constexpr int Q = CH / EP;                      // x loads in flight per lane
     // products of one row in LDS; the pad keeps the sums of the wave's rows on different
     // banks
     static constexpr int STRIDE = CH * NV + 16 / (int)sizeof(VT);
 };
 
-template <typename VT, typename IT, int NV, int OP>
+template <typename VT, typename IT, int NV, int OP, int EPX>
 __global__ __launch_bounds__(64) void k_spmv_wave(
     const uint32_t *__restrict__ row, const IT *__restrict__ col, const VT *__restrict__ val,
     const uint32_t *__restrict__ pbase, int shift, int64_t nrows, const VT *__restrict__ x,
     void *__restrict__ yv, const VT *__restrict__ b, const VT *__restrict__ isd,
     const VT *__restrict__ rr, VT *__restrict__ out2, void *__restrict__ xupdv, VT c, int last,
     int x_zero, int out_f32, const int *__restrict__ done, VT c2) {
-    using S = WaveShape<VT, NV>;
+    using S = WaveShape<VT, NV, EPX>;
     constexpr int W = S::W, L = S::L, GL = S::GL, EP = S::EP, CH = S::CH, Q = S::Q;
     using P = Pack<VT, W>;
     __shared__ __align__(16) VT prod[S::G * S::STRIDE];
@@ -155,14 +156,25 @@ __global__ __launch_bounds__(64) void k_spmv_wave(
     }
 }
 
-template <typename VT, typename IT, int NV, int OP>
-void launch(const Mat &A, const void *x, void *y, const SpmvArgs &a, hipStream_t s) {
-    constexpr int G = WaveShape<VT, NV>::G;
-    hipLaunchKernelGGL((k_spmv_wave<VT, IT, NV, OP>), dim3((unsigned)((A.nrows + G - 1) / G)),
+template <typename VT, typename IT, int NV, int OP, int EPX>
+void launch_ep(const Mat &A, const void *x, void *y, const SpmvArgs &a, hipStream_t s) {
+    constexpr int G = WaveShape<VT, NV, EPX>::G;
+    hipLaunchKernelGGL((k_spmv_wave<VT, IT, NV, OP, EPX>), dim3((unsigned)((A.nrows + G - 1) / G)),
                        dim3(64), 0, s, A.row, (const IT *)A.col, (const VT *)A.val, A.panel_base,
                        A.panel_shift, A.nrows, (const VT *)x, y, (const VT *)a.b,
                        (const VT *)a.isd, (const VT *)a.r, (VT *)a.out2, a.xupd, (VT)a.c, a.last,
                        a.x_zero, a.out_f32, a.done, (VT)a.c2);
+}
+
+template <typename VT, typename IT, int NV, int OP>
+void launch(const Mat &A, const void *x, void *y, const SpmvArgs &a, hipStream_t s) {
+    // one lane per entry and many rows: 4 lanes per row, so a wave's instructions serve 16
+    // rows (262144 rows of 26 entries, us with 16 / 4 lanes: fp64 nv = 2 43 / 36, fp32 nv = 1
+    // 24 / 18, nv = 4 44 / 26); with fewer rows than fill the chip the longer batches lose
+    if constexpr (WaveShape<VT, NV, 4>::L == 1)
+        if (wave_entries(A, NV) == 4)
+            return launch_ep<VT, IT, NV, OP, 4>(A, x, y, a, s);
+    launch_ep<VT, IT, NV, OP, 16>(A, x, y, a, s);
 }
 
 template <typename VT, typename IT, int NV>
@@ -241,6 +253,8 @@ bool takes_wave(const Mat &A, SpmvOp op, int nv) {
 
 int wave_entries(const Mat &A, int nv) {
     const int L = nv / std::min(nv, A.prec == F64 ? 2 : 4);
+    if (L == 1 && A.nrows > 65536)
+        return 4;
     return L >= 4 ? 64 / L : 16;
 }
 

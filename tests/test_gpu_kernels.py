@@ -208,6 +208,24 @@ def test_spmv_long_row_kernel_bit_exact(gpu, O, nv, prec):
         X.set_option("spmv_wave_enable", 2)
 
 
+@pytest.mark.parametrize("nv,prec", [(1, 0), (1, 1), (2, 0), (4, 1)])
+def test_spmv_many_long_rows_few_rhs_bit_exact(gpu, O, nv, prec):
+    # more than 65536 rows: 4 lanes per row
+    X = gpu
+    row, col, val = X.q1fem27(41, 41, 41)[:3]
+    n = len(row) - 1
+    dt = np.float64 if prec == 0 else np.float32
+    x = np.random.default_rng(nv).standard_normal(n * nv).astype(dt)
+    A = X.Matrix(row, col, val, prec=prec)
+    dx, dy = X.DeviceArray.from_host(x), X.DeviceArray(n * nv, dt)
+    X.set_option("spmv_wave_enable", 1)
+    try:
+        A.spmv(nv, dx, dy)
+    finally:
+        X.set_option("spmv_wave_enable", 2)
+    assert np.array_equal(dy.to_host(), O.spmv(row, col, val, x, nv, f32=prec == 1))
+
+
 @pytest.mark.parametrize("smoother,nv,mg_prec", [("Chebyshev", 1, 0), ("Chebyshev", 8, 2),
                                                  ("Chebyshev", 32, 1), ("Jacobi", 4, 0),
                                                  ("HSGS", 2, 2), ("Chebyshev", 64, 0)])
