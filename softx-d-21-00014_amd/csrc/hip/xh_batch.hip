@@ -2,7 +2,7 @@
 // together, each iteration one sequence of launches over all systems (captured as one
 // hipGraph by the runtime).  A launch walks a list of work items (system, row range);
 // a fixed grid of workgroups takes items blockIdx.x, blockIdx.x + gridDim.x, ..., so
-// uneven systems share one launch.  Inside an item a lane owns (row, RHS) of that
+// uneven systems share one launch.  Inside an item a lane owns one or two RHS of a row of that
 // system (nv <= 16 lanes per row, 256/nv rows per pass).
 //
 // Each system follows the single-system arithmetic exactly: SpMV row sums in stored
@@ -85,18 +85,74 @@ __device__ __forceinline__ void batch_item(const BatchDev &d, const BatchItem &w
     }
     // B_CHEBZ: the zero-x first step's coefficient, applied to every gathered entry
     const double cz = OP == B_CHEBZ ? d.cheb[(size_t)w.sys * kChebMax + ci + 1] : 0.0;
+    constexpr bool SPMV = OP == B_RESID0 || OP == B_DOT1 || OP == B_DOT3 || OP == B_CHEB ||
+                          OP == B_CHEBZ;
+    // A row's entries go in chunks of CHK: the L >= 2 lanes of a row load one entry each and
+    // broadcast column and value across the row's lanes (DPP; the lanes of a row are active
+    // together), a single lane loads 4.  The row pointers run two rows ahead and the first
+    // chunk of the next row one row ahead, so a row waits for its x rows only (batched
+    // Chebyshev step over 64 systems: 379 -> 325 us; before, a row waited for its pointers,
+    // its entries and its x one after the other).
+    constexpr int E = L == 1 ? 4 : 1, CHK = L == 1 ? 4 : L;
+    struct Entries {
+        uint32_t c[E];
+        double a[E], d[E];
+    };
+    const uint32_t lr = (uint32_t)(tid % L);
+    auto load_entries = [&](uint32_t j, uint32_t j1, Entries &n) __attribute__((always_inline)) {
+        if (j < j1)
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                const uint32_t jj = j + (L == 1 ? (uint32_t)q : lr);
+                const uint32_t jc = jj < j1 ? jj : j1 - 1; // in bounds, never added
+                n.c[q] = d.col[jc];
+                n.a[q] = d.val[jc];
+                // B_CHEBZ: the entry's column scale, a load that depends on the column's
+                if constexpr (OP == B_CHEBZ)
+                    n.d[q] = d.isd[gb + n.c[q]];
+            }
+    };
+    uint32_t j0 = 0, j1 = 0, nj0 = 0, nj1 = 0;
+    Entries cur, nxt;
+    if constexpr (SPMV)
+        if (tr < rpp) {
+            const int64_t i = w.r0 + tr;
+            if (i < w.r1) {
+                j0 = d.row[gb + i];
+                j1 = d.row[gb + i + 1];
+            }
+            if (i + rpp < w.r1) {
+                nj0 = d.row[gb + i + rpp];
+                nj1 = d.row[gb + i + rpp + 1];
+            }
+            load_entries(j0, j1, cur);
+        }
     if (tr < rpp)
         for (int64_t i = w.r0 + tr; i < w.r1; i += rpp) {
             const size_t ob = vo + (size_t)i * nv + k0;
             const int64_t g = gb + i;
-            if constexpr (OP == B_RESID0 || OP == B_DOT1 || OP == B_DOT3 || OP == B_CHEB ||
-                          OP == B_CHEBZ) {
+            if constexpr (SPMV) {
                 const double *xs = v.in + vo;
+                load_entries(nj0, nj1, nxt);
+                uint32_t mj0 = 0, mj1 = 0;
+                if (i + 2 * rpp < w.r1) {
+                    mj0 = d.row[g + 2 * rpp];
+                    mj1 = d.row[g + 2 * rpp + 1];
+                }
+                // the epilogue's operands, in flight with the x rows
+                double ev[W], di = 0.0;
+                {
+                    const double *ep = OP == B_RESID0 ? v.b : OP == B_CHEBZ ? v.in : v.o1;
+#pragma unroll
+                    for (int u = 0; u < W; ++u)
+                        ev[u] = ep[ob + u];
+                    if constexpr (OP == B_CHEB || OP == B_CHEBZ)
+                        di = d.isd[g];
+                }
                 double acc[W];
 #pragma unroll
                 for (int u = 0; u < W; ++u)
                     acc[u] = 0.0;
-                const uint32_t j1 = d.row[g + 1];
                 // x row of entry column c: W consecutive RHS (16-B aligned for W = 2:
                 // system vectors start on 256 B, k0 and nv even)
                 auto ldx = [&](uint32_t c, double (&xq)[W]) __attribute__((always_inline)) {
@@ -120,93 +176,66 @@ __device__ __forceinline__ void batch_item(const BatchDev &d, const BatchItem &w
                             xq[u] = t * dc;
                         }
                 };
-                if constexpr (L == 1) {
-                    // entries in batches of EB: columns and values of the batch, then its x
-                    // rows, all in flight together; slots past the row end re-read the last
-                    // entry (in bounds) and are not added, so the sum keeps the stored order
-                    constexpr int EB = 4;
-                    for (uint32_t j = d.row[g]; j < j1; j += EB) {
-                        uint32_t c[EB];
-                        double a[EB], xv[EB][W], dz[EB];
-#pragma unroll
-                        for (int q = 0; q < EB; ++q) {
-                            const uint32_t jj = j + q < j1 ? j + q : j1 - 1;
-                            c[q] = d.col[jj];
-                            a[q] = d.val[jj];
-                        }
-#pragma unroll
-                        for (int q = 0; q < EB; ++q) {
-                            ldx(c[q], xv[q]);
+                for (uint32_t j = j0; j < j1; j += CHK) {
+                    Entries more;
+                    load_entries(j + CHK, j1, more); // a longer row's next chunk
+                    uint32_t c[CHK];
+                    double a[CHK], xv[CHK][W], dz[CHK];
+                    static_for<0, CHK>([&](auto qc) {
+                        constexpr int q = decltype(qc)::value;
+                        if constexpr (L == 1) {
+                            c[q] = cur.c[q];
+                            a[q] = cur.a[q];
                             if constexpr (OP == B_CHEBZ)
-                                dz[q] = d.isd[gb + c[q]];
-                        }
-#pragma unroll
-                        for (int q = 0; q < EB; ++q)
-                            if (j + q < j1) {
-                                zstep(xv[q], dz[q]);
-#pragma unroll
-                                for (int u = 0; u < W; ++u)
-                                    acc[u] = acc[u] + xv[q][u] * a[q];
-                            }
-                    }
-                } else {
-                    // the L lanes of the row load L consecutive entries, one each, and
-                    // broadcast column and value across the row's lanes (DPP); then the L x
-                    // rows are loaded together and added in stored order (slots past the
-                    // row end re-read the last entry and are not added).  The lanes of a
-                    // row are active together, as the broadcast needs.
-                    const uint32_t lr = (uint32_t)(tid % L);
-                    for (uint32_t j = d.row[g]; j < j1; j += L) {
-                        const uint32_t jm = j + lr < j1 ? j + lr : j1 - 1;
-                        const uint32_t cm = d.col[jm];
-                        const double am = d.val[jm];
-                        // B_CHEBZ: the entry's column scale, loaded by the same lane
-                        const double dm = OP == B_CHEBZ ? d.isd[gb + cm] : 0.0;
-                        uint32_t c[L];
-                        double a[L], xv[L][W], dz[L];
-                        static_for<0, L>([&](auto qc) {
-                            constexpr int q = decltype(qc)::value;
-                            c[q] = (uint32_t)bcast<L, q>((int)cm);
-                            a[q] = bcast<L, q>(am);
+                                dz[q] = cur.d[q];
+                        } else {
+                            c[q] = (uint32_t)bcast<L, q>((int)cur.c[0]);
+                            a[q] = bcast<L, q>(cur.a[0]);
                             if constexpr (OP == B_CHEBZ)
-                                dz[q] = bcast<L, q>(dm);
-                        });
+                                dz[q] = bcast<L, q>(cur.d[0]);
+                        }
+                    });
 #pragma unroll
-                        for (int q = 0; q < L; ++q)
+                    for (int q = 0; q < CHK; ++q)
+                        if (j + q < j1)
                             ldx(c[q], xv[q]);
 #pragma unroll
-                        for (int q = 0; q < L; ++q)
-                            if (j + q < j1) {
-                                zstep(xv[q], dz[q]);
+                    for (int q = 0; q < CHK; ++q)
+                        if (j + q < j1) {
+                            zstep(xv[q], dz[q]);
 #pragma unroll
-                                for (int u = 0; u < W; ++u)
-                                    acc[u] = acc[u] + xv[q][u] * a[q];
-                            }
-                    }
+                            for (int u = 0; u < W; ++u)
+                                acc[u] = acc[u] + xv[q][u] * a[q];
+                        }
+                    cur = more;
                 }
+                j0 = nj0;
+                j1 = nj1;
+                nj0 = mj0;
+                nj1 = mj1;
+                cur = nxt;
 #pragma unroll
                 for (int u = 0; u < W; ++u) {
                     const size_t o = ob + u;
                     if constexpr (OP == B_RESID0) {
                         // r0 = b - A x ; p = r = r0 ; (r0, r0)
-                        const double t = v.b[o] - acc[u];
+                        const double t = ev[u] - acc[u];
                         part[0][u] = part[0][u] + t * t;
                         v.out[o] = t;
                         v.out2[o] = t;
                         v.out3[o] = t;
                     } else if constexpr (OP == B_DOT1) {
                         v.out[o] = acc[u];
-                        part[0][u] = part[0][u] + acc[u] * v.o1[o];
+                        part[0][u] = part[0][u] + acc[u] * ev[u];
                     } else if constexpr (OP == B_DOT3) {
-                        const double sv = v.o1[o];
+                        const double sv = ev[u];
                         v.out[o] = acc[u];
                         part[0][u] = part[0][u] + acc[u] * sv;
                         part[1][u] = part[1][u] + acc[u] * acc[u];
                         part[2][u] = part[2][u] + sv * sv;
                     } else if constexpr (OP == B_CHEB) {
                         // r = b*isd ; t1 = c*r + (A u)*isd ; u' = t1*isd or x = t1*isd
-                        const double di = d.isd[g];
-                        const double rv = v.o1[o] * di;
+                        const double rv = ev[u] * di;
                         const double t2 = acc[u] * di;
                         double t1 = c1[u] * rv + t2;
                         t1 = t1 * di;
@@ -215,8 +244,7 @@ __device__ __forceinline__ void batch_item(const BatchDev &d, const BatchItem &w
                         else
                             v.out[o] = t1;
                     } else { // B_CHEBZ: r = b*isd ; t1 = c*r + (A u)*isd ; u' or x = t1*isd
-                        const double di = d.isd[g];
-                        const double rv = v.in[o] * di;
+                        const double rv = ev[u] * di;
                         const double t2 = acc[u] * di;
                         double t1 = c1[u] * rv + t2;
                         t1 = t1 * di;
