@@ -25,6 +25,7 @@
 #include <cstring>
 #include <memory>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 namespace xh {
@@ -38,13 +39,9 @@ __device__ __forceinline__ float bf2f(bf16_t v) {
     return __uint_as_float((uint32_t)v << 16);
 }
 
-// round to nearest even
+// round to nearest even (v_cvt_pk_bf16_f32)
 __device__ __forceinline__ bf16_t f2bf(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7f800000u) == 0x7f800000u) // inf / nan: keep, quiet nan
-        return (bf16_t)((u >> 16) | ((u & 0xffffu) ? 0x40u : 0u));
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (bf16_t)(u >> 16);
+    return __builtin_bit_cast(bf16_t, (__bf16)f);
 }
 
 __device__ __forceinline__ bf16x8 pack8(const bf16_t (&e)[8]) {
@@ -245,11 +242,11 @@ __device__ __forceinline__ void conv_tile_store(const Dims &g, int nb, int z0, i
     for (int t = 0; t < NT; ++t) {
         const int li = wave * LPW + t / XT, xt = t % XT;
         const int iz = li / TY, iy = li % TY;
-        const int64_t mo =
-            (((int64_t)nb * g.d + z0 + iz) * g.h + y0 + iy) * g.w + x0 + 16 * xt + r;
+        // the line's first output (the same for the whole wave) and the lane's place in it
+        const int64_t line = ((((int64_t)nb * g.d + z0 + iz) * g.h + y0 + iy) * g.w + x0) * COUT;
 #pragma unroll
         for (int c = 0; c < CT; ++c) {
-            const int64_t o0 = mo * COUT + 16 * c + 4 * kg;
+            const int64_t o0 = line + ((16 * xt + r) * COUT + 16 * c + 4 * kg);
             float v[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i)
@@ -280,74 +277,96 @@ __global__ __launch_bounds__(256) void k_conv_tile(Dims g, const bf16_t *__restr
                                                    const bf16_t *__restrict__ add, int relu,
                                                    bf16_t *__restrict__ out) {
     constexpr int CIN = 8 * NCG;
+    constexpr int TXS = UP ? TX / 2 : TX;     // staged voxels of a line without its halo
     constexpr int SZ = UP ? kTZ / 2 + 2 : kTZ + 2;
     constexpr int SY = UP ? TY / 2 + 2 : TY + 2;
-    constexpr int SX = UP ? TX / 2 + 2 : TX + 2;
-    constexpr int NCH = SZ * SY * SX * NCG; // 16-byte chunks staged
-    constexpr int PER = (NCH + 255) / 256;
+    constexpr int SX = TXS + 2;
+    constexpr int NL = SZ * SY;               // staged lines
+    constexpr int NCH = NL * SX * NCG;        // 16-byte chunks staged
+    constexpr int IC = TXS * NCG;             // chunks of a line without its halo
+    constexpr int IP = IC / 64;               // passes of a wave over them
+    constexpr int LW = (NL + 3) / 4;          // lines a wave stages
+    constexpr int HC = NL * 2 * NCG, HP = (HC + 255) / 256; // halo chunks
     constexpr int XT = TX / 16;               // 16-voxel tiles per line
     constexpr int LPW = kTZ * TY / 4;         // lines per wave
     constexpr int NT = LPW * XT;              // tiles per wave
-    constexpr int KS = (27 * CIN + 31) / 32; // k steps (kpad == 32 * KS)
+    constexpr int KS = (27 * CIN + 31) / 32;  // k steps (kpad == 32 * KS)
     constexpr bool PRE = CT == 1 && KS <= 16; // all weight fragments preloaded
-    static_assert(LPW >= 1 && (kTZ * TY) % 4 == 0, "tile lines must split over 4 waves");
+    constexpr int PF = PRE ? 1 : 4;           // else loaded PF steps ahead
+    static_assert(LPW >= 1 && (kTZ * TY) % 4 == 0 && TY % LPW == 0 && IC % 64 == 0,
+                  "tile lines must split over 4 waves");
     __shared__ uint4 sm[NCH];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ntx = g.w / TX, nty = g.h / TY, ntz = g.d / kTZ;
-    int64_t bid = blockIdx.x;
-    const int tx = (int)(bid % ntx);
+    int bid = blockIdx.x;
+    const int tx = bid % ntx;
     bid /= ntx;
-    const int ty = (int)(bid % nty);
+    const int ty = bid % nty;
     bid /= nty;
-    const int tz = (int)(bid % ntz);
-    const int nb = (int)(bid / ntz);
+    const int tz = bid % ntz;
+    const int nb = bid / ntz;
     const int x0 = tx * TX, y0 = ty * TY, z0 = tz * kTZ;
     const int r = lane & 15, kg = lane >> 4;
     // lane's weight row (output channel 16c + r of channel tile c at + 16c * kpad)
     const bf16_t *wrow = wt + (size_t)r * kpad + 8 * kg;
     // the staged volume (coarse with UP) and the tile's origin in it
     const int sd = UP ? g.d / 2 : g.d, sh = UP ? g.h / 2 : g.h, sw = UP ? g.w / 2 : g.w;
-    const int oz = (UP ? z0 / 2 : z0) - 1, oy = (UP ? y0 / 2 : y0) - 1,
-              ox = (UP ? x0 / 2 : x0) - 1;
+    const int oz = (UP ? z0 / 2 : z0) - 1, oy = (UP ? y0 / 2 : y0) - 1, ox = UP ? x0 / 2 : x0;
     {
-        uint4 st[PER];
+        // wave w stages the lines w, w + 4, ...: a line's address and whether it lies in the
+        // volume are the same for the whole wave, and its chunks are contiguous
+        uint4 st[LW][IP], hv[HP];
 #pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            const int q = tid + 256 * j;
+        for (int q = 0; q < LW; ++q) {
+            const int line = wave + 4 * q, zz = oz + line / SY, yy = oy + line % SY;
+            const bool ok = line < NL && zz >= 0 && zz < sd && yy >= 0 && yy < sh;
+            const uint4 *src = reinterpret_cast<const uint4 *>(
+                in + ((((int64_t)nb * sd + (ok ? zz : 0)) * sh + (ok ? yy : 0)) * sw + ox) * CIN);
+#pragma unroll
+            for (int p = 0; p < IP; ++p)
+                st[q][p] = ok ? src[lane + 64 * p] : make_uint4(0, 0, 0, 0);
+        }
+        // the halo voxels at both ends of every line
+        int hidx[HP];
+#pragma unroll
+        for (int p = 0; p < HP; ++p) {
+            const int e = tid + 256 * p, line = e / (2 * NCG), w = e % (2 * NCG);
+            const int cg = w % NCG, right = w / NCG;
+            const int zz = oz + line / SY, yy = oy + line % SY, xx = right ? ox + TXS : ox - 1;
+            hidx[p] = e < HC ? (line * NCG + cg) * SX + (right ? TXS + 1 : 0) : -1;
             uint4 v = make_uint4(0, 0, 0, 0);
-            if (q < NCH) {
-                const int line = q / (SX * NCG), rem = q - line * (SX * NCG);
-                const int sx = rem / NCG, cg = rem - sx * NCG;
-                const int zz = oz + line / SY, yy = oy + line % SY, xx = ox + sx;
-                if (zz >= 0 && zz < sd && yy >= 0 && yy < sh && xx >= 0 && xx < sw)
-                    v = *reinterpret_cast<const uint4 *>(
-                        in + ((((int64_t)nb * sd + zz) * sh + yy) * sw + xx) * CIN + 8 * cg);
-            }
-            st[j] = v;
+            if (e < HC && zz >= 0 && zz < sd && yy >= 0 && yy < sh && xx >= 0 && xx < sw)
+                v = *reinterpret_cast<const uint4 *>(
+                    in + ((((int64_t)nb * sd + zz) * sh + yy) * sw + xx) * CIN + 8 * cg);
+            hv[p] = v;
+        }
+        int lidx[IP]; // the lane's chunks in a staged line
+#pragma unroll
+        for (int p = 0; p < IP; ++p) {
+            const int c = lane + 64 * p;
+            lidx[p] = (c % NCG) * SX + c / NCG + 1;
         }
 #pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            const int q = tid + 256 * j;
-            if (q < NCH) {
-                const int line = q / (SX * NCG), rem = q - line * (SX * NCG);
-                const int sx = rem / NCG, cg = rem - sx * NCG;
-                sm[(line * NCG + cg) * SX + sx] = st[j];
-            }
+        for (int q = 0; q < LW; ++q) {
+            const int line = wave + 4 * q;
+            if (line < NL)
+#pragma unroll
+                for (int p = 0; p < IP; ++p)
+                    sm[line * (NCG * SX) + lidx[p]] = st[q][p];
         }
+#pragma unroll
+        for (int p = 0; p < HP; ++p)
+            if (hidx[p] >= 0)
+                sm[hidx[p]] = hv[p];
     }
     // weight fragments, issued once the staged values have left the registers
-    uint4 qa[PRE ? KS : 1];
-    if constexpr (PRE) {
+    uint4 qa[PRE ? KS : PF][CT];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
-            qa[ks] = *reinterpret_cast<const uint4 *>(wrow + 32 * ks);
-    }
-    uint4 qn[CT];
-    if constexpr (!PRE) {
+    for (int ks = 0; ks < (PRE ? KS : PF); ++ks)
 #pragma unroll
         for (int c = 0; c < CT; ++c)
-            qn[c] = *reinterpret_cast<const uint4 *>(wrow + (size_t)16 * c * kpad);
-    }
+            qa[ks][c] = *reinterpret_cast<const uint4 *>(wrow + (size_t)16 * c * kpad + 32 * ks);
     __syncthreads();
     f32x4 acc[NT][CT];
 #pragma unroll
@@ -355,64 +374,62 @@ __global__ __launch_bounds__(256) void k_conv_tile(Dims g, const bf16_t *__restr
 #pragma unroll
         for (int c = 0; c < CT; ++c)
             acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-    constexpr int K = 27 * CIN;
-    // tap and channel of the lane's first k, advanced by 32 per step (as in k_conv)
-    int tt = (8 * kg) / CIN, cc = 8 * kg - tt * CIN;
-    auto step = [&](int ks, const uint4 (&qb)[CT]) {
-        const bool kok = 32 * ks + 8 * kg < K;
-        const int dz = tt / 9 - 1, dy = (tt / 3) % 3 - 1, dx = tt % 3 - 1;
-        const int cg = cc >> 3;
+    // Staged chunk of tile t = (line tl of the wave, xt) at k step ks: lane (r, kg) reads
+    // channels 8 ((4 ks + kg) % NCG) of tap (4 ks + kg) / NCG at voxel r.  The offset is the
+    // lane's own part, constants of (ks, tl, xt), and one select where the step's 32 k
+    // cross from one tap into the next (kg >= thr).
+    const int iz = wave * LPW / TY, iy = wave * LPW % TY; // the wave's first line
+    const int lbase = kg * SX + (UP ? (iy / 2) * (NCG * SX) : r + (iz * SY + iy) * (NCG * SX));
+    int rx[3], zo[3]; // UP: coarse x of fine r + dx, coarse z offset of fine iz + dz
+    if constexpr (UP)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const int li = wave * LPW + t / XT, xt = t % XT;
-            const int iz = li / TY, iy = li % TY;
-            int sz, sy, sx;
-            if constexpr (UP) {
-                // fine offset -1 maps to coarse -1 (staged zero), as the fine bounds test
-                sz = ((iz + dz) >> 1) + 1;
-                sy = ((iy + dy) >> 1) + 1;
-                sx = ((16 * xt + r + dx) >> 1) + 1;
-            } else {
-                sz = iz + dz + 1;
-                sy = iy + dy + 1;
-                sx = 16 * xt + r + dx + 1;
-            }
-            uint4 q = sm[kok ? ((sz * SY + sy) * NCG + cg) * SX + sx : 0];
-            if (!kok)
-                q = make_uint4(0, 0, 0, 0);
-            // weights as the A operand: D[co][voxel], each lane 4 channels of one voxel
-#pragma unroll
-            for (int c = 0; c < CT; ++c)
-                acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    __builtin_bit_cast(bf16x8, qb[c]), __builtin_bit_cast(bf16x8, q), acc[t][c],
-                    0, 0, 0);
+        for (int q = 0; q < 3; ++q) {
+            rx[q] = ((r + q - 1) >> 1) + 1;
+            zo[q] = (((iz + q - 1) >> 1) + 1) * (SY * NCG * SX);
         }
-        cc += 32;
-        while (cc >= CIN) {
-            cc -= CIN;
-            ++tt;
-        }
+    auto tap_at = [&](auto tc, auto tlc) __attribute__((always_inline)) {
+        constexpr int t = decltype(tc)::value < 27 ? decltype(tc)::value : 26;
+        constexpr int tl = decltype(tlc)::value;
+        constexpr int dz = t / 9 - 1, dy = (t / 3) % 3 - 1, dx = t % 3 - 1;
+        if constexpr (UP) // fine offset -1 maps to coarse -1 (staged zero)
+            return rx[dx + 1] + zo[dz + 1] + (((tl + dy) >> 1) + 1) * (NCG * SX);
+        else
+            return (((dz + 1) * SY + dy + 1 + tl) * NCG) * SX + dx + 1;
     };
-    if constexpr (PRE) {
+    static_for<0, KS>([&](auto ksc) {
+        constexpr int ks = decltype(ksc)::value;
+        constexpr int tap = 4 * ks / NCG, s0 = 4 * ks % NCG, thr = NCG - s0;
+        uint4 qb[CT];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const uint4 qb[1] = {qa[ks]};
-            step(ks, qb);
+        for (int c = 0; c < CT; ++c) {
+            qb[c] = qa[PRE ? ks : ks % PF][c];
+            if (!PRE && ks + PF < KS)
+                qa[ks % PF][c] = *reinterpret_cast<const uint4 *>(wrow + (size_t)16 * c * kpad +
+                                                                  32 * (ks + PF));
         }
-    } else {
-        for (int ks = 0; ks < KS; ++ks) {
-            uint4 qb[CT];
+        static_for<0, LPW>([&](auto tlc) {
+            constexpr int tl = decltype(tlc)::value;
+            int a = tap_at(std::integral_constant<int, tap>(), tlc) + s0 * SX;
+            if constexpr (thr < 4) {
+                const int b = tap_at(std::integral_constant<int, tap + 1>(), tlc) - thr * SX;
+                a = kg >= thr ? b : a;
+            }
+            a += lbase;
 #pragma unroll
-            for (int c = 0; c < CT; ++c)
-                qb[c] = qn[c];
-            if (ks + 1 < KS)
+            for (int xt = 0; xt < XT; ++xt) {
+                uint4 q = sm[a + (UP ? 8 : 16) * xt];
+                if constexpr (32 * ks + 32 > 27 * CIN) // the padded last step: k past the taps
+                    if (32 * ks + 8 * kg >= 27 * CIN)
+                        q = make_uint4(0, 0, 0, 0);
+                // weights as the A operand: D[co][voxel], each lane 4 channels of one voxel
 #pragma unroll
                 for (int c = 0; c < CT; ++c)
-                    qn[c] = *reinterpret_cast<const uint4 *>(wrow + (size_t)16 * c * kpad +
-                                                             32 * (ks + 1));
-            step(ks, qb);
-        }
-    }
+                    acc[tl * XT + xt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        __builtin_bit_cast(bf16x8, qb[c]), __builtin_bit_cast(bf16x8, q),
+                        acc[tl * XT + xt][c], 0, 0, 0);
+            }
+        });
+    });
     conv_tile_store<CT, NT, XT, LPW, TY>(g, nb, z0, y0, x0, wave, r, kg, acc, bias, add, relu,
                                          out);
 }
