@@ -270,23 +270,29 @@ __device__ __forceinline__ void conv_tile_store(const Dims &g, int nb, int z0, i
     }
 }
 
+// Whether a workgroup walks several z steps, keeping the planes two steps share in a ring and
+// loading the next step's while it computes: pays for the 16 -> 16 convolution (1682 ->
+// 1440 us at 128^3, 32 volumes), whose weights stay in registers; the others lost their
+// occupancy to the planes held in flight (32 -> 32 727 -> 839, upsampled 64 -> 48 341 -> 726).
+template <int NCG, int CT, bool UP>
+constexpr bool conv_marches = NCG == 2 && CT == 1 && !UP;
+
 template <int NCG, int CT, int TY, bool UP, int TX = kTX>
 __global__ __launch_bounds__(256) void k_conv_tile(Dims g, const bf16_t *__restrict__ in,
                                                    const bf16_t *__restrict__ wt, int kpad,
                                                    const float *__restrict__ bias,
                                                    const bf16_t *__restrict__ add, int relu,
-                                                   bf16_t *__restrict__ out) {
+                                                   int mz, bf16_t *__restrict__ out) {
     constexpr int CIN = 8 * NCG;
     constexpr int TXS = UP ? TX / 2 : TX;     // staged voxels of a line without its halo
     constexpr int SZ = UP ? kTZ / 2 + 2 : kTZ + 2;
     constexpr int SY = UP ? TY / 2 + 2 : TY + 2;
     constexpr int SX = TXS + 2;
-    constexpr int NL = SZ * SY;               // staged lines
-    constexpr int NCH = NL * SX * NCG;        // 16-byte chunks staged
+    constexpr int NP = UP ? 1 : 2;            // staged planes one step of kTZ planes adds
+    constexpr bool MARCH = conv_marches<NCG, CT, UP>;
+    constexpr int NCH = SZ * SY * SX * NCG;   // 16-byte chunks staged
     constexpr int IC = TXS * NCG;             // chunks of a line without its halo
     constexpr int IP = IC / 64;               // passes of a wave over them
-    constexpr int LW = (NL + 3) / 4;          // lines a wave stages
-    constexpr int HC = NL * 2 * NCG, HP = (HC + 255) / 256; // halo chunks
     constexpr int XT = TX / 16;               // 16-voxel tiles per line
     constexpr int LPW = kTZ * TY / 4;         // lines per wave
     constexpr int NT = LPW * XT;              // tiles per wave
@@ -298,7 +304,7 @@ __global__ __launch_bounds__(256) void k_conv_tile(Dims g, const bf16_t *__restr
     __shared__ uint4 sm[NCH];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int ntx = g.w / TX, nty = g.h / TY, ntz = g.d / kTZ;
+    const int ntx = g.w / TX, nty = g.h / TY, ntz = g.d / kTZ / mz;
     int bid = blockIdx.x;
     const int tx = bid % ntx;
     bid /= ntx;
@@ -306,20 +312,29 @@ __global__ __launch_bounds__(256) void k_conv_tile(Dims g, const bf16_t *__restr
     bid /= nty;
     const int tz = bid % ntz;
     const int nb = bid / ntz;
-    const int x0 = tx * TX, y0 = ty * TY, z0 = tz * kTZ;
+    const int x0 = tx * TX, y0 = ty * TY;
+    int z0 = tz * kTZ * mz;
     const int r = lane & 15, kg = lane >> 4;
     // lane's weight row (output channel 16c + r of channel tile c at + 16c * kpad)
     const bf16_t *wrow = wt + (size_t)r * kpad + 8 * kg;
     // the staged volume (coarse with UP) and the tile's origin in it
     const int sd = UP ? g.d / 2 : g.d, sh = UP ? g.h / 2 : g.h, sw = UP ? g.w / 2 : g.w;
-    const int oz = (UP ? z0 / 2 : z0) - 1, oy = (UP ? y0 / 2 : y0) - 1, ox = UP ? x0 / 2 : x0;
-    {
-        // wave w stages the lines w, w + 4, ...: a line's address and whether it lies in the
-        // volume are the same for the whole wave, and its chunks are contiguous
-        uint4 st[LW][IP], hv[HP];
+    const int oy = (UP ? y0 / 2 : y0) - 1, ox = UP ? x0 / 2 : x0;
+    // Staging of planes: wave w takes the lines w, w + 4, ...: a line's address and whether
+    // it lies in the volume are the same for the whole wave, and its chunks are
+    // contiguous; the halo voxels at both line ends go over all threads.  Plane pz of the
+    // staged volume lives in ring slot (pz - first plane) % SZ.
+    int lidx[IP]; // the lane's chunks in a staged line
+#pragma unroll
+    for (int p = 0; p < IP; ++p) {
+        const int c = lane + 64 * p;
+        lidx[p] = (c % NCG) * SX + c / NCG + 1;
+    }
+    auto load_planes = [&](int pz, auto np, auto &st, auto &hv) __attribute__((always_inline)) {
+        constexpr int NL = decltype(np)::value * SY, LW = (NL + 3) / 4, HC = NL * 2 * NCG;
 #pragma unroll
         for (int q = 0; q < LW; ++q) {
-            const int line = wave + 4 * q, zz = oz + line / SY, yy = oy + line % SY;
+            const int line = wave + 4 * q, zz = pz + line / SY, yy = oy + line % SY;
             const bool ok = line < NL && zz >= 0 && zz < sd && yy >= 0 && yy < sh;
             const uint4 *src = reinterpret_cast<const uint4 *>(
                 in + ((((int64_t)nb * sd + (ok ? zz : 0)) * sh + (ok ? yy : 0)) * sw + ox) * CIN);
@@ -327,111 +342,144 @@ __global__ __launch_bounds__(256) void k_conv_tile(Dims g, const bf16_t *__restr
             for (int p = 0; p < IP; ++p)
                 st[q][p] = ok ? src[lane + 64 * p] : make_uint4(0, 0, 0, 0);
         }
-        // the halo voxels at both ends of every line
-        int hidx[HP];
 #pragma unroll
-        for (int p = 0; p < HP; ++p) {
+        for (int p = 0; p < (HC + 255) / 256; ++p) {
             const int e = tid + 256 * p, line = e / (2 * NCG), w = e % (2 * NCG);
-            const int cg = w % NCG, right = w / NCG;
-            const int zz = oz + line / SY, yy = oy + line % SY, xx = right ? ox + TXS : ox - 1;
-            hidx[p] = e < HC ? (line * NCG + cg) * SX + (right ? TXS + 1 : 0) : -1;
+            const int zz = pz + line / SY, yy = oy + line % SY,
+                      xx = w >= NCG ? ox + TXS : ox - 1;
             uint4 v = make_uint4(0, 0, 0, 0);
             if (e < HC && zz >= 0 && zz < sd && yy >= 0 && yy < sh && xx >= 0 && xx < sw)
                 v = *reinterpret_cast<const uint4 *>(
-                    in + ((((int64_t)nb * sd + zz) * sh + yy) * sw + xx) * CIN + 8 * cg);
+                    in + ((((int64_t)nb * sd + zz) * sh + yy) * sw + xx) * CIN + 8 * (w % NCG));
             hv[p] = v;
         }
-        int lidx[IP]; // the lane's chunks in a staged line
-#pragma unroll
-        for (int p = 0; p < IP; ++p) {
-            const int c = lane + 64 * p;
-            lidx[p] = (c % NCG) * SX + c / NCG + 1;
-        }
+    };
+    auto store_planes = [&](int slot, auto np, const auto &st, const auto &hv) __attribute__((always_inline)) {
+        constexpr int NL = decltype(np)::value * SY, LW = (NL + 3) / 4, HC = NL * 2 * NCG;
+        auto at = [&](int line) { // LDS chunk of a line: its plane's slot wraps around
+            int sl = slot + line / SY;
+            sl = sl >= SZ ? sl - SZ : sl;
+            return (sl * SY + line % SY) * (NCG * SX);
+        };
 #pragma unroll
         for (int q = 0; q < LW; ++q) {
             const int line = wave + 4 * q;
             if (line < NL)
 #pragma unroll
                 for (int p = 0; p < IP; ++p)
-                    sm[line * (NCG * SX) + lidx[p]] = st[q][p];
+                    sm[at(line) + lidx[p]] = st[q][p];
         }
 #pragma unroll
-        for (int p = 0; p < HP; ++p)
-            if (hidx[p] >= 0)
-                sm[hidx[p]] = hv[p];
+        for (int p = 0; p < (HC + 255) / 256; ++p) {
+            const int e = tid + 256 * p, line = e / (2 * NCG), w = e % (2 * NCG);
+            if (e < HC)
+                sm[at(line) + (w % NCG) * SX + (w >= NCG ? TXS + 1 : 0)] = hv[p];
+        }
+    };
+    {
+        constexpr int NL = SZ * SY;
+        uint4 st[(NL + 3) / 4][IP], hv[(NL * 2 * NCG + 255) / 256];
+        const std::integral_constant<int, SZ> np;
+        load_planes((UP ? z0 / 2 : z0) - 1, np, st, hv);
+        store_planes(0, np, st, hv);
     }
     // weight fragments, issued once the staged values have left the registers
     uint4 qa[PRE ? KS : PF][CT];
+    auto load_weights = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int ks = 0; ks < (PRE ? KS : PF); ++ks)
+        for (int ks = 0; ks < (PRE ? KS : PF); ++ks)
 #pragma unroll
-        for (int c = 0; c < CT; ++c)
-            qa[ks][c] = *reinterpret_cast<const uint4 *>(wrow + (size_t)16 * c * kpad + 32 * ks);
+            for (int c = 0; c < CT; ++c)
+                qa[ks][c] = *reinterpret_cast<const uint4 *>(wrow + (size_t)16 * c * kpad + 32 * ks);
+    };
+    load_weights();
     __syncthreads();
-    f32x4 acc[NT][CT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int c = 0; c < CT; ++c)
-            acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
     // Staged chunk of tile t = (line tl of the wave, xt) at k step ks: lane (r, kg) reads
     // channels 8 ((4 ks + kg) % NCG) of tap (4 ks + kg) / NCG at voxel r.  The offset is the
-    // lane's own part, constants of (ks, tl, xt), and one select where the step's 32 k
-    // cross from one tap into the next (kg >= thr).
+    // lane's own part, the tap's plane slot, constants of (ks, tl, xt), and one select where
+    // the step's 32 k cross from one tap into the next (kg >= thr).
     const int iz = wave * LPW / TY, iy = wave * LPW % TY; // the wave's first line
-    const int lbase = kg * SX + (UP ? (iy / 2) * (NCG * SX) : r + (iz * SY + iy) * (NCG * SX));
-    int rx[3], zo[3]; // UP: coarse x of fine r + dx, coarse z offset of fine iz + dz
-    if constexpr (UP)
+    const int lbase = kg * SX + (UP ? iy / 2 : iy) * (NCG * SX) + (UP ? 0 : r);
+    int rx[3], zo[3]; // UP: coarse x of fine r + dx; LDS offset of the plane at fine iz + dz
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+        rx[q] = ((r + q - 1) >> 1) + 1;
+    int slot = 0; // ring slot of the step's first staged plane
+    // the planes the next step adds, loaded while this step computes
+    constexpr int NLN = NP * SY;
+    uint4 nst[(NLN + 3) / 4][IP], nhv[(NLN * 2 * NCG + 255) / 256];
+    const std::integral_constant<int, NP> nnp;
+    const int steps = MARCH ? mz : 1;
+    for (int step = 0; step < steps; ++step, z0 += kTZ) {
+        if (MARCH && step + 1 < steps)
+            load_planes((UP ? z0 / 2 : z0) - 1 + SZ, nnp, nst, nhv);
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
-            rx[q] = ((r + q - 1) >> 1) + 1;
-            zo[q] = (((iz + q - 1) >> 1) + 1) * (SY * NCG * SX);
+            int sl = slot + (UP ? ((iz + q - 1) >> 1) + 1 : iz + q);
+            sl = sl >= SZ ? sl - SZ : sl;
+            zo[q] = sl * (SY * NCG * SX);
         }
-    auto tap_at = [&](auto tc, auto tlc) __attribute__((always_inline)) {
-        constexpr int t = decltype(tc)::value < 27 ? decltype(tc)::value : 26;
-        constexpr int tl = decltype(tlc)::value;
-        constexpr int dz = t / 9 - 1, dy = (t / 3) % 3 - 1, dx = t % 3 - 1;
-        if constexpr (UP) // fine offset -1 maps to coarse -1 (staged zero)
-            return rx[dx + 1] + zo[dz + 1] + (((tl + dy) >> 1) + 1) * (NCG * SX);
-        else
-            return (((dz + 1) * SY + dy + 1 + tl) * NCG) * SX + dx + 1;
-    };
-    static_for<0, KS>([&](auto ksc) {
-        constexpr int ks = decltype(ksc)::value;
-        constexpr int tap = 4 * ks / NCG, s0 = 4 * ks % NCG, thr = NCG - s0;
-        uint4 qb[CT];
+        f32x4 acc[NT][CT];
 #pragma unroll
-        for (int c = 0; c < CT; ++c) {
-            qb[c] = qa[PRE ? ks : ks % PF][c];
-            if (!PRE && ks + PF < KS)
-                qa[ks % PF][c] = *reinterpret_cast<const uint4 *>(wrow + (size_t)16 * c * kpad +
-                                                                  32 * (ks + PF));
-        }
-        static_for<0, LPW>([&](auto tlc) {
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+                acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        auto tap_at = [&](auto tc, auto tlc) __attribute__((always_inline)) {
+            constexpr int t = decltype(tc)::value < 27 ? decltype(tc)::value : 26;
             constexpr int tl = decltype(tlc)::value;
-            int a = tap_at(std::integral_constant<int, tap>(), tlc) + s0 * SX;
-            if constexpr (thr < 4) {
-                const int b = tap_at(std::integral_constant<int, tap + 1>(), tlc) - thr * SX;
-                a = kg >= thr ? b : a;
-            }
-            a += lbase;
+            constexpr int dz = t / 9 - 1, dy = (t / 3) % 3 - 1, dx = t % 3 - 1;
+            if constexpr (UP) // fine offset -1 maps to coarse -1 (staged zero)
+                return rx[dx + 1] + zo[dz + 1] + (((tl + dy) >> 1) + 1) * (NCG * SX);
+            else
+                return zo[dz + 1] + (dy + 1 + tl) * (NCG * SX) + dx + 1;
+        };
+        static_for<0, KS>([&](auto ksc) {
+            constexpr int ks = decltype(ksc)::value;
+            constexpr int tap = 4 * ks / NCG, s0 = 4 * ks % NCG, thr = NCG - s0;
+            uint4 qb[CT];
 #pragma unroll
-            for (int xt = 0; xt < XT; ++xt) {
-                uint4 q = sm[a + (UP ? 8 : 16) * xt];
-                if constexpr (32 * ks + 32 > 27 * CIN) // the padded last step: k past the taps
-                    if (32 * ks + 8 * kg >= 27 * CIN)
-                        q = make_uint4(0, 0, 0, 0);
-                // weights as the A operand: D[co][voxel], each lane 4 channels of one voxel
-#pragma unroll
-                for (int c = 0; c < CT; ++c)
-                    acc[tl * XT + xt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        __builtin_bit_cast(bf16x8, qb[c]), __builtin_bit_cast(bf16x8, q),
-                        acc[tl * XT + xt][c], 0, 0, 0);
+            for (int c = 0; c < CT; ++c) {
+                qb[c] = qa[PRE ? ks : ks % PF][c];
+                if (!PRE && ks + PF < KS)
+                    qa[ks % PF][c] = *reinterpret_cast<const uint4 *>(wrow + (size_t)16 * c * kpad +
+                                                                      32 * (ks + PF));
             }
+            static_for<0, LPW>([&](auto tlc) {
+                constexpr int tl = decltype(tlc)::value;
+                int a = tap_at(std::integral_constant<int, tap>(), tlc) + s0 * SX;
+                if constexpr (thr < 4) {
+                    const int b = tap_at(std::integral_constant<int, tap + 1>(), tlc) - thr * SX;
+                    a = kg >= thr ? b : a;
+                }
+                a += lbase;
+#pragma unroll
+                for (int xt = 0; xt < XT; ++xt) {
+                    uint4 q = sm[a + (UP ? 8 : 16) * xt];
+                    if constexpr (32 * ks + 32 > 27 * CIN) // the padded last step: k past the taps
+                        if (32 * ks + 8 * kg >= 27 * CIN)
+                            q = make_uint4(0, 0, 0, 0);
+                    // weights as the A operand: D[co][voxel], each lane 4 channels of one voxel
+#pragma unroll
+                    for (int c = 0; c < CT; ++c)
+                        acc[tl * XT + xt][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            __builtin_bit_cast(bf16x8, qb[c]), __builtin_bit_cast(bf16x8, q),
+                            acc[tl * XT + xt][c], 0, 0, 0);
+                }
+            });
         });
-    });
-    conv_tile_store<CT, NT, XT, LPW, TY>(g, nb, z0, y0, x0, wave, r, kg, acc, bias, add, relu,
-                                         out);
+        conv_tile_store<CT, NT, XT, LPW, TY>(g, nb, z0, y0, x0, wave, r, kg, acc, bias, add, relu,
+                                             out);
+        if (MARCH && step + 1 < steps) {
+            if (!PRE)
+                load_weights(); // the first ones again, in flight over the barriers
+            __syncthreads(); // every wave has read the slots that are replaced
+            store_planes(slot, nnp, nst, nhv);
+            __syncthreads();
+            slot += NP;
+            slot = slot >= SZ ? slot - SZ : slot;
+        }
+    }
 }
 
 // The single-channel input layer (cin = 1, K = 27 taps in one k step of 32) over the same
@@ -692,23 +740,34 @@ __global__ __launch_bounds__(256) void k_reduce_parts(const float *__restrict__ 
 }
 
 // ---- elementwise layers ----
-// 2x2x2 average pooling (fine dims g, coarse g/2), C channels
+// 2x2x2 average pooling (fine dims g, coarse g/2), 8 of the C channels per thread
 __global__ void k_pool(Dims gf, int C, const bf16_t *__restrict__ in, bf16_t *__restrict__ out) {
-    const int D = gf.d / 2, H = gf.h / 2, W = gf.w / 2;
-    const int64_t n = (int64_t)gf.n * D * H * W * C;
+    const int D = gf.d / 2, H = gf.h / 2, W = gf.w / 2, C8 = C / 8;
+    const int64_t n = (int64_t)gf.n * D * H * W * C8;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i % C);
-        int64_t v = i / C;
+        const int c = (int)(i % C8);
+        const int64_t v = i / C8;
         const int x = (int)(v % W), y = (int)((v / W) % H), z = (int)((v / ((int64_t)W * H)) % D);
         const int b = (int)(v / ((int64_t)W * H * D));
-        float s = 0.f;
+        float s[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            s[j] = 0.f;
+#pragma unroll
         for (int q = 0; q < 8; ++q) {
             const int64_t f = (((int64_t)b * gf.d + 2 * z + (q >> 2)) * gf.h + 2 * y + ((q >> 1) & 1)) *
                                   gf.w + 2 * x + (q & 1);
-            s = s + bf2f(in[f * C + c]);
+            const Bf8 u = ld8(in + f * C + 8 * c);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                s[j] = s[j] + bf2f(u.e[j]);
         }
-        out[i] = f2bf(s * 0.125f);
+        Bf8 o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            o.e[j] = f2bf(s[j] * 0.125f);
+        st8(out + v * C + 8 * c, o);
     }
 }
 
@@ -1309,9 +1368,15 @@ template <int NCG, int CT, int TY, bool UP, int TX = kTX>
 void launch_conv_tile(const Dims &g, const bf16_t *in, const bf16_t *wt, int kpad,
                       const float *bias, const bf16_t *add, int relu, bf16_t *out,
                       hipStream_t s) {
-    const dim3 grid((unsigned)(g.vox() / (TX * TY * kTZ))), blk(256);
+    // z steps of a workgroup: up to 8, a divisor of the volume's, while 2048 workgroups are
+    // left to balance the chip
+    const int64_t tiles = g.vox() / (TX * TY * kTZ);
+    int mz = 1;
+    while (conv_marches<NCG, CT, UP> && mz < 8 && (g.d / kTZ) % (2 * mz) == 0 && tiles / (2 * mz) >= 2048)
+        mz *= 2;
+    const dim3 grid((unsigned)(tiles / mz)), blk(256);
     hipLaunchKernelGGL((k_conv_tile<NCG, CT, TY, UP, TX>), grid, blk, 0, s, g, in, wt, kpad,
-                       bias, add, relu, out);
+                       bias, add, relu, mz, out);
 }
 
 // up: `in` is the coarse input of a nearest x2 upsampling onto g (fused)
@@ -1494,7 +1559,7 @@ void forward(xh_unet_s *U, Work &W, bool infer = false) {
         conv_fwd(U, U->enc[2 * l], g, W.in[l], nullptr, true, W.a[l]);
         conv_fwd(U, U->enc[2 * l + 1], g, W.a[l], nullptr, true, W.s[l]);
         if (l + 1 < L) {
-            const int64_t n = W.g[l + 1].vox() * U->ch[l];
+            const int64_t n = W.g[l + 1].vox() * U->ch[l] / 8;
             hipLaunchKernelGGL(k_pool, dim3(grid1(n)), dim3(256), 0, st, g, U->ch[l], W.s[l], W.in[l + 1]);
         }
     }
