@@ -121,11 +121,17 @@ __global__ __launch_bounds__(256) void k_conv(Dims g, const bf16_t *__restrict__
 #pragma unroll
         for (int c = 0; c < CT; ++c)
             acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // tap and channel of the lane's first k, advanced by 32 per step (cin % 8 == 0)
+    // The operands of the next PF k steps are in flight while a step computes: on the deep
+    // levels (a few hundred waves, 54 steps of 64 channels) a step otherwise waits a memory
+    // round trip (16 volumes of 4^3, 64 channels: 77 -> 29 us).
+    constexpr int PF = 3;
+    bf16x8 a[PF][MT];
+    uint4 qb[PF][CT];
+    // tap and channel of the lane's k in the step being loaded, advanced by 32 per step
+    // (cin % 8 == 0)
     int tt = (8 * kg) / cin, cc = 8 * kg - tt * cin;
-    for (int kb = 0; kb < kpad; kb += 32) {
+    auto load = [&](int kb, bf16x8 (&av)[MT], uint4 (&bv)[CT]) __attribute__((always_inline)) {
         const int k0 = kb + 8 * kg;
-        bf16x8 a[MT];
         if (UP || (cin & 7) == 0) { // the fused upsampling is only used with cin % 8 == 0
             // 8 consecutive channels of one tap
             const int dz = tt / 9 - 1, dy = (tt / 3) % 3 - 1, dx = tt % 3 - 1;
@@ -143,7 +149,7 @@ __global__ __launch_bounds__(256) void k_conv(Dims g, const bf16_t *__restrict__
                         nb = m0 + 16 * t + r + ((int64_t)dz * g.h + dy) * g.w + dx;
                     q = *reinterpret_cast<const uint4 *>(in + nb * cin + cc);
                 }
-                a[t] = __builtin_bit_cast(bf16x8, q);
+                av[t] = __builtin_bit_cast(bf16x8, q);
             }
             cc += 32;
             while (cc >= cin) {
@@ -172,16 +178,31 @@ __global__ __launch_bounds__(256) void k_conv(Dims g, const bf16_t *__restrict__
                     }
                     e[j] = v;
                 }
-                a[t] = pack8(e);
+                av[t] = pack8(e);
             }
         }
 #pragma unroll
-        for (int c = 0; c < CT; ++c) {
-            const uint4 qb = *reinterpret_cast<const uint4 *>(wt + (size_t)(c * 16 + r) * kpad + k0);
+        for (int c = 0; c < CT; ++c)
+            bv[c] = *reinterpret_cast<const uint4 *>(wt + (size_t)(c * 16 + r) * kpad + k0);
+    };
 #pragma unroll
-            for (int t = 0; t < MT; ++t)
-                acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                    a[t], __builtin_bit_cast(bf16x8, qb), acc[t][c], 0, 0, 0);
+    for (int q = 0; q < PF; ++q)
+        if (32 * q < kpad)
+            load(32 * q, a[q], qb[q]);
+    for (int kb = 0; kb < kpad; kb += 32 * PF) {
+#pragma unroll
+        for (int q = 0; q < PF; ++q) {
+            const int ks = kb + 32 * q;
+            if (ks < kpad) { // uniform
+#pragma unroll
+                for (int c = 0; c < CT; ++c)
+#pragma unroll
+                    for (int t = 0; t < MT; ++t)
+                        acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            a[q][t], __builtin_bit_cast(bf16x8, qb[q][c]), acc[t][c], 0, 0, 0);
+                if (ks + 32 * PF < kpad)
+                    load(ks + 32 * PF, a[q], qb[q]);
+            }
         }
     }
 #pragma unroll
