@@ -250,7 +250,8 @@ __device__ __forceinline__ void conv_tile_store(const Dims &g, int nb, int z0, i
                                                 int wave, int r, int kg,
                                                 const f32x4 (&acc)[NT][CT],
                                                 const float *__restrict__ bias,
-                                                const bf16_t *__restrict__ add, int relu,
+                                                const bf16_t *__restrict__ add,
+                                                const bf16_t *__restrict__ mask, int relu,
                                                 bf16_t *__restrict__ out) {
     constexpr int COUT = 16 * CT;
     float bv[CT][4];
@@ -283,6 +284,13 @@ __device__ __forceinline__ void conv_tile_store(const Dims &g, int nb, int z0, i
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     v[i] = v[i] > 0.f ? v[i] : 0.f;
+            if (mask) { // gradient through the relu that made `mask`
+                const uint2 a = *reinterpret_cast<const uint2 *>(mask + o0);
+                v[0] = bf2f((bf16_t)(a.x & 0xffffu)) > 0.f ? v[0] : 0.f;
+                v[1] = bf2f((bf16_t)(a.x >> 16)) > 0.f ? v[1] : 0.f;
+                v[2] = bf2f((bf16_t)(a.y & 0xffffu)) > 0.f ? v[2] : 0.f;
+                v[3] = bf2f((bf16_t)(a.y >> 16)) > 0.f ? v[3] : 0.f;
+            }
             uint2 o;
             o.x = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
             o.y = (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
@@ -302,7 +310,8 @@ template <int NCG, int CT, int TY, bool UP, int TX = kTX>
 __global__ __launch_bounds__(256) void k_conv_tile(Dims g, const bf16_t *__restrict__ in,
                                                    const bf16_t *__restrict__ wt, int kpad,
                                                    const float *__restrict__ bias,
-                                                   const bf16_t *__restrict__ add, int relu,
+                                                   const bf16_t *__restrict__ add,
+                                                   const bf16_t *__restrict__ mask, int relu,
                                                    int mz, bf16_t *__restrict__ out) {
     constexpr int CIN = 8 * NCG;
     constexpr int TXS = UP ? TX / 2 : TX;     // staged voxels of a line without its halo
@@ -489,8 +498,8 @@ __global__ __launch_bounds__(256) void k_conv_tile(Dims g, const bf16_t *__restr
                 }
             });
         });
-        conv_tile_store<CT, NT, XT, LPW, TY>(g, nb, z0, y0, x0, wave, r, kg, acc, bias, add, relu,
-                                             out);
+        conv_tile_store<CT, NT, XT, LPW, TY>(g, nb, z0, y0, x0, wave, r, kg, acc, bias, add, mask,
+                                             relu, out);
         if (MARCH && step + 1 < steps) {
             if (!PRE)
                 load_weights(); // the first ones again, in flight over the barriers
@@ -506,17 +515,18 @@ __global__ __launch_bounds__(256) void k_conv_tile(Dims g, const bf16_t *__restr
 // The single-channel input layer (cin = 1, K = 27 taps in one k step of 32) over the same
 // tiles: the staged line holds one bf16 per voxel and each lane assembles its 8 taps of
 // the A fragment from LDS, as k_conv assembles them from element gathers.
+template <int TX>
 __global__ __launch_bounds__(256) void k_conv_tile1(Dims g, const bf16_t *__restrict__ in,
                                                     const bf16_t *__restrict__ wt, int kpad,
                                                     const float *__restrict__ bias, int relu,
                                                     bf16_t *__restrict__ out) {
-    constexpr int SZ = kTZ + 2, SY = kTY + 2, SX = kTX + 2;
+    constexpr int SZ = kTZ + 2, SY = kTY + 2, SX = TX + 2;
     constexpr int NS = SZ * SY * SX;
     constexpr int PER = (NS + 255) / 256;
-    constexpr int XT = kTX / 16, LPW = kTZ * kTY / 4, NT = LPW * XT;
+    constexpr int XT = TX / 16, LPW = kTZ * kTY / 4, NT = LPW * XT;
     __shared__ bf16_t sm[NS];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int ntx = g.w / kTX, nty = g.h / kTY, ntz = g.d / kTZ;
+    const int ntx = g.w / TX, nty = g.h / kTY, ntz = g.d / kTZ;
     int64_t bid = blockIdx.x;
     const int tx = (int)(bid % ntx);
     bid /= ntx;
@@ -524,7 +534,7 @@ __global__ __launch_bounds__(256) void k_conv_tile1(Dims g, const bf16_t *__rest
     bid /= nty;
     const int tz = (int)(bid % ntz);
     const int nb = (int)(bid / ntz);
-    const int x0 = tx * kTX, y0 = ty * kTY, z0 = tz * kTZ;
+    const int x0 = tx * TX, y0 = ty * kTY, z0 = tz * kTZ;
     {
         bf16_t st[PER];
 #pragma unroll
@@ -566,7 +576,7 @@ __global__ __launch_bounds__(256) void k_conv_tile1(Dims g, const bf16_t *__rest
             __builtin_bit_cast(bf16x8, qb), pack8(e), f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     }
     conv_tile_store<1, NT, XT, LPW, kTY>(g, nb, z0, y0, x0, wave, r, kg, acc, bias, nullptr,
-                                         relu, out);
+                                         nullptr, relu, out);
 }
 
 // ---- weight gradient ----
@@ -1385,85 +1395,71 @@ void launch_conv(const Dims &g, const bf16_t *in, int cin, const bf16_t *wt, int
 // 0: every forward convolution runs as k_conv (no LDS-staged tiles)
 int g_conv_tile = 1;
 
-template <int NCG, int CT, int TY, bool UP, int TX = kTX>
-void launch_conv_tile(const Dims &g, const bf16_t *in, const bf16_t *wt, int kpad,
-                      const float *bias, const bf16_t *add, int relu, bf16_t *out,
-                      hipStream_t s) {
+template <int NCG, int CT, int TY, bool UP, int TX>
+bool launch_conv_tile(const Dims &g, const bf16_t *in, const bf16_t *wt, int kpad,
+                      const float *bias, const bf16_t *add, const bf16_t *mask, int relu,
+                      bf16_t *out, hipStream_t s) {
     // z steps of a workgroup: up to 8, a divisor of the volume's, while 2048 workgroups are
     // left to balance the chip
     const int64_t tiles = g.vox() / (TX * TY * kTZ);
     int mz = 1;
-    while (conv_marches<NCG, CT, UP> && mz < 8 && (g.d / kTZ) % (2 * mz) == 0 && tiles / (2 * mz) >= 2048)
+    while (conv_marches<NCG, CT, UP> && mz < 8 && (g.d / kTZ) % (2 * mz) == 0 &&
+           tiles / (2 * mz) >= 2048)
         mz *= 2;
     const dim3 grid((unsigned)(tiles / mz)), blk(256);
     hipLaunchKernelGGL((k_conv_tile<NCG, CT, TY, UP, TX>), grid, blk, 0, s, g, in, wt, kpad,
-                       bias, add, relu, mz, out);
+                       bias, add, mask, relu, mz, out);
+    return true;
+}
+
+// The convolution cin -> cout over LDS-staged tiles, if it has a tile kernel and the tiles
+// divide the volume (false: nothing launched).  16 output channels on lines of 64 or 32
+// voxels, 32 on lines of 64, 48 on lines of 32 (the widths those layers have at 128^3 and on
+// 32^3 crops); the staged input is at most 68 KB: 32 plain input channels take tiles of 2
+// lines.  16 crops of 32^3, 16 -> 16: 26 us, 59 by k_conv.
+bool conv_tiled(const Dims &g, const bf16_t *in, int cin, int cout, const bf16_t *wt, int kpad,
+                const float *bias, const bf16_t *add, const bf16_t *mask, int relu, bf16_t *out,
+                bool up, hipStream_t st) {
+    if (!g_conv_tile || g.h % kTY || g.d % kTZ || g.w % 32)
+        return false;
+    const bool wide = g.w % 64 == 0;
+    if (cin == 1 && cout == 16 && !up && !add && !mask) {
+        const dim3 grid((unsigned)(g.vox() / ((wide ? 64 : 32) * kTY * kTZ))), blk(256);
+        hipLaunchKernelGGL(wide ? k_conv_tile1<64> : k_conv_tile1<32>, grid, blk, 0, st, g, in, wt,
+                           kpad, bias, relu, out);
+        return true;
+    }
+#define XH_TILE(CIN, COUT, UPV, NCG, CT, TY, TX)                                               \
+    if (cin == CIN && cout == COUT && up == UPV && g.w % TX == 0)                              \
+        return launch_conv_tile<NCG, CT, TY, UPV, TX>(g, in, wt, kpad, bias, add, mask, relu,  \
+                                                      out, st);
+    XH_TILE(16, 16, false, 2, 1, 4, 64)
+    XH_TILE(16, 16, true, 2, 1, 4, 64)
+    XH_TILE(32, 16, true, 4, 1, 4, 64)
+    XH_TILE(16, 16, false, 2, 1, 4, 32)
+    XH_TILE(32, 16, true, 4, 1, 4, 32)
+    XH_TILE(16, 32, false, 2, 2, 4, 64)
+    XH_TILE(32, 32, false, 4, 2, 2, 64)
+    XH_TILE(32, 32, true, 4, 2, 4, 64)
+    XH_TILE(48, 32, true, 6, 2, 4, 64)
+    XH_TILE(16, 32, false, 2, 2, 4, 32)
+    XH_TILE(32, 48, false, 4, 3, 4, 32)
+    XH_TILE(48, 48, false, 6, 3, 2, 32)
+    XH_TILE(64, 48, true, 8, 3, 4, 32)
+#undef XH_TILE
+    return false;
 }
 
 // up: `in` is the coarse input of a nearest x2 upsampling onto g (fused)
 void conv_fwd(xh_unet_s *U, const Conv &c, const Dims &g, const bf16_t *in, const bf16_t *add,
               bool relu, bf16_t *out, bool up = false) {
-    // 16 or 32 output channels on volumes the tiles divide: LDS-staged tiles (the staged
-    // input at most 68 KB: 32 plain input channels take tiles of 2 lines)
-    const bool tiles = g_conv_tile && g.w % kTX == 0 && g.h % kTY == 0 && g.d % kTZ == 0;
-    hipStream_t st = U->stream;
-    const int rl = (int)relu;
-    if (tiles && c.cout == 16 && c.cin == 1 && !up && !add) {
-        const dim3 grid((unsigned)(g.vox() / (kTX * kTY * kTZ))), blk(256);
-        hipLaunchKernelGGL(k_conv_tile1, grid, blk, 0, st, g, in, c.wt, c.kpad, c.b, rl, out);
+    if (conv_tiled(g, in, c.cin, c.cout, c.wt, c.kpad, c.b, add, nullptr, (int)relu, out, up,
+                   U->stream))
         return;
-    }
-    if (tiles && c.cout == 16) {
-        if (c.cin == 16 && !up) {
-            launch_conv_tile<2, 1, 4, false>(g, in, c.wt, c.kpad, c.b, add, rl, out, st);
-            return;
-        }
-        if (c.cin == 16 && up) {
-            launch_conv_tile<2, 1, 4, true>(g, in, c.wt, c.kpad, c.b, add, rl, out, st);
-            return;
-        }
-        if (c.cin == 32 && up) {
-            launch_conv_tile<4, 1, 4, true>(g, in, c.wt, c.kpad, c.b, add, rl, out, st);
-            return;
-        }
-    }
-    if (tiles && c.cout == 32) {
-        if (c.cin == 16 && !up) {
-            launch_conv_tile<2, 2, 4, false>(g, in, c.wt, c.kpad, c.b, add, rl, out, st);
-            return;
-        }
-        if (c.cin == 32 && !up) {
-            launch_conv_tile<4, 2, 2, false>(g, in, c.wt, c.kpad, c.b, add, rl, out, st);
-            return;
-        }
-        if (c.cin == 32 && up) {
-            launch_conv_tile<4, 2, 4, true>(g, in, c.wt, c.kpad, c.b, add, rl, out, st);
-            return;
-        }
-        if (c.cin == 48 && up) {
-            launch_conv_tile<6, 2, 4, true>(g, in, c.wt, c.kpad, c.b, add, rl, out, st);
-            return;
-        }
-    }
-    // 48 output channels on lines of 32 voxels (the third level of a 128^3 grid)
-    if (g_conv_tile && c.cout == 48 && g.w % 32 == 0 && g.h % kTY == 0 && g.d % kTZ == 0) {
-        if (c.cin == 32 && !up) {
-            launch_conv_tile<4, 3, 4, false, 32>(g, in, c.wt, c.kpad, c.b, add, rl, out, st);
-            return;
-        }
-        if (c.cin == 48 && !up) {
-            launch_conv_tile<6, 3, 2, false, 32>(g, in, c.wt, c.kpad, c.b, add, rl, out, st);
-            return;
-        }
-        if (c.cin == 64 && up) {
-            launch_conv_tile<8, 3, 4, true, 32>(g, in, c.wt, c.kpad, c.b, add, rl, out, st);
-            return;
-        }
-    }
 #define XH_CONV_CASE(CTV)                                                                      \
     if (up)                                                                                    \
         launch_conv<CTV, true>(g, in, c.cin, c.wt, c.kpad, c.b, add, nullptr, (int)relu,      \
-                               out, U->stream);                                                     \
+                               out, U->stream);                                                \
     else                                                                                       \
         launch_conv<CTV, false>(g, in, c.cin, c.wt, c.kpad, c.b, add, nullptr, (int)relu,     \
                                 out, U->stream);
@@ -1488,6 +1484,9 @@ void conv_fwd(xh_unet_s *U, const Conv &c, const Dims &g, const bf16_t *in, cons
 // activation that conv read, whose relu the gradient goes through
 void conv_data(xh_unet_s *U, const Conv &c, const Dims &g, const bf16_t *gout,
                const bf16_t *mask, bf16_t *gin) {
+    if (conv_tiled(g, gout, c.cout, c.cin, c.wtf, c.kpadf, nullptr, nullptr, mask, 0, gin, false,
+                   U->stream))
+        return;
     switch (c.cin / 16) {
     case 1:
         launch_conv<1>(g, gout, c.cout, c.wtf, c.kpadf, nullptr, nullptr, mask, 0, gin, U->stream);

@@ -67,6 +67,7 @@ def test_loss_and_gradients_match_oracle(gpu, channels, size, batch):
 
 @pytest.mark.parametrize("channels,dims", [
     ((16, 32, 48, 64), (3, 8, 16, 24)),  # levels down to 1 x 2 x 3 voxels, several samples
+    ((16, 32), (2, 6, 8, 32)),           # tiles of 32-voxel lines, data gradients too
     ((64,), (1, 5, 3, 7)),               # one level, no edge a power of two
     ((48, 16), (2, 6, 10, 34)),          # lines just over a box edge, 16 -> 48 upsampling
     ((32, 64), (1, 2, 2, 66)),
@@ -188,6 +189,25 @@ def test_tiled_convolution_is_identical(gpu):
     finally:
         X.set_option("unet_conv_tile", 1)
         X.set_option("unet_fuse_up", 1)
+
+
+def test_narrow_tiles_are_identical(gpu):
+    # 32-voxel lines (w % 64 != 0): tiles against the per-tap gathers, one and many z steps
+    X = gpu
+    net = X.UNet((16, 32), seed=5)
+    try:
+        for (nx, ny, nz), nv in (((32, 8, 8), 1), ((96, 16, 24), 4), ((32, 32, 32), 16)):
+            V = nx * ny * nz
+            b = X.DeviceArray.from_host(np.random.default_rng(nx + nv).standard_normal(V * nv))
+            outs = []
+            for tile in (0, 1):
+                X.set_option("unet_conv_tile", tile)
+                x = X.DeviceArray(V * nv)
+                net.infer(nx, ny, nz, nv, b, x)
+                outs.append(x.to_host())
+            assert np.array_equal(outs[0], outs[1]), (nx, ny, nz)
+    finally:
+        X.set_option("unet_conv_tile", 1)
 
 
 @pytest.mark.parametrize("nv", [2, 3])
