@@ -260,6 +260,7 @@ struct SolverState {
     int nv, max_iters, conv_check, hist_len;
     float abs_tol, rel_tol;
     double *hist; // [hist_len][nv] sqrt(res) per convergence check, or nullptr
+    double *x;    // the solution vector of the solve (single-system solves)
     unsigned long long t_done; // device wall clock (wall_clock64) when `done` was set
 };
 
@@ -338,8 +339,10 @@ enum VecOp : int {
     V_RB_UPDATE_MERGED = 15,
 };
 
+// x of the ops that update it is SolverState::x, set at the start of a solve: a captured
+// iteration then does not depend on the caller's vector
 struct VecArgs {
-    void *x = nullptr, *p = nullptr, *s = nullptr, *r = nullptr, *r0 = nullptr;
+    void *p = nullptr, *s = nullptr, *r = nullptr, *r0 = nullptr;
     const void *v = nullptr, *t = nullptr, *b = nullptr, *p_ = nullptr, *s_ = nullptr;
     SolverState *st = nullptr;
     double *partials = nullptr;

@@ -1008,7 +1008,7 @@ int enqueue_replacement(xh_solver_s *S, double *x) {
 }
 
 // one PCG iteration (pcg.inl:101-160)
-void enqueue_iteration_pcg(xh_solver_s *S, double *x) {
+void enqueue_iteration_pcg(xh_solver_s *S) {
     const int nv = S->nv;
     hipStream_t st = S->stream;
     SpmvArgs a = args(S);
@@ -1018,7 +1018,6 @@ void enqueue_iteration_pcg(xh_solver_s *S, double *x) {
     finalize(FIN_CG_ALPHA, S->st, S->partials, np, nv, st);
     VecArgs vx;
     vx.st = S->st;
-    vx.x = x;
     vx.p_ = S->p;
     vx.t = S->v;
     vx.r = S->r;
@@ -1040,7 +1039,7 @@ void enqueue_iteration_pcg(xh_solver_s *S, double *x) {
 
 // one RBiCGStab / MergedRBiCGStab iteration (rbicgstab.inl:124-216,
 // merged_rbicgstab.inl:124-216)
-void enqueue_iteration_rbicgstab(xh_solver_s *S, double *x, bool merged) {
+void enqueue_iteration_rbicgstab(xh_solver_s *S, bool merged) {
     const int nv = S->nv;
     hipStream_t st = S->stream;
     SpmvArgs a = args(S);
@@ -1066,7 +1065,6 @@ void enqueue_iteration_rbicgstab(xh_solver_s *S, double *x, bool merged) {
     precond(S, S->t, S->p_);                              // 14: z = M^{-1} t
     VecArgs vu;
     vu.st = S->st;
-    vu.x = x;
     vu.p = S->p;
     vu.s = S->p_;
     vu.r = S->r;
@@ -1080,9 +1078,9 @@ void enqueue_iteration_rbicgstab(xh_solver_s *S, double *x, bool merged) {
 void enqueue_iteration(xh_solver_s *S, double *x, bool replace) {
     const int m = S->prm.solver.method;
     if (m == XH_PCG)
-        return enqueue_iteration_pcg(S, x);
+        return enqueue_iteration_pcg(S);
     if (is_rbicgstab(m))
-        return enqueue_iteration_rbicgstab(S, x, m == XH_MERGED_RBICGSTAB);
+        return enqueue_iteration_rbicgstab(S, m == XH_MERGED_RBICGSTAB);
     const int nv = S->nv;
     hipStream_t st = S->stream;
     const bool pre = is_preconditioned(m);
@@ -1111,8 +1109,7 @@ void enqueue_iteration(xh_solver_s *S, double *x, bool replace) {
         finalize(FIN_OMEGA_MERGED, S->st, S->partials, np, nv, st);
         VecArgs vx;
         vx.st = S->st;
-        vx.x = x;
-        vx.p_ = S->p;
+            vx.p_ = S->p;
         vx.s_ = S->s;
         vx.gate = 1;
         vec_op(V_X_UPDATE, S->n, nv, vx, st);
@@ -1127,8 +1124,7 @@ void enqueue_iteration(xh_solver_s *S, double *x, bool replace) {
         finalize(FIN_BETA, S->st, S->partials, np, nv, st);
         VecArgs v5;
         v5.st = S->st;
-        v5.x = x;
-        v5.p = S->p;
+            v5.p = S->p;
         v5.s = S->s;
         v5.r = S->r;
         v5.v = S->v;
@@ -1138,7 +1134,6 @@ void enqueue_iteration(xh_solver_s *S, double *x, bool replace) {
     finalize(FIN_OMEGA, S->st, S->partials, np, nv, st);
     VecArgs vx;
     vx.st = S->st;
-    vx.x = x;
     vx.p_ = pp;
     vx.s_ = ss;
     vx.s = S->s;
@@ -1194,6 +1189,7 @@ int solve_impl(xh_solver_s *S, const double *db, double *dx) {
     h.rel_tol = S->prm.solver.rel_tol;
     h.hist = S->hist;
     h.hist_len = S->hist_len;
+    h.x = dx;
     XH_HIP(hipMemcpyAsync(S->st, S->hst, sizeof(SolverState), hipMemcpyHostToDevice, S->stream));
     S->dflag = &S->st->done;
     if (g_ledger) {
@@ -1207,7 +1203,10 @@ int solve_impl(xh_solver_s *S, const double *db, double *dx) {
     const bool use_graph = S->prm.graph != 0;
     const int period = S->prm.true_res_period;
     S->bcur = db;
-    if (use_graph && (S->gexec == nullptr || S->g_x != dx || S->g_b != db)) {
+    // an iteration reads x from the solver state and b not at all, so its graph serves every
+    // solve (capturing it anew for another x cost ~0.3 ms); only a residual replacement
+    // (period > 0) holds both vectors
+    if (use_graph && (S->gexec == nullptr || (period > 0 && (S->g_x != dx || S->g_b != db)))) {
         free_graphs(S);
         XH_HIP(hipStreamBeginCapture(S->stream, hipStreamCaptureModeThreadLocal));
         enqueue_iteration(S, dx, false);

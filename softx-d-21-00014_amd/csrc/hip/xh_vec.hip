@@ -54,8 +54,7 @@ __device__ __forceinline__ void block_partials(double (&p)[ND], double *__restri
 enum Gate : int { GATE_NOT_DONE = 0, GATE_CONV_ALL = 1 };
 
 template <int NV, int OP>
-__global__ __launch_bounds__(kBlock) void k_vec(int64_t n, int64_t chunk, double *__restrict__ x,
-                                                double *__restrict__ p, double *__restrict__ s,
+__global__ __launch_bounds__(kBlock) void k_vec(int64_t n, int64_t chunk, double *__restrict__ p, double *__restrict__ s,
                                                 double *__restrict__ r,
                                                 const double *__restrict__ r0,
                                                 const double *__restrict__ v,
@@ -74,6 +73,11 @@ __global__ __launch_bounds__(kBlock) void k_vec(int64_t n, int64_t chunk, double
         : (OP == V_DOT3)                                                             ? 3
                                                                                      : 0;
     constexpr int RPB = kBlock / NV;
+    constexpr bool X = OP == V_XR_UPDATE || OP == V_X_UPDATE || OP == V_GROUP5 || OP == V_CG_XR ||
+                       OP == V_RB_UPDATE || OP == V_RB_UPDATE_MERGED;
+    // global memory: a pointer read from memory would otherwise make flat accesses
+    typedef __attribute__((address_space(1))) double gdouble;
+    gdouble *__restrict__ x = X ? (gdouble *)st->x : nullptr;
     const int64_t lb = logical_block();
     const int64_t start = lb * chunk;
     const int64_t end = start + chunk < n ? start + chunk : n;
@@ -201,7 +205,7 @@ int vec_nv(VecOp op, int64_t n, const VecArgs &a, int gate, hipStream_t s) {
 #define XH_VEC_CASE(OPV)                                                                        \
     case OPV:                                                                                   \
         hipLaunchKernelGGL((k_vec<NV, OPV>), dim3(g), dim3(kBlock), 0, s, n, chunk,             \
-                           (double *)a.x, (double *)a.p, (double *)a.s, (double *)a.r,          \
+                           (double *)a.p, (double *)a.s, (double *)a.r,                         \
                            (const double *)a.r0, (const double *)a.v, (const double *)a.t,      \
                            (const double *)a.p_, (const double *)a.s_, a.st, gate, a.partials); \
         break;
