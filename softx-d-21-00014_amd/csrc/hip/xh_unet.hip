@@ -242,18 +242,45 @@ __global__ __launch_bounds__(256) void k_conv(Dims g, const bf16_t *__restrict__
 // and d % kTZ == 0.
 constexpr int kTX = 64, kTY = 4, kTZ = 2;
 
-// Epilogue of the tiled convolutions: lane (r, kg) of tile t, channel tile c holds
-// channels 16c + 4kg .. 16c + 4kg + 3 of voxel r, written (and `add` read) as 8 bytes.
-// Per element act(acc + bias + add), as in k_conv.
+// The lane's values of a tensor of the output's shape, 8 bytes per tile and channel tile, all
+// loaded before any is used: read tile by tile between the epilogue's stores, each cost the
+// wave a memory latency.  Upsampled tiles at 128^3 and its halving, 32 volumes: 32 -> 16 2266
+// -> 1884 us, 48 -> 32 858 -> 753.  The marching 16 -> 16 kernel, at its registers' limit,
+// lost 9 % with it and reads in place.
 template <int CT, int NT, int XT, int LPW, int TY>
+__device__ __forceinline__ void conv_tile_fetch(const Dims &g, int nb, int z0, int y0, int x0,
+                                                int wave, int r, int kg,
+                                                const bf16_t *__restrict__ src,
+                                                uint2 (&v)[NT][CT]) {
+    constexpr int COUT = 16 * CT;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int li = wave * LPW + t / XT, xt = t % XT;
+        const int iz = li / TY, iy = li % TY;
+        const int64_t line = ((((int64_t)nb * g.d + z0 + iz) * g.h + y0 + iy) * g.w + x0) * COUT;
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+            v[t][c] = *reinterpret_cast<const uint2 *>(
+                src + (line + ((16 * xt + r) * COUT + 16 * c + 4 * kg)));
+    }
+}
+
+// Epilogue of the tiled convolutions: lane (r, kg) of tile t, channel tile c holds
+// channels 16c + 4kg .. 16c + 4kg + 3 of voxel r, written as 8 bytes.  Per element
+// act(acc + bias + add), as in k_conv; av holds `add`.
+template <int CT, int NT, int XT, int LPW, int TY, bool AHEAD>
 __device__ __forceinline__ void conv_tile_store(const Dims &g, int nb, int z0, int y0, int x0,
                                                 int wave, int r, int kg,
                                                 const f32x4 (&acc)[NT][CT],
                                                 const float *__restrict__ bias,
                                                 const bf16_t *__restrict__ add,
+                                                const uint2 (&av)[NT][CT],
                                                 const bf16_t *__restrict__ mask, int relu,
                                                 bf16_t *__restrict__ out) {
     constexpr int COUT = 16 * CT;
+    uint2 mv[NT][CT];
+    if (AHEAD && mask)
+        conv_tile_fetch<CT, NT, XT, LPW, TY>(g, nb, z0, y0, x0, wave, r, kg, mask, mv);
     float bv[CT][4];
 #pragma unroll
     for (int c = 0; c < CT; ++c)
@@ -274,7 +301,7 @@ __device__ __forceinline__ void conv_tile_store(const Dims &g, int nb, int z0, i
             for (int i = 0; i < 4; ++i)
                 v[i] = acc[t][c][i] + bv[c][i];
             if (add) {
-                const uint2 a = *reinterpret_cast<const uint2 *>(add + o0);
+                const uint2 a = AHEAD ? av[t][c] : *reinterpret_cast<const uint2 *>(add + o0);
                 v[0] = v[0] + bf2f((bf16_t)(a.x & 0xffffu));
                 v[1] = v[1] + bf2f((bf16_t)(a.x >> 16));
                 v[2] = v[2] + bf2f((bf16_t)(a.y & 0xffffu));
@@ -285,7 +312,7 @@ __device__ __forceinline__ void conv_tile_store(const Dims &g, int nb, int z0, i
                 for (int i = 0; i < 4; ++i)
                     v[i] = v[i] > 0.f ? v[i] : 0.f;
             if (mask) { // gradient through the relu that made `mask`
-                const uint2 a = *reinterpret_cast<const uint2 *>(mask + o0);
+                const uint2 a = AHEAD ? mv[t][c] : *reinterpret_cast<const uint2 *>(mask + o0);
                 v[0] = bf2f((bf16_t)(a.x & 0xffffu)) > 0.f ? v[0] : 0.f;
                 v[1] = bf2f((bf16_t)(a.x >> 16)) > 0.f ? v[1] : 0.f;
                 v[2] = bf2f((bf16_t)(a.y & 0xffffu)) > 0.f ? v[2] : 0.f;
@@ -406,11 +433,14 @@ __global__ __launch_bounds__(256) void k_conv_tile(Dims g, const bf16_t *__restr
                 sm[at(line) + (w % NCG) * SX + (w >= NCG ? TXS + 1 : 0)] = hv[p];
         }
     };
+    uint2 av[NT][CT]; // the values of `add`
     {
         constexpr int NL = SZ * SY;
         uint4 st[(NL + 3) / 4][IP], hv[(NL * 2 * NCG + 255) / 256];
         const std::integral_constant<int, SZ> np;
         load_planes((UP ? z0 / 2 : z0) - 1, np, st, hv);
+        if (!MARCH && add) // in flight with the staged planes
+            conv_tile_fetch<CT, NT, XT, LPW, TY>(g, nb, z0, y0, x0, wave, r, kg, add, av);
         store_planes(0, np, st, hv);
     }
     // weight fragments, issued once the staged values have left the registers
@@ -498,8 +528,8 @@ __global__ __launch_bounds__(256) void k_conv_tile(Dims g, const bf16_t *__restr
                 }
             });
         });
-        conv_tile_store<CT, NT, XT, LPW, TY>(g, nb, z0, y0, x0, wave, r, kg, acc, bias, add, mask,
-                                             relu, out);
+        conv_tile_store<CT, NT, XT, LPW, TY, !MARCH>(g, nb, z0, y0, x0, wave, r, kg, acc, bias, add,
+                                                     av, mask, relu, out);
         if (MARCH && step + 1 < steps) {
             if (!PRE)
                 load_weights(); // the first ones again, in flight over the barriers
@@ -575,8 +605,9 @@ __global__ __launch_bounds__(256) void k_conv_tile1(Dims g, const bf16_t *__rest
         acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
             __builtin_bit_cast(bf16x8, qb), pack8(e), f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     }
-    conv_tile_store<1, NT, XT, LPW, kTY>(g, nb, z0, y0, x0, wave, r, kg, acc, bias, nullptr,
-                                         nullptr, relu, out);
+    const uint2 av[NT][1] = {}; // no `add` here
+    conv_tile_store<1, NT, XT, LPW, kTY, true>(g, nb, z0, y0, x0, wave, r, kg, acc, bias, nullptr,
+                                               av, nullptr, relu, out);
 }
 
 // ---- weight gradient ----
