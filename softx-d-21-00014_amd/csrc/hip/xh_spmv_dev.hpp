@@ -51,7 +51,7 @@ struct Width {
 };
 
 // Operands of the fused epilogue of one row, loaded by epi_load (right before the
-// epilogue in k_spmv, a few passes ahead in k_spmv_grid).
+// epilogue in k_spmv, a few passes ahead in k_spmv_sweep).
 template <typename VT, int W>
 struct EpiIn {
     Pack<VT, W> a, b, c;

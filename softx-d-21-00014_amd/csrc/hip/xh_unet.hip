@@ -8,7 +8,7 @@
 //   data grad    gin[m][ci] = sum_{t,co} g[m + off_t][co] * W[26 - t][ci][co] (same kernel,
 //                flipped and transposed weights)
 //   weight grad  gW[t][ci][co] = sum_m in[m + off_t][ci] * g[m][co]          (LDS-staged
-//                MFMA per (voxel chunk, tap), chunk partials reduced in fixed order)
+//                MFMA per box of voxels, all taps; partials reduced in fixed order)
 // Weights are fp32 masters (Adam) with bf16 copies in the two GEMM layouts.
 //
 // MFMA 16x16x32 bf16 operand layout (CDNA3/CDNA4): lane l holds A[l % 16][8*(l/16) + j],
@@ -1579,7 +1579,9 @@ void conv_wgrad(xh_unet_s *U, const Conv &c, const Dims &g, const bf16_t *in, co
     const size_t lds = (size_t)((1 << bx.lx) + 2) * ((1 << bx.ly) + 2) * ((1 << bx.lz) + 2) * 32 +
                        ((size_t)CT << lv) * 32;
     const dim3 grid(nchunk, cit), blk(256);
-#define XH_WG(CTV)                                                                                 hipLaunchKernelGGL((k_wgrad<CTV, UP>), grid, blk, lds, U->stream, g, bx, in, c.cin, gout,                         (int)nboxes, U->part, len);
+#define XH_WG(CTV)                                                                              \
+    hipLaunchKernelGGL((k_wgrad<CTV, UP>), grid, blk, lds, U->stream, g, bx, in, c.cin, gout,   \
+                       (int)nboxes, U->part, len);
     switch (CT) {
     case 1:
         XH_WG(1)

@@ -7,8 +7,7 @@
 // merged_rbicgstab_group2 (src/blas/detail/specific/blas_merged_rbicgstab.inl:120-196),
 // base_solver::convergence_check / converged (src/solvers/solver.h:173-241),
 // merged_jacobi (src/blas/detail/specific/blas_merged_jacobi.inl:33-90),
-// dense_Ax_y
-// (src/blas2/detail/dense_matvec.inl:72-121), vector::convert
+// dense_Ax_y (src/blas2/detail/dense_matvec.inl:72-121), vector::convert
 // (src/primitives/vector/operations/convert.inl:31-83).
 //
 // Every expression keeps the reference's operand order; the file is built with
