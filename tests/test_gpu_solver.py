@@ -277,6 +277,30 @@ def test_graph_and_eager_are_identical(gpu):
     assert xs[0][1] == xs[1][1] and np.array_equal(xs[0][0], xs[1][0])
 
 
+@pytest.mark.parametrize("method,period", [("MergedPBiCGStab", 0), ("PBiCGStab", 0), ("PCG", 0),
+                                           ("MergedRBiCGStab", 0), ("MergedPBiCGStab", 2)])
+def test_graph_serves_every_vector(gpu, method, period):
+    # one captured iteration, solves that alternate between vectors: each equals the
+    # eager solve of the same right-hand side, and leaves the other vectors alone
+    X = gpu
+    N, nv = 16, 4
+    levels = levels_for(X, N)
+    S = [X.Solver(X.Hier(levels), X.default_params(method=method, smoother="Chebyshev",
+                                                   poly_order=4, graph=graph,
+                                                   true_res_period=period), nv)
+         for graph in (0, 1)]
+    bs = [X.rhs_uniform(30 + i, N ** 3, nv) for i in range(2)]
+    eager = [S[0].solve(b) for b in bs]
+    db = [X.DeviceArray.from_host(b) for b in bs]
+    dx = [X.DeviceArray(N ** 3 * nv) for _ in range(2)]
+    for i, j in ((0, 0), (1, 1), (1, 0), (0, 1), (0, 1), (0, 0)):
+        other = dx[1 - j].to_host()
+        dx[j].zero()
+        S[1].solve_device(db[i], dx[j])
+        assert np.array_equal(dx[j].to_host(), eager[i])
+        assert np.array_equal(dx[1 - j].to_host(), other, equal_nan=True)
+
+
 def test_hsgs_block_drift_against_exact_gauss_seidel(gpu, O):
     # the GPU HSGS uses many core blocks (Jacobi coupling between them); against the
     # reference at one core (exact symmetric GS) the iteration count drifts by at most 1
