@@ -347,13 +347,14 @@ int xh_batch_get_x(xh_batch B, int s, double *x);
  * the last xh_batch_solve until system s finished (device clock, ms) */
 int xh_batch_stats(xh_batch B, int s, int32_t *iters, int32_t *conv, double *abs_res,
                    double *rel_res, double *latency_ms);
-/* Autotuner: for each nv class present (1, 2, 4, 8, 16) times `reps` batched SpMVs per
- * candidate layout -- RHS per lane (the nv tile width of a lane: 1, or 2 for nv >= 2, so
- * nv or nv/2 lanes per row) times work-item size (1..32 passes of 256*w/nv rows) -- and
- * keeps the fastest; tile_passes (nullable) receives the 5 pass choices.
+/* Autotuner: for each nv class present (1, 2, 4, 8, 16) times `reps` batched Chebyshev
+ * steps (vector updates where the preconditioner is no polynomial) per candidate layout --
+ * RHS per lane (the nv tile width of a lane: 1, or 2 for nv >= 2, so nv or nv/2 lanes per
+ * row) times work-item size (1..32 passes of 256*w/nv rows) -- and keeps the fastest;
+ * tile_passes (nullable) receives the 5 pass choices.
  * xh_batch_set_tiles sets the passes, xh_batch_set_layout passes and RHS per lane,
- * xh_batch_get_layout reads both.  The layout changes only the grouping of the dot
- * partial sums, not any RHS's arithmetic. */
+ * xh_batch_get_layout reads both.  The layout is that of the operations without dot
+ * products; those with dots run in a fixed layout, so no layout changes the results. */
 int xh_batch_autotune(xh_batch B, int reps, int32_t *tile_passes);
 /* Times `reps` launches of the batched Chebyshev step (y = D^-1/2 (c r + D^-1/2 A u), the
  * preconditioner's SpMV) over every work item with every system active; returns the mean

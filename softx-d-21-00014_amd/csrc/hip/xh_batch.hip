@@ -9,7 +9,9 @@
 // order without FMA contraction (csr_Ax_y, src/blas2/detail/csr_matvec.inl:149-260), the
 // Chebyshev steps of chebyshev.inl:179-196 and the BiCGStab updates of
 // src/solvers/detail/pbicgstab.inl:141-230; dot partials go one block per item and are
-// reduced per system, in item order, by finalize_body.
+// reduced per system, in item order, by finalize_body.  The operations with dots walk a work
+// list of their own, fixed by each system's size and RHS count: the item decides which rows
+// a partial sums, so a list chosen by timing would let the clock choose the rounding.
 #include "xh_internal.hpp"
 #include "xh_krylov.hpp"
 
@@ -43,8 +45,8 @@ __device__ __forceinline__ void item_partials(const double (&part)[3][W], int nd
 
 // One work item of one batched operation with W right-hand sides per lane (L = nv/W
 // lanes per row, kBlock/L rows per pass).  Each RHS gets the arithmetic of the
-// single-system kernels; W changes only which lane holds it and so the grouping of the
-// dot partials.
+// single-system kernels; W changes only which lane holds it and, where the operation has
+// dots, the grouping of their partials.
 template <int OP, int W, int L>
 __device__ __forceinline__ void batch_item(const BatchDev &d, const BatchItem &w,
                                            const BatchVecs &v, int ci, int last,
@@ -342,15 +344,17 @@ __global__ __launch_bounds__(kBlock) void k_batch(BatchDev d, const BatchItem *_
     batch_phase<OP>(d, items, n, v, ci, last, partials, blockIdx.x, gridDim.x);
 }
 
-// Work list of the systems not yet done: workgroup s copies system s's items (when it is
-// not done) to the position after the items of the active systems before it; workgroup 0
-// writes the total.  Every workgroup reads the same done flags (set by earlier launches).
-__global__ __launch_bounds__(256) void k_batch_compact(const BatchItem *__restrict__ items,
-                                                       const int *__restrict__ item_start,
-                                                       const int *__restrict__ item_count,
+// Work lists of the systems not yet done (blockIdx.y: which of the two): workgroup s copies
+// system s's items (when it is not done) to the position after the items of the active
+// systems before it; workgroup 0 writes the total.  Every workgroup reads the same done
+// flags (set by earlier launches).
+__global__ __launch_bounds__(256) void k_batch_compact(BatchList la, BatchList lb,
                                                        const SolverState *__restrict__ st,
-                                                       int nsys, BatchItem *__restrict__ out,
-                                                       int *__restrict__ nact) {
+                                                       int nsys) {
+    const BatchList l = blockIdx.y == 0 ? la : lb;
+    const BatchItem *__restrict__ items = l.items;
+    const int *__restrict__ item_start = l.start;
+    const int *__restrict__ item_count = l.count;
     const int s = blockIdx.x;
     __shared__ int s_off;
     if (threadIdx.x == 0) {
@@ -362,7 +366,7 @@ __global__ __launch_bounds__(256) void k_batch_compact(const BatchItem *__restri
             int tot = 0;
             for (int q = 0; q < nsys; ++q)
                 tot += st[q].done ? 0 : item_count[q];
-            *nact = tot;
+            *l.nact = tot;
         }
     }
     __syncthreads();
@@ -370,7 +374,7 @@ __global__ __launch_bounds__(256) void k_batch_compact(const BatchItem *__restri
         return;
     const int b = item_start[s], c = item_count[s], off = s_off;
     for (int q = threadIdx.x; q < c; q += blockDim.x)
-        out[off + q] = items[b + q];
+        l.act[off + q] = items[b + q];
 }
 
 __global__ __launch_bounds__(256) void k_batch_finalize(int op, SolverState *__restrict__ st,
@@ -518,7 +522,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_solve(BatchSolve P) {
         v.out = P.r0;
         v.out2 = P.p;
         v.out3 = P.r;
-        batch_phase<B_RESID0>(d, P.items, P.nitems, v, 0, 0, P.partials, wg, nwg);
+        batch_phase<B_RESID0>(d, P.dot_items, P.ndot_items, v, 0, 0, P.partials, wg, nwg);
         if (!sync() || !fin(FIN_INIT))
             return;
     }
@@ -541,7 +545,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_solve(BatchSolve P) {
         v1.in = pp;
         v1.o1 = P.r0;
         v1.out = P.v;
-        batch_phase<B_DOT1>(d, P.items, P.nitems, v1, 0, 0, P.partials, wg, nwg);
+        batch_phase<B_DOT1>(d, P.dot_items, P.ndot_items, v1, 0, 0, P.partials, wg, nwg);
         if (!sync() || !fin(FIN_ALPHA))
             return;
         BatchVecs vs;
@@ -557,7 +561,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_solve(BatchSolve P) {
         v3.in = ss;
         v3.o1 = P.s;
         v3.out = P.t;
-        batch_phase<B_DOT3>(d, P.items, P.nitems, v3, 0, 0, P.partials, wg, nwg);
+        batch_phase<B_DOT3>(d, P.dot_items, P.ndot_items, v3, 0, 0, P.partials, wg, nwg);
         if (!sync() || !fin(FIN_OMEGA))
             return;
         BatchVecs vx;
@@ -568,7 +572,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_solve(BatchSolve P) {
         vx.t = P.t;
         vx.o1 = P.r0;
         vx.out = P.r;
-        batch_phase<B_XR_UPDATE>(d, P.items, P.nitems, vx, 0, 0, P.partials, wg, nwg);
+        batch_phase<B_XR_UPDATE>(d, P.dot_items, P.ndot_items, vx, 0, 0, P.partials, wg, nwg);
         if (!sync() || !fin(FIN_BETA))
             return;
         BatchVecs vp;
@@ -635,11 +639,9 @@ void batch_finalize(FinOp op, SolverState *st, const double *partials, const int
                        item_start, item_count, nvs);
 }
 
-void batch_compact(const BatchItem *items, const int *item_start, const int *item_count,
-                   const SolverState *st, int nsys, BatchItem *items_act, int *nact,
+void batch_compact(const BatchList &a, const BatchList &b, const SolverState *st, int nsys,
                    hipStream_t s) {
-    hipLaunchKernelGGL(k_batch_compact, dim3(nsys), dim3(256), 0, s, items, item_start,
-                       item_count, st, nsys, items_act, nact);
+    hipLaunchKernelGGL(k_batch_compact, dim3(nsys, 2), dim3(256), 0, s, a, b, st, nsys);
 }
 
 void batch_all_done(const SolverState *st, int nsys, int *flag, hipStream_t s) {

@@ -449,8 +449,9 @@ struct BatchSolve {
     BatchDev d;
     BatchBarrier *bar = nullptr;
     unsigned long long wait_ticks = 0; // longest barrier wait, wall-clock ticks
-    const BatchItem *items = nullptr;
-    int nitems = 0, nsys = 0, max_iters = 0, pre = 0, order = 0;
+    const BatchItem *items = nullptr, *dot_items = nullptr;
+    int nitems = 0, ndot_items = 0, nsys = 0, max_iters = 0, pre = 0, order = 0;
+    // of the dot items per system
     const int *item_start = nullptr, *item_count = nullptr, *nvs = nullptr;
     double *partials = nullptr;
     double *x = nullptr, *r0 = nullptr, *r = nullptr, *p = nullptr, *v = nullptr, *s = nullptr;
@@ -465,9 +466,14 @@ hipError_t batch_solve_launch(const BatchSolve &P, int grid, hipStream_t s);
 void batch_launch(BatchOp op, const BatchDev &d, const BatchItem *items, int nitems, int grid,
                   const BatchVecs &v, int ci, int last, double *partials, hipStream_t s,
                   const int *nact = nullptr);
-// items_act / *nact = the items of the systems not done, in item order
-void batch_compact(const BatchItem *items, const int *item_start, const int *item_count,
-                   const SolverState *st, int nsys, BatchItem *items_act, int *nact,
+// one work list on the device: its items, first item and item count per system, and the
+// items of the systems not done (act, *nact of them)
+struct BatchList {
+    BatchItem *items = nullptr, *act = nullptr;
+    int *start = nullptr, *count = nullptr, *nact = nullptr;
+};
+// act / *nact of both lists = the items of the systems not done, in item order
+void batch_compact(const BatchList &a, const BatchList &b, const SolverState *st, int nsys,
                    hipStream_t s);
 void batch_finalize(FinOp op, SolverState *st, const double *partials, const int *item_start,
                     const int *item_count, const int *nvs, int nsys, hipStream_t s);

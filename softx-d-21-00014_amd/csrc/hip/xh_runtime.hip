@@ -2250,11 +2250,7 @@ struct xh_batch_s {
     uint32_t *row = nullptr, *col = nullptr;
     double *val = nullptr, *isd = nullptr, *cheb = nullptr;
     int64_t *d_rbase = nullptr, *d_voff = nullptr;
-    int *d_nv = nullptr, *d_item_start = nullptr, *d_item_count = nullptr, *d_flag = nullptr;
-    BatchItem *d_items = nullptr;
-    // the items of the systems not yet done (rebuilt after every iteration) and their count
-    BatchItem *d_items_act = nullptr;
-    int *d_nact = nullptr;
+    int *d_nv = nullptr, *d_flag = nullptr;
     SolverState *st = nullptr;
     double *partials = nullptr;
     double *x = nullptr, *b = nullptr, *r0 = nullptr, *r = nullptr, *p = nullptr, *v = nullptr;
@@ -2262,9 +2258,11 @@ struct xh_batch_s {
            *cu2 = nullptr;
     unsigned long long *d_t0 = nullptr;
     BatchBarrier *d_bar = nullptr; // grid barriers of the single-launch solve
-    // host
-    std::vector<BatchItem> items;
-    std::vector<int> item_start, item_count;
+    // Work lists: of the operations without dots, by the layout that xh_batch_autotune or the
+    // caller picks, and of the operations with dots, by kDotPasses and kDotRhsPerLane.  The
+    // active items are rebuilt after every iteration.
+    BatchList vec, dot;
+    int nvec = 0, ndot = 0;
     int tile_passes[5] = {8, 8, 8, 8, 8}; // per nv class 1, 2, 4, 8, 16
     int tile_w[5] = {1, 1, 1, 1, 1};      // RHS per lane per nv class (1 or 2)
     int grid = 2048;
@@ -2284,10 +2282,18 @@ namespace {
 
 int nv_class(int nv) { return nv == 1 ? 0 : nv == 2 ? 1 : nv == 4 ? 2 : nv == 8 ? 3 : 4; }
 
-// work items of the systems whose nv class is in `mask`, tile_passes[class] passes of
-// 256/nv rows each; item_start/count filled when all classes are included
-void build_items(xh_batch_s *B, unsigned mask, std::vector<BatchItem> &items,
-                 std::vector<int> *start, std::vector<int> *count) {
+// Layout of the operations with dots, per nv class 1, 2, 4, 8, 16.  An item's rows and their
+// split over lanes are the grouping of its dot partials, so this layout is a constant: the
+// same systems give the same bits whatever layout the other operations run with, and
+// whatever a tuning run measured.
+constexpr int kDotPasses[5] = {4, 4, 8, 4, 8};
+constexpr int kDotRhsPerLane[5] = {1, 2, 2, 2, 2};
+
+// work items of the systems whose nv class is in `mask`, passes[class] passes of
+// 256 * w[class] / nv rows each; start/count (nullable): of each system
+void build_items(const xh_batch_s *B, unsigned mask, const int *passes, const int *w,
+                 std::vector<BatchItem> &items, std::vector<int> *start,
+                 std::vector<int> *count) {
     items.clear();
     if (start) {
         start->assign(B->nsys, 0);
@@ -2297,8 +2303,8 @@ void build_items(xh_batch_s *B, unsigned mask, std::vector<BatchItem> &items,
         const int c = nv_class(B->nv[s]);
         if (!(mask & (1u << c)))
             continue;
-        const int wpl = B->nv[s] >= 2 ? B->tile_w[c] : 1;
-        const int64_t tile = (int64_t)B->tile_passes[c] * (kBlock * wpl / B->nv[s]);
+        const int wpl = B->nv[s] >= 2 ? w[c] : 1;
+        const int64_t tile = (int64_t)passes[c] * (kBlock * wpl / B->nv[s]);
         if (start)
             (*start)[s] = (int)items.size();
         for (int64_t r0 = 0; r0 < B->n[s]; r0 += tile)
@@ -2309,33 +2315,52 @@ void build_items(xh_batch_s *B, unsigned mask, std::vector<BatchItem> &items,
     }
 }
 
+void free_list(BatchList &l) {
+    for (void *q : {(void *)l.items, (void *)l.act, (void *)l.start, (void *)l.count,
+                    (void *)l.nact})
+        if (q)
+            (void)hipFree(q);
+    l = BatchList();
+}
+
+// builds a list of all systems with the given layout and uploads it; on failure `out` stays
+int upload_list(xh_batch_s *B, const int *passes, const int *w, BatchList &out, int &n) {
+    std::vector<BatchItem> items;
+    std::vector<int> start, count;
+    build_items(B, 0x1f, passes, w, items, &start, &count);
+    BatchList l;
+    auto up = [&]() -> int {
+        size_t acc = 0;
+        int rc;
+        if ((rc = dmalloc(&l.items, items.size(), acc)) ||
+            (rc = dmalloc(&l.act, items.size(), acc)) || (rc = dmalloc(&l.start, B->nsys, acc)) ||
+            (rc = dmalloc(&l.count, B->nsys, acc)) || (rc = dmalloc(&l.nact, 1, acc)))
+            return rc;
+        XH_HIP(hipMemcpy(l.items, items.data(), items.size() * sizeof(BatchItem),
+                         hipMemcpyHostToDevice));
+        XH_HIP(hipMemcpy(l.start, start.data(), B->nsys * sizeof(int), hipMemcpyHostToDevice));
+        XH_HIP(hipMemcpy(l.count, count.data(), B->nsys * sizeof(int), hipMemcpyHostToDevice));
+        return 0;
+    };
+    const int rc = up();
+    if (rc == 0) {
+        std::swap(l, out);
+        n = (int)items.size();
+    }
+    free_list(l);
+    return rc;
+}
+
+// the list of the operations without dots, after a change of its layout
 int upload_items(xh_batch_s *B) {
-    build_items(B, 0x1f, B->items, &B->item_start, &B->item_count);
-    (void)hipFree(B->d_items);
-    (void)hipFree(B->d_items_act);
-    (void)hipFree(B->partials);
-    B->d_items = nullptr;
-    B->d_items_act = nullptr;
-    B->partials = nullptr;
-    size_t acc = 0;
-    int rc;
-    if ((rc = dmalloc(&B->d_items, B->items.size(), acc)) ||
-        (rc = dmalloc(&B->d_items_act, B->items.size(), acc)) ||
-        (rc = dmalloc(&B->partials, B->items.size() * kBatchPart, acc)))
-        return rc;
-    XH_HIP(hipMemcpy(B->d_items, B->items.data(), B->items.size() * sizeof(BatchItem),
-                     hipMemcpyHostToDevice));
-    XH_HIP(hipMemcpy(B->d_item_start, B->item_start.data(), B->nsys * sizeof(int),
-                     hipMemcpyHostToDevice));
-    XH_HIP(hipMemcpy(B->d_item_count, B->item_count.data(), B->nsys * sizeof(int),
-                     hipMemcpyHostToDevice));
+    const int rc = upload_list(B, B->tile_passes, B->tile_w, B->vec, B->nvec);
     if (B->gexec) {
         (void)hipGraphExecDestroy(B->gexec);
         (void)hipGraphDestroy(B->graph);
         B->gexec = nullptr;
         B->graph = nullptr;
     }
-    return 0;
+    return rc;
 }
 
 BatchDev batch_dev(const xh_batch_s *B) {
@@ -2355,9 +2380,9 @@ BatchDev batch_dev(const xh_batch_s *B) {
 // the work list of the systems not yet done
 void batch_precond(xh_batch_s *B, const double *b, double *x) {
     const BatchDev d = batch_dev(B);
-    const int nit = (int)B->items.size();
-    const BatchItem *items = B->d_items_act;
-    const int *na = B->d_nact;
+    const int nit = B->nvec;
+    const BatchItem *items = B->vec.act;
+    const int *na = B->vec.nact;
     hipStream_t st = B->stream;
     if (B->prm.precond.method == XH_CHEBYSHEV) {
         const int k = B->prm.precond.poly_order;
@@ -2400,15 +2425,14 @@ void batch_precond(xh_batch_s *B, const double *b, double *x) {
 // iteration is rebuilt at the end
 void batch_iteration(xh_batch_s *B) {
     const BatchDev d = batch_dev(B);
-    const int nit = (int)B->items.size();
-    const BatchItem *items = B->d_items_act;
-    const int *na = B->d_nact;
+    const int nit = B->nvec, ndot = B->ndot;
+    const BatchItem *items = B->vec.act, *ditems = B->dot.act;
+    const int *na = B->vec.nact, *nad = B->dot.nact;
     hipStream_t st = B->stream;
     const bool pre = B->prm.solver.method != XH_BICGSTAB;
     double *pp = pre ? B->p_ : B->p, *ss = pre ? B->s_ : B->s;
     auto fin = [&](FinOp op) {
-        batch_finalize(op, B->st, B->partials, B->d_item_start, B->d_item_count, B->d_nv,
-                       B->nsys, st);
+        batch_finalize(op, B->st, B->partials, B->dot.start, B->dot.count, B->d_nv, B->nsys, st);
     };
     if (pre)
         batch_precond(B, B->p, B->p_);
@@ -2416,7 +2440,7 @@ void batch_iteration(xh_batch_s *B) {
     v1.in = pp;
     v1.o1 = B->r0;
     v1.out = B->v;
-    batch_launch(B_DOT1, d, items, nit, B->grid, v1, 0, 0, B->partials, st, na);
+    batch_launch(B_DOT1, d, ditems, ndot, B->grid, v1, 0, 0, B->partials, st, nad);
     fin(FIN_ALPHA);
     BatchVecs vs;
     vs.b = B->r;
@@ -2429,7 +2453,7 @@ void batch_iteration(xh_batch_s *B) {
     v3.in = ss;
     v3.o1 = B->s;
     v3.out = B->t;
-    batch_launch(B_DOT3, d, items, nit, B->grid, v3, 0, 0, B->partials, st, na);
+    batch_launch(B_DOT3, d, ditems, ndot, B->grid, v3, 0, 0, B->partials, st, nad);
     fin(FIN_OMEGA);
     BatchVecs vx;
     vx.x = B->x;
@@ -2439,7 +2463,7 @@ void batch_iteration(xh_batch_s *B) {
     vx.t = B->t;
     vx.o1 = B->r0;
     vx.out = B->r;
-    batch_launch(B_XR_UPDATE, d, items, nit, B->grid, vx, 0, 0, B->partials, st, na);
+    batch_launch(B_XR_UPDATE, d, ditems, ndot, B->grid, vx, 0, 0, B->partials, st, nad);
     fin(FIN_BETA);
     BatchVecs vp;
     vp.b = B->r;
@@ -2447,8 +2471,7 @@ void batch_iteration(xh_batch_s *B) {
     vp.out = B->p;
     batch_launch(B_P_UPDATE, d, items, nit, B->grid, vp, 0, 0, nullptr, st, na);
     batch_all_done(B->st, B->nsys, B->d_flag, st);
-    batch_compact(B->d_items, B->d_item_start, B->d_item_count, B->st, B->nsys,
-                  B->d_items_act, B->d_nact, st);
+    batch_compact(B->vec, B->dot, B->st, B->nsys, st);
 }
 
 void free_batch(xh_batch_s *B) {
@@ -2460,14 +2483,14 @@ void free_batch(xh_batch_s *B) {
         (void)hipGraphDestroy(B->graph);
     for (void *q : {(void *)B->row, (void *)B->col, (void *)B->val, (void *)B->isd,
                     (void *)B->cheb, (void *)B->d_rbase, (void *)B->d_voff, (void *)B->d_nv,
-                    (void *)B->d_item_start, (void *)B->d_item_count, (void *)B->d_flag,
-                    (void *)B->d_items, (void *)B->d_items_act, (void *)B->d_nact,
-                    (void *)B->st, (void *)B->partials, (void *)B->x,
+                    (void *)B->d_flag, (void *)B->st, (void *)B->partials, (void *)B->x,
                     (void *)B->b, (void *)B->r0, (void *)B->r, (void *)B->p, (void *)B->v,
                     (void *)B->s, (void *)B->t, (void *)B->p_, (void *)B->s_,
                     (void *)B->cu1, (void *)B->cu2, (void *)B->d_t0, (void *)B->d_bar})
         if (q)
             (void)hipFree(q);
+    free_list(B->vec);
+    free_list(B->dot);
     if (B->hst)
         (void)hipHostFree(B->hst);
     if (B->hflag)
@@ -2576,9 +2599,7 @@ extern "C" int xh_batch_create(int nsys, const int64_t *nrows, const int32_t *nv
         (rc = dmalloc(&B->val, std::max<int64_t>(1, nnz), acc)) || (rc = dmalloc(&B->isd, rows, acc)) ||
         (rc = dmalloc(&B->cheb, (size_t)nsys * kChebMax, acc)) ||
         (rc = dmalloc(&B->d_rbase, nsys, acc)) || (rc = dmalloc(&B->d_voff, nsys, acc)) ||
-        (rc = dmalloc(&B->d_nv, nsys, acc)) || (rc = dmalloc(&B->d_item_start, nsys, acc)) ||
-        (rc = dmalloc(&B->d_item_count, nsys, acc)) || (rc = dmalloc(&B->d_flag, 2, acc)) ||
-        (rc = dmalloc(&B->d_nact, 1, acc)) ||
+        (rc = dmalloc(&B->d_nv, nsys, acc)) || (rc = dmalloc(&B->d_flag, 2, acc)) ||
         (rc = dmalloc(&B->st, nsys, acc)) || (rc = dmalloc(&B->d_t0, 1, acc)) ||
         (rc = dmalloc(&B->d_bar, 1, acc)))
         return bail(rc);
@@ -2618,7 +2639,8 @@ extern "C" int xh_batch_create(int nsys, const int64_t *nrows, const int32_t *nv
     if (e != hipSuccess)
         return bail(fail(XH_EHIP, std::string("xh_batch_create: ") + hipGetErrorString(e)));
     B->wall_khz = khz;
-    if ((rc = upload_items(B)))
+    if ((rc = upload_list(B, kDotPasses, kDotRhsPerLane, B->dot, B->ndot)) ||
+        (rc = dmalloc(&B->partials, (size_t)B->ndot * kBatchPart, acc)) || (rc = upload_items(B)))
         return bail(rc);
     *out = B;
     return 0;
@@ -2661,14 +2683,16 @@ extern "C" int xh_batch_solve(xh_batch B) {
         // init and every iteration in one cooperative launch; no host round trip
         BatchSolve P;
         P.d = batch_dev(B);
-        P.items = B->d_items;
-        P.nitems = (int)B->items.size();
+        P.items = B->vec.items;
+        P.nitems = B->nvec;
+        P.dot_items = B->dot.items;
+        P.ndot_items = B->ndot;
         P.nsys = nsys;
         P.max_iters = std::max(1, B->prm.solver.max_iters);
         P.pre = B->prm.solver.method != XH_BICGSTAB;
         P.order = B->prm.precond.method == XH_CHEBYSHEV ? B->prm.precond.poly_order : 0;
-        P.item_start = B->d_item_start;
-        P.item_count = B->d_item_count;
+        P.item_start = B->dot.start;
+        P.item_count = B->dot.count;
         P.nvs = B->d_nv;
         P.partials = B->partials;
         P.x = B->x;
@@ -2687,7 +2711,7 @@ extern "C" int xh_batch_solve(xh_batch B) {
         if (cap < 1)
             return fail(XH_EHIP, "xh_batch_solve: no resident workgroup count for the "
                                  "single-launch solve");
-        const int grid = std::max(1, std::min(cap, std::max(P.nitems, nsys)));
+        const int grid = std::max(1, std::min(cap, std::max({P.nitems, P.ndot_items, nsys})));
         P.bar = B->d_bar;
         P.wait_ticks = (unsigned long long)(B->wall_khz * 2000.0); // 2 s per barrier
         XH_HIP(hipMemsetAsync(B->d_bar, 0, sizeof(BatchBarrier), st));
@@ -2707,11 +2731,9 @@ extern "C" int xh_batch_solve(xh_batch B) {
     v.out2 = B->p;
     v.out3 = B->r;
     const BatchDev d = batch_dev(B);
-    batch_launch(B_RESID0, d, B->d_items, (int)B->items.size(), B->grid, v, 0, 0, B->partials, st);
-    batch_finalize(FIN_INIT, B->st, B->partials, B->d_item_start, B->d_item_count, B->d_nv,
-                   nsys, st);
-    batch_compact(B->d_items, B->d_item_start, B->d_item_count, B->st, nsys, B->d_items_act,
-                  B->d_nact, st);
+    batch_launch(B_RESID0, d, B->dot.items, B->ndot, B->grid, v, 0, 0, B->partials, st);
+    batch_finalize(FIN_INIT, B->st, B->partials, B->dot.start, B->dot.count, B->d_nv, nsys, st);
+    batch_compact(B->vec, B->dot, B->st, nsys, st);
     int rc = check_launch();
     if (rc)
         return rc;
@@ -2787,7 +2809,11 @@ extern "C" int xh_batch_autotune(xh_batch B, int reps, int32_t *tile_passes) {
     XH_HIP(hipMemcpy(B->st, B->hst, sizeof(SolverState) * B->nsys, hipMemcpyHostToDevice));
     std::vector<BatchItem> items;
     BatchItem *d_items = nullptr;
-    double *d_part = nullptr;
+    // what the layout is used for most: the preconditioner's step, or without a polynomial
+    // the vector updates
+    const BatchOp op = B->prm.solver.method != XH_BICGSTAB && B->prm.precond.method == XH_CHEBYSHEV
+                           ? B_CHEB
+                           : B_S_UPDATE;
     int rc = 0;
     for (int c = 0; c < 5 && rc == 0; ++c) {
         bool present = false;
@@ -2801,24 +2827,21 @@ extern "C" int xh_batch_autotune(xh_batch B, int reps, int32_t *tile_passes) {
             const int p = cand[cw % 6], wl = 1 + cw / 6;
             B->tile_passes[c] = p;
             B->tile_w[c] = wl;
-            build_items(B, 1u << c, items, nullptr, nullptr);
+            build_items(B, 1u << c, B->tile_passes, B->tile_w, items, nullptr, nullptr);
             (void)hipFree(d_items);
-            (void)hipFree(d_part);
             size_t acc = 0;
-            if ((rc = dmalloc(&d_items, items.size(), acc)) ||
-                (rc = dmalloc(&d_part, items.size() * kBatchPart, acc)))
+            if ((rc = dmalloc(&d_items, items.size(), acc)))
                 break;
             XH_HIP(hipMemcpy(d_items, items.data(), items.size() * sizeof(BatchItem),
                              hipMemcpyHostToDevice));
             BatchVecs v;
-            v.in = B->b;
-            v.o1 = B->b;
+            v.in = v.b = v.o1 = B->b;
             v.out = B->t;
             const BatchDev d = batch_dev(B);
-            batch_launch(B_DOT1, d, d_items, (int)items.size(), B->grid, v, 0, 0, d_part, st);
+            batch_launch(op, d, d_items, (int)items.size(), B->grid, v, 0, 0, nullptr, st);
             XH_HIP(hipEventRecord(e0, st));
             for (int q = 0; q < reps; ++q)
-                batch_launch(B_DOT1, d, d_items, (int)items.size(), B->grid, v, 0, 0, d_part, st);
+                batch_launch(op, d, d_items, (int)items.size(), B->grid, v, 0, 0, nullptr, st);
             XH_HIP(hipEventRecord(e1, st));
             XH_HIP(hipEventSynchronize(e1));
             float ms = 0;
@@ -2833,7 +2856,6 @@ extern "C" int xh_batch_autotune(xh_batch B, int reps, int32_t *tile_passes) {
         B->tile_w[c] = best_w;
     }
     (void)hipFree(d_items);
-    (void)hipFree(d_part);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc)
@@ -2869,11 +2891,11 @@ extern "C" int xh_batch_spmv_timed(xh_batch B, int reps, double *us_per_launch,
     v.o1 = B->b;
     v.out = B->t;
     const BatchDev d = batch_dev(B);
-    const int nit = (int)B->items.size();
-    batch_launch(B_CHEB, d, B->d_items, nit, B->grid, v, 0, 0, nullptr, st);
+    const int nit = B->nvec;
+    batch_launch(B_CHEB, d, B->vec.items, nit, B->grid, v, 0, 0, nullptr, st);
     XH_HIP(hipEventRecord(e0, st));
     for (int q = 0; q < reps; ++q)
-        batch_launch(B_CHEB, d, B->d_items, nit, B->grid, v, 0, 0, nullptr, st);
+        batch_launch(B_CHEB, d, B->vec.items, nit, B->grid, v, 0, 0, nullptr, st);
     XH_HIP(hipEventRecord(e1, st));
     XH_HIP(hipEventSynchronize(e1));
     float ms = 0;

@@ -83,7 +83,7 @@ def test_batch_graph_eager_and_retiling(gpu):
     assert all(t in (1, 2, 4, 8, 16, 32) for t in tiles)
     B.solve()
     for s in range(len(sizes)):
-        # other tiles change only the order of the dot partial sums
+        # the tiles are those of the operations without dots
         assert abs(B.stats(s)["iters"] - its[s]) <= 1
         assert rel_diff(B.x(s), xs[1][s], nvs[s]) <= 1e-6
     B.set_tiles([1, 1, 1, 1, 1])
@@ -143,9 +143,8 @@ def test_batch_single_launch_is_identical(gpu, O, method, precond):
 @pytest.mark.parametrize("persistent", [False, True])
 def test_batch_two_rhs_per_lane_layout(gpu, O, persistent):
     # two RHS per lane (nv/2 lanes per row, twice the rows per pass) for every class with
-    # nv >= 2: each RHS's arithmetic is unchanged, only the dot partials group rows
-    # differently, so every system meets the oracle bar; graph and eager runs of one
-    # layout are identical
+    # nv >= 2: each RHS's arithmetic is unchanged, so every system meets the oracle bar;
+    # graph and eager runs of one layout are identical
     X = gpu
     sizes = (6, 9, 12, 7, 10, 5)
     nvs = (1, 2, 4, 8, 16, 4)
@@ -176,6 +175,37 @@ def test_batch_two_rhs_per_lane_layout(gpu, O, persistent):
         assert rel_diff(B.x(s), o["x"], nvs[s]) <= 1e-6
     with pytest.raises(X.XamgError):  # nv = 1 takes one RHS per lane only
         B.set_layout([1, 1, 1, 1, 1], [2, 2, 2, 2, 2])
+
+
+@pytest.mark.parametrize("method,precond", [("PBiCGStab", "Chebyshev"), ("BiCGStab", None)])
+def test_batch_bits_do_not_depend_on_the_layout(gpu, method, precond):
+    # the operations with dots walk a list fixed by each system's size and RHS count, so the
+    # iterates are the same bits in every layout, set or tuned (two tunings may pick two
+    # layouts).  Every system has several items of several passes in each layout, or is
+    # smaller than one item.
+    X = gpu
+    sizes, nvs = (17, 14, 13, 12, 11, 5), (1, 2, 4, 8, 16, 4)
+    sy = systems(X, sizes, seed=90, sigma=1.0 if precond else 0.0)
+    B, _ = run_batch(X, sy, nvs, params(X, method, precond))
+    ref = [(B.x(s), B.stats(s)["iters"]) for s in range(len(sizes))]
+
+    def same(what):
+        B.solve()
+        for s in range(len(sizes)):
+            assert B.stats(s)["iters"] == ref[s][1], (what, s)
+            assert np.array_equal(B.x(s), ref[s][0]), (what, s)
+
+    for passes, w in (([1] * 5, [1] * 5), ([32, 1, 3, 2, 5], [1, 2, 1, 2, 2]),
+                      ([2, 16, 1, 1, 1], [1, 2, 2, 2, 2])):
+        B.set_layout(passes, w)
+        same((passes, w))
+    B.set_tiles([3, 4, 5, 6, 7])
+    same("tiles")
+    for _ in range(2):
+        B.autotune(reps=2)
+        same(("tuned", B.layout()))
+    B.set_persistent(True)
+    same("single launch")
 
 
 def test_batch_rejects_unsupported(gpu):
