@@ -213,6 +213,7 @@ struct Tuning {
     int st7_min_seg = 32;           // shortest x segment of a work item
 };
 extern Tuning g_tune;
+extern unsigned g_tune_changes; // options set so far: a captured iteration is of one count
 
 // ---- launch accounting (xh_solver_profile) ----
 // While a profile solve runs, every launch helper of the solve path brackets its kernel

@@ -714,6 +714,7 @@ struct xh_solver_s {
     hipGraphExec_t gexec = nullptr, gexec_rep = nullptr; // plain / residual-replacing
     hipGraph_t graph = nullptr, graph_rep = nullptr;
     const double *g_x = nullptr, *g_b = nullptr; // pointers the graphs were captured with
+    unsigned g_changes = 0;                      // g_tune_changes at the capture
     const double *bcur = nullptr;                // b of the solve being enqueued
     size_t bytes = 0;
     int err = 0;
@@ -1205,8 +1206,10 @@ int solve_impl(xh_solver_s *S, const double *db, double *dx) {
     S->bcur = db;
     // an iteration reads x from the solver state and b not at all, so its graph serves every
     // solve (capturing it anew for another x cost ~0.3 ms); only a residual replacement
-    // (period > 0) holds both vectors
-    if (use_graph && (S->gexec == nullptr || (period > 0 && (S->g_x != dx || S->g_b != db)))) {
+    // (period > 0) holds both vectors.  An option set since chooses other kernels or launch
+    // shapes: captured anew
+    if (use_graph && (S->gexec == nullptr || S->g_changes != g_tune_changes ||
+                      (period > 0 && (S->g_x != dx || S->g_b != db)))) {
         free_graphs(S);
         XH_HIP(hipStreamBeginCapture(S->stream, hipStreamCaptureModeThreadLocal));
         enqueue_iteration(S, dx, false);
@@ -1220,6 +1223,7 @@ int solve_impl(xh_solver_s *S, const double *db, double *dx) {
         }
         S->g_x = dx;
         S->g_b = db;
+        S->g_changes = g_tune_changes;
     }
     const int maxit = std::max(1, S->prm.solver.max_iters) + 1;
     for (int it = 0; it < maxit; ++it) {
@@ -1987,9 +1991,9 @@ extern "C" int xh_set_option(const char *key, int64_t value) {
         unet::set_fuse_up((int)value);
     else if (k == "unet_conv_tile" && (value == 0 || value == 1))
         unet::set_conv_tile((int)value);
-
     else
         return fail(XH_EINVAL, "xh_set_option: unknown key or value out of range: " + k);
+    ++g_tune_changes;
     return 0;
 }
 

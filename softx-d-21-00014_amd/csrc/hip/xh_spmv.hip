@@ -25,6 +25,7 @@
 namespace xh {
 
 Tuning g_tune;
+unsigned g_tune_changes = 0;
 
 namespace {
 

@@ -301,6 +301,40 @@ def test_graph_serves_every_vector(gpu, method, period):
         assert np.array_equal(dx[1 - j].to_host(), other, equal_nan=True)
 
 
+@pytest.mark.parametrize("period", [0, 2])
+def test_captured_solve_follows_later_options(gpu, period):
+    # an option set after a solver captured its iteration counts from its next solve on: the
+    # partial counts of the dot products change the rounding, so the solution is bit for bit
+    # that of an eager solver under the same options, and again the first one afterwards
+    X = gpu
+    N, nv = 24, 8
+    levels = levels_for(X, N)
+    S, E = [X.Solver(X.Hier(levels), X.default_params(method="PBiCGStab", smoother="Chebyshev",
+                                                      poly_order=4, graph=graph,
+                                                      true_res_period=period), nv)
+            for graph in (1, 0)]
+    db = X.DeviceArray.from_host(X.rhs_uniform(6, N ** 3, nv))
+    dx = X.DeviceArray(N ** 3 * nv)
+
+    def solve(solver):
+        dx.zero()
+        solver.solve_device(db, dx)
+        return dx.to_host()
+
+    first = solve(S)
+    assert np.array_equal(first, solve(E))
+    try:
+        X.set_option("dot_groups", 16)
+        X.set_option("vec_dot_groups", 16)
+        eager = solve(E)
+        assert not np.array_equal(eager, first)
+        assert np.array_equal(solve(S), eager)
+    finally:
+        X.set_option("dot_groups", 1024)
+        X.set_option("vec_dot_groups", 2048)
+    assert np.array_equal(solve(S), first)
+
+
 def test_hsgs_block_drift_against_exact_gauss_seidel(gpu, O):
     # the GPU HSGS uses many core blocks (Jacobi coupling between them); against the
     # reference at one core (exact symmetric GS) the iteration count drifts by at most 1
