@@ -974,19 +974,30 @@ bool takes_codes(const Mat &A, SpmvOp op) {
            g_tune.grid_enable == 2 && A.nnz >= kGridMinRowNnz * A.nrows;
 }
 
-// Whether op on A runs as the LDS-window line sweep (k_spmv_sweep).  By default only the
-// Krylov SpMMs with dot partials of a large fp64 long-row operator with 32 right-hand
-// sides: 340 against 385 us at 96^3 (x of 226 MB); everywhere else the row-parallel kernel
-// is the faster one (y = A x at 64^3, nv = 32: 118 against 72 us; fp32 at 96^3: 194 against
-// 128; nv = 8 at 24^3: 67 against 6, the sweep's lines being too few to fill the chip).
+// Whether op on A runs as the LDS-window line sweep (k_spmv_sweep).  By default only the fp64
+// SpMMs with dot partials of a long-row operator, with 16 or 32 right-hand sides, and only
+// when the launch's work items (tile of lines x segment) fill at least 4/5 of the 2048
+// workgroups the chip holds: a workgroup stages its own window, so with fewer items the
+// chip idles and with a few more than 2048 half of it waits for second items.  27-point
+// operators, DOT1 + DOT3 in us, sweep / row-parallel (columns), by that share:
+// 32 right-hand sides 0.52 (92^3) 728 / 641, 0.57 (112^3) 1171 / 1123, 0.73 (151x190x122)
+// 2791 / 2774, 0.81 (86x101x125) 903 / 879, 0.84 (96^3) 692 / 714, 0.97 (164x87x72) 802 / 850,
+// 1.0 (128^3) 1504 / 1642; 16: 0.60 (152x110x87) 714 / 724, 0.81 (156x137x92) 960 / 973,
+// 0.86 (131x79x174) 845 / 886, 0.97 (184x163x74) 1027 / 1089, 1.0 (128^3) 908 / 1004.  With 8
+// the row-parallel kernel is the faster one or even at every share (0.92 and 0.99: 1183 /
+// 1099, 1235 / 1238), with 64 it is by 10 to 20 % (tiles of 8 rows, so more halo); y = A x at
+// 96^3 in fp32: 194 against 128.
 bool takes_sweep(const Mat &A, SpmvOp op, int nv) {
     if (A.idx == IDX_U8 || op == OP_OFFBLOCK || op == OP_PROLONG32 || op == OP_CHEBZ ||
         op == OP_CHEBR || A.gcode == nullptr || A.row_ind != nullptr || g_tune.grid_enable == 0)
         return false;
-    return g_tune.grid_enable == 1 ||
-           (A.prec == F64 && nv == 32 && A.nnz >= kGridMinRowNnz * A.nrows &&
-            (op == OP_DOT1 || op == OP_DOT3 || op == OP_RDOT4 || op == OP_RESID0) &&
-            A.nrows * nv * 8 >= ((int64_t)192 << 20));
+    if (g_tune.grid_enable == 1)
+        return true;
+    if (A.prec != F64 || (nv != 16 && nv != 32) || A.nnz < kGridMinRowNnz * A.nrows ||
+        !(op == OP_DOT1 || op == OP_DOT3 || op == OP_RDOT4 || op == OP_RESID0))
+        return false;
+    const GridLaunch G = grid_plan(A.gx, A.gy, A.gz, kBlock / (nv / 2), g_tune.grid_dot_groups);
+    return 5 * (int64_t)G.g.nitems >= 4 * (int64_t)G.g.ipw * 2048;
 }
 
 namespace {

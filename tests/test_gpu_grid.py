@@ -99,6 +99,42 @@ def test_grid_path_by_row_length(gpu):
         assert any(k.startswith("k_spmv_grid<") for k in names) == want, (name, names)
 
 
+@pytest.mark.parametrize("dims,nv,want", [
+    ((64, 40, 44), 32, True),    # 110 tiles of 16 lines x 16 segments: 1760 of 2048
+    ((64, 40, 36), 32, False),   # 1440 work items
+    ((64, 60, 36), 32, False),   # 2160: two for some workgroups
+    ((64, 60, 60), 16, True),    # 120 tiles of 32 lines x 16
+    ((64, 40, 44), 16, False),
+    ((64, 40, 44), 8, False),
+    ((64, 40, 44), 64, False),
+])
+def test_sweep_by_filled_workgroups(gpu, dims, nv, want):
+    # in the default mode the SpMMs with dots run the line sweep where its work items fill the
+    # chip (here with segments of 4 rows, so that small grids can); the solution does not
+    # depend on it beyond the order of the dot partials
+    X = gpu
+    row, col, val = X.q1fem27(*dims)[:3]
+    n = len(row) - 1
+    H = X.Hier(X.Amg(row, col, val, max_levels=1).export())
+    S = X.Solver(H, X.default_params(method="PBiCGStab", precond="Chebyshev", poly_order=8,
+                                     max_iters=400, rel_tol=1e-10), nv)
+    b = X.rhs_uniform(5, n, nv)
+    db, dx = X.DeviceArray.from_host(b), X.DeviceArray(n * nv)
+    try:
+        X.set_option("spmv_grid_min_seg", 4)
+        dx.zero()
+        names = {k["kernel"] for k in S.profile(db, dx, 2)}
+        x = S.solve(b)
+        X.set_option("spmv_grid_enable", 0)
+        x0 = S.solve(b)
+    finally:
+        X.set_option("spmv_grid_enable", 2)
+        X.set_option("spmv_grid_min_seg", 32)
+    for op in ("OP_DOT1", "OP_DOT3", "OP_RESID0"):
+        assert (f"k_spmv_sweep<double,{nv},{op}>" in names) == want, names
+    assert (np.abs(x - x0).reshape(n, nv).max(0) / np.abs(x0).reshape(n, nv).max(0)).max() <= 1e-6
+
+
 def test_no_grid_view_for_partial_grids(gpu):
     X = gpu
     row, col, val = X.cube(8, 6, 5)
