@@ -191,6 +191,8 @@ struct Tuning {
     // the rules at takes_codes and takes_sweep
     int grid_enable = 2;
     int grid_dot_groups = 2048;     // work items of a grid-path launch that writes partials
+    // neighbour codes for more than 4 RHS: launches of at least this many bytes (takes_codes)
+    int64_t codes_min_bytes = 200 * 1000 * 1000;
     // 1: a Chebyshev smoother from a zero x runs its first two steps as one SpMV
     // (OP_CHEBZ) where OP_CHEB would run row-parallel
     int chebz_enable = 1;

@@ -1977,6 +1977,8 @@ extern "C" int xh_set_option(const char *key, int64_t value) {
         g_tune.wave_enable = (int)value;
     else if (k == "spmv_grid_enable" && value >= 0 && value <= 2)
         g_tune.grid_enable = (int)value;
+    else if (k == "spmv_codes_min_bytes" && value >= 0)
+        g_tune.codes_min_bytes = value;
     else if (k == "spmv_st7_enable" && (value == 0 || value == 1))
         g_tune.st7_enable = (int)value;
     else if (k == "spmv_st7_waves" && value >= 8 && value <= (1 << 20))

@@ -966,12 +966,30 @@ bool spmv_wide_batches(const Mat &A, int rpb) {
 
 // Whether the row-parallel kernel reads the grid codes of A (1 byte per entry) instead of
 // its columns (2 or 4): matrices with a grid view whose rows are long enough for the index
-// bytes to show.  27-point operator at 96^3, y = A x, us (columns / codes): fp64 nv = 4
-// 106 / 76, 8 123 / 99, 32 312 / 296; fp32 nv = 4 119 / 80, 32 149 / 128; equal at 48^3 and
-// below, where the matrix stays in cache.
-bool takes_codes(const Mat &A, SpmvOp op) {
-    return op != OP_OFFBLOCK && op != OP_PROLONG32 && A.gcode != nullptr && A.row_ind == nullptr &&
-           g_tune.grid_enable == 2 && A.nnz >= kGridMinRowNnz * A.nrows;
+// bytes to show, where the fewer bytes pay for decoding them.  27-point operators, us
+// (columns / codes):
+// - up to 4 right-hand sides the matrix is most of the traffic: y = A x in fp64, nv = 1 48^3
+//   22 / 14, 96^3 175 / 122, nv = 4 48^3 14.8 / 13.0, 96^3 90 / 75; fp32 nv = 4 48^3 18 / 14, 96^3
+//   117 / 78.  In fp32 with 1 or 2 (one lane per row) the decoding shows: 96^3 128 / 158;
+// - launches with dots, in fp64: nv = 8 72^3 126 / 118, 96^3 338 / 307 (DOT1 + DOT3), but nv = 16
+//   96^3 460 / 480, 128^3 1004 / 1048, nv = 32 64^3 228 / 234, 112^3 1123 / 1157, nv = 64 96^3
+//   1463 / 1532;
+// - others, once matrix, x and y together leave the 256 MB last-level cache: fp64 nv = 8 64^3
+//   (100 MB) 30.4 / 31.2, 96^3 (350 MB) 121 / 98, nv = 16 48^3 22.6 / 23.7, 96^3 181 / 168, nv = 32
+//   48^3 33.9 / 35.9, 80^3 158 / 142, 96^3 305 / 296; fp32 nv = 16 64^3 26.1 / 26.6, 112^3 170 / 132,
+//   nv = 32 64^3 42 / 45, 96^3 132 / 127.  fp32 nv = 8 is slower or mixed at every size: 64^3 25.6 /
+//   30.2, 96^3 74.9 / 79.5, 128^3 224 / 212, 144^3 342 / 378.
+bool takes_codes(const Mat &A, SpmvOp op, int nv) {
+    if (op == OP_OFFBLOCK || op == OP_PROLONG32 || A.gcode == nullptr || A.row_ind != nullptr ||
+        g_tune.grid_enable != 2 || A.nnz < kGridMinRowNnz * A.nrows)
+        return false;
+    if (nv <= 4)
+        return A.prec == F64 || nv == 4;
+    if (op == OP_DOT1 || op == OP_DOT3 || op == OP_RDOT4 || op == OP_RESID0)
+        return nv == 8;
+    const int64_t sv = A.prec == F64 ? 8 : 4, si = A.idx == IDX_U16 ? 2 : 4;
+    return (A.prec == F64 || nv != 8) &&
+           A.nnz * (sv + si) + 2 * A.nrows * nv * sv >= g_tune.codes_min_bytes;
 }
 
 // Whether op on A runs as the LDS-window line sweep (k_spmv_sweep).  By default only the fp64
@@ -1054,7 +1072,7 @@ int launch_t(const Mat &A, const void *x, void *y, const SpmvArgs &a, hipStream_
         }
     }
     if constexpr (sizeof(IT) != 1 && OP != OP_OFFBLOCK && OP != OP_PROLONG32) {
-        if (takes_codes(A, (SpmvOp)OP)) {
+        if (takes_codes(A, (SpmvOp)OP, NV)) {
             hipLaunchKernelGGL((k_spmv<VT, GridCol, NV, OP>), dim3(L.grid), dim3(kBlock), 0, s,
                                A.row, (const GridCol *)A.gcode, (const VT *)A.val,
                                (const uint32_t *)nullptr, A.gx, L.sc, (const VT *)x, y,
@@ -1275,7 +1293,7 @@ int spmv(const Mat &A, int nv, const void *x, void *y, SpmvOp op, const SpmvArgs
         const bool st7 = takes_st7(A, op, nv);
         const bool sweep = !st7 && takes_sweep(A, op, nv);
         const bool wave = !st7 && !sweep && takes_wave(A, op, nv);
-        const bool grid = !st7 && !sweep && !wave && takes_codes(A, op);
+        const bool grid = !st7 && !sweep && !wave && takes_codes(A, op, nv);
         const bool wide = !st7 && !sweep && !grid && !wave && (nv == 8 || nv == 32) && A.idx != IDX_U8 &&
                           (op == OP_SET || op == OP_ADD || op == OP_RESID || op == OP_CHEB0 ||
                            op == OP_CHEB || op == OP_CHEBZ || op == OP_CHEBR) &&

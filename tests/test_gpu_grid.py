@@ -62,6 +62,7 @@ def test_grid_codes_bit_identical(gpu, prec, dims):
     levels = X.Amg(row, col, val, coarse_size=40).export()
     prm = X.default_params(smoother="Chebyshev", poly_order=4, mg_prec=2 * prec)
     try:
+        X.set_option("spmv_codes_min_bytes", 0)  # at this size for every RHS count
         for nv in (1, 2, 4, 8, 16, 32, 64):
             x = X.DeviceArray.from_host(np.random.default_rng(nv).standard_normal(n * nv).astype(dt))
             S = X.Solver(X.Hier(levels), prm, nv)
@@ -79,6 +80,37 @@ def test_grid_codes_bit_identical(gpu, prec, dims):
                 assert np.array_equal(a, b), nv
     finally:
         X.set_option("spmv_grid_enable", 2)
+        X.set_option("spmv_codes_min_bytes", 200000000)
+
+
+@pytest.mark.parametrize("mg_prec,nv,reached,want", [
+    (0, 1, False, True), (0, 4, False, True), (0, 8, False, False), (0, 8, True, True),
+    (0, 64, False, False), (0, 64, True, True), (2, 2, True, False), (2, 4, False, True),
+    (2, 8, True, False), (2, 16, False, False), (2, 16, True, True)])
+def test_codes_by_rhs_and_bytes(gpu, mg_prec, nv, reached, want):
+    # which launches of a 27-point operator read neighbour codes: a smoother's residual by
+    # precision, RHS count and the bytes of matrix, x and y on both sides of the line; a
+    # launch with dots (fp64) up to 8 RHS
+    X = gpu
+    row, col, val = X.q1fem27(20, 20, 20)[:3]
+    n, prec = len(row) - 1, int(mg_prec == 2)
+    sv, si = (4 if prec else 8), X.Matrix(row, col, val, prec=prec).info()["index_bits"] // 8
+    nbytes = len(col) * (sv + si) + 2 * n * nv * sv
+    levels = X.Amg(row, col, val, coarse_size=300).export()
+    prm = X.default_params(method="MergedPBiCGStab", smoother="Jacobi", sweeps=2, mg_prec=mg_prec)
+    S = X.Solver(X.Hier(levels), prm, nv)
+    db, dx = X.DeviceArray.from_host(X.rhs_uniform(1, n, nv)), X.DeviceArray(n * nv)
+    dx.zero()
+    try:
+        X.set_option("spmv_codes_min_bytes", nbytes + (0 if reached else 1))
+        X.set_option("spmv_wave_enable", 0)
+        names = {(k["kernel"], k["level"]) for k in S.profile(db, dx, 1)}
+    finally:
+        X.set_option("spmv_codes_min_bytes", 200000000)
+        X.set_option("spmv_wave_enable", 2)
+    t = "float" if prec else "double"
+    assert ((f"k_spmv_grid<{t},{nv},OP_RESID>", 0) in names) == want, names
+    assert any(k == f"k_spmv_grid<double,{nv},OP_DOT1>" for k, _ in names) == (nv <= 8), names
 
 
 def test_grid_path_by_row_length(gpu):
