@@ -308,6 +308,8 @@ struct SpmvArgs {
     int grid_cap = 0;           // 0: default
 };
 
+// whether the row-parallel kernel reads the neighbour codes of A for op
+bool takes_codes(const Mat &A, SpmvOp op, int nv);
 // the kernel for few, long rows (xh_spmv_wave.hip) and whether op on A takes it
 bool takes_wave(const Mat &A, SpmvOp op, int nv);
 int wave_entries(const Mat &A, int nv); // entries of a row it loads side by side

@@ -227,9 +227,14 @@ void by_nv(const Mat &A, int nv, const void *x, void *y, SpmvOp op, const SpmvAr
 // 24 entries 27366 rows 7.5 / 9.8; L = 4 (nv = 8): 5663 rows 9.3 / 6.6, 17391 rows 7.3 / 12.0;
 // L = 8 (nv = 16): 1259 rows 10.7 / 5.6, 4375 rows 9.5 / 9.6; L = 16 (nv = 32): 440 rows
 // 14.2 / 10.8, 1596 rows 11.8 / 11.7, 4375 rows 8.8 / 15.5.  Short rows (restrictions, 6 to
-// 11 entries) leave less to gain: half the waves.  One right-hand side wins at every size
-// with long rows (262144 rows of 26: 52.9 / 27.8), as the row-parallel kernel then has each
-// lane load its own entries.  Below 4 entries a row is one batch there.
+// 11 entries) leave less to gain: half the waves.  Below 4 entries a row is one batch there.
+// One right-hand side, and two in fp32, win at every size with long rows (262144 rows of 26:
+// fp64 nv = 1 52.9 / 24.8, fp32 nv = 2 41.1 / 21.8; 163868 rows of 14: 15.0 / 13.0, 12.6 /
+// 11.7), as the row-parallel kernel then has each lane load its own entries.  Two in fp64
+// win past the cap from 18 entries per row (442368 rows of 18.6: 55.6 / 50.7, 110592 of 26:
+// 22.2 / 17.9; but 119404 of 16: 13.9 / 16.7, 955225 of 16: 91.3 / 106.4), and against the
+// neighbour codes from 2^17 rows (135000 of 26: 22.8 / 21.1, 262144: 47.8 / 36.2; but 64000: 9.4
+// / 12.1, 110592: 14.4 / 18.0).
 bool takes_wave(const Mat &A, SpmvOp op, int nv) {
     if (!(op == OP_SET || op == OP_ADD || op == OP_RESID || op == OP_CHEB0 || op == OP_CHEB ||
           op == OP_CHEBZ || op == OP_CHEBR) ||
@@ -240,7 +245,9 @@ bool takes_wave(const Mat &A, SpmvOp op, int nv) {
     if (g_tune.wide_batches == 0 || A.nnz < 4 * A.nrows)
         return false;
     const bool longrows = A.nnz >= 12 * A.nrows;
-    if (nv <= 2 && longrows)
+    if (longrows && (nv == 1 || (nv == 2 && (A.prec == F32 ||
+                                             (A.nnz >= 18 * A.nrows &&
+                                              (!takes_codes(A, op, nv) || A.nrows >= 1 << 17))))))
         return true;
     const int L = nv / std::min(nv, A.prec == F64 ? 2 : 4);
     if (A.gcode != nullptr && L > 1)

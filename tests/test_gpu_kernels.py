@@ -226,6 +226,25 @@ def test_spmv_many_long_rows_few_rhs_bit_exact(gpu, O, nv, prec):
     assert np.array_equal(dy.to_host(), O.spmv(row, col, val, x, nv, f32=prec == 1))
 
 
+@pytest.mark.parametrize("nv,mg_prec,dims,want", [
+    (1, 0, (40, 40, 40), True), (2, 0, (40, 40, 40), False), (2, 0, (52, 51, 51), True),
+    (2, 2, (40, 40, 40), True), (2, 0, (30, 30, 30), True), (4, 0, (30, 30, 30), False)])
+def test_long_row_kernel_by_size_on_codes(gpu, nv, mg_prec, dims, want):
+    # 27-point operators in the default mode: fp64 with two RHS reads codes between the cap of
+    # 32768 rows and 2^17 rows; one RHS, and two in fp32, take the long-row kernel there
+    X = gpu
+    row, col, val = X.q1fem27(*dims)[:3]
+    n = len(row) - 1
+    levels = X.Amg(row, col, val, agg_num_levels=1, coarse_size=500).export()
+    prm = X.default_params(method="MergedPBiCGStab", smoother="Jacobi", sweeps=2, mg_prec=mg_prec)
+    S = X.Solver(X.Hier(levels), prm, nv)
+    db, dx = X.DeviceArray.from_host(X.rhs_uniform(1, n, nv)), X.DeviceArray(n * nv)
+    dx.zero()
+    names = {k["kernel"] for k in S.profile(db, dx, 1) if k["level"] == 0}
+    took = [k for k in names if k.startswith("k_spmv_wave<") and "OP_RESID" in k]
+    assert bool(took) == want, names
+
+
 @pytest.mark.parametrize("smoother,nv,mg_prec", [("Chebyshev", 1, 0), ("Chebyshev", 8, 2),
                                                  ("Chebyshev", 32, 1), ("Jacobi", 4, 0),
                                                  ("HSGS", 2, 2), ("Chebyshev", 64, 0)])
