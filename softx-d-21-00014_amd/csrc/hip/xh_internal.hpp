@@ -312,7 +312,7 @@ struct SpmvArgs {
 bool takes_codes(const Mat &A, SpmvOp op, int nv);
 // the kernel for few, long rows (xh_spmv_wave.hip) and whether op on A takes it
 bool takes_wave(const Mat &A, SpmvOp op, int nv);
-int wave_entries(const Mat &A, int nv); // entries of a row it loads side by side
+int wave_entries(const Mat &A, int nv); // its EPX
 void spmv_wave(const Mat &A, int nv, const void *x, void *y, SpmvOp op, const SpmvArgs &a,
                hipStream_t s);
 // returns the number of partial blocks written (DOT ops) or 0

@@ -1302,11 +1302,10 @@ int spmv(const Mat &A, int nv, const void *x, void *y, SpmvOp op, const SpmvArgs
                                  (wide   ? std::string(",16>")
                                   : wave ? "," + std::to_string(wave_entries(A, nv)) + ">"
                                          : std::string(">"));
-        led.kernel = st7    ? std::string("k_spmv_st7<") + prec_name(A.prec) + "," + tail
+        led.kernel = st7     ? std::string("k_spmv_st7<") + prec_name(A.prec) + "," + tail
                      : sweep ? std::string("k_spmv_sweep<") + prec_name(A.prec) + "," + tail
-                     : grid ? std::string("k_spmv_grid<") + prec_name(A.prec) + "," + tail
-                            : std::string(wave ? "k_spmv_wave<" : "k_spmv<") + prec_name(A.prec) + "," +
-                                  idx_name(A.idx) + "," + tail;
+                             : std::string(wave ? "k_spmv_wave<" : "k_spmv<") + prec_name(A.prec) +
+                                   "," + (grid ? "grid" : idx_name(A.idx)) + "," + tail;
         led.bytes = spmv_bytes(A, nv, op, a, grid || sweep, st7) +
                     (np > 0 ? (double)np * op_ndots(op) * nv * 8.0 : 0.0);
     }

@@ -262,7 +262,7 @@ int wave_entries(const Mat &A, int nv) {
     const int L = nv / std::min(nv, A.prec == F64 ? 2 : 4);
     if (L == 1 && A.nrows > 65536)
         return 4;
-    return L >= 4 ? 64 / L : 16;
+    return 16;
 }
 
 void spmv_wave(const Mat &A, int nv, const void *x, void *y, SpmvOp op, const SpmvArgs &a,

@@ -25,16 +25,19 @@ VEC = ["V_S_UPDATE", "V_XR_UPDATE", "V_P_UPDATE", "V_GROUP1", "V_X_UPDATE", "V_R
 
 def short(name):
     """kernel template instance with the op enums named, without namespace and arguments"""
+    name = name.replace("(anonymous namespace)::", "")
     m = re.search(r"(k_\w+)<([^()]*)>", name)
     if not m:
         return name.split("(")[0]
+    types = {"unsigned short": "u16", "unsigned int": "u32", "unsigned char": "u8",
+             "xh::GridCol": "grid"}
     k, args = m.group(1), [a.strip() for a in m.group(2).split(",")]
-    args = ["u16" if a == "unsigned short" else "u32" if a == "unsigned int" else a
-            for a in args]
-    if k == "k_spmv" and len(args) == 5 and args[3].isdigit():
+    args = [types.get(a, a) for a in args]
+    if k in ("k_spmv", "k_spmv_wave") and len(args) == 5 and args[3].isdigit():
         # k_spmv<VT, IT, NV, OP, BX>: the x loads per batch shown only when not 8, as the
         # solver's launch accounting names the kernel
-        args = args[:3] + [OPS["k_spmv"][int(args[3])]] + ([args[4]] if args[4] != "8" else [])
+        plain = k == "k_spmv" and args[4] == "8"
+        args = args[:3] + [OPS["k_spmv"][int(args[3])]] + ([] if plain else [args[4]])
     elif k.startswith("k_spmv") and args[-1].isdigit():
         args[-1] = OPS["k_spmv"][int(args[-1])]
     if k == "k_vec" and args[-1].isdigit():

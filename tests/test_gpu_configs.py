@@ -57,7 +57,7 @@ def test_q1fem27_hsgs_preconditioner_bit_exact(codes_everywhere, O, mg_prec, nv)
     dx.zero()
     names = {k["kernel"] for k in S.profile(db, dx, 1)}
     prec = "double" if mg_prec == 0 else "float"
-    assert (f"k_spmv_grid<{prec},{nv},OP_RESID>" in names) == ((mg_prec, nv) != (2, 8)), names
+    assert (f"k_spmv<{prec},grid,{nv},OP_RESID>" in names) == ((mg_prec, nv) != (2, 8)), names
 
 
 def test_varcoef7_chebyshev8_without_amg(gpu, O):

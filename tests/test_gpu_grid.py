@@ -109,13 +109,14 @@ def test_codes_by_rhs_and_bytes(gpu, mg_prec, nv, reached, want):
         X.set_option("spmv_codes_min_bytes", 200000000)
         X.set_option("spmv_wave_enable", 2)
     t = "float" if prec else "double"
-    assert ((f"k_spmv_grid<{t},{nv},OP_RESID>", 0) in names) == want, names
-    assert any(k == f"k_spmv_grid<double,{nv},OP_DOT1>" for k, _ in names) == (nv <= 8), names
+    assert ((f"k_spmv<{t},grid,{nv},OP_RESID>", 0) in names) == want, names
+    assert any(k == f"k_spmv<double,grid,{nv},OP_DOT1>" for k, _ in names) == (nv <= 8), names
 
 
 def test_grid_path_by_row_length(gpu):
-    # the default takes the grid path for the 27-point operator (27 entries per interior
-    # row) and the row-parallel kernel for the 7-point cube: the launches of a solve show it
+    # the default reads neighbour codes for the 27-point operator (27 entries per interior
+    # row; at this size its launches with dots) and columns for the 7-point cube: the
+    # launches of a solve show it, none of them a line sweep
     X = gpu
     X.set_option("spmv_grid_enable", 2)
     nv = 8
@@ -128,7 +129,8 @@ def test_grid_path_by_row_length(gpu):
         db = X.DeviceArray.from_host(X.rhs_uniform(3, n, nv))
         dx = X.DeviceArray(n * nv)
         names = {k["kernel"] for k in S.profile(db, dx, 1)}
-        assert any(k.startswith("k_spmv_grid<") for k in names) == want, (name, names)
+        assert any(k.startswith("k_spmv<double,grid,") for k in names) == want, (name, names)
+        assert not any(k.startswith("k_spmv_sweep<") for k in names), (name, names)
 
 
 @pytest.mark.parametrize("dims,nv,want", [
