@@ -330,17 +330,13 @@ const char *hsgs_t(const Mat &A, const void *t, void *x, int x_zero, double rela
     const int grid = (int)((nblk + G - 1) / G);
     const size_t lds = (size_t)64 * B * sizeof(VT);
     if constexpr (sizeof(IT) == 4) {
-        // a padded core-block matrix of this block size whose blocks fit in LDS: staged
-        // sweeps.  Per group: x with its zero row, values and inverse diagonal (VT), then
-        // columns and row pointers (u32)
-        const size_t gb = ((size_t)(B + 1) * NV * sizeof(VT) +
-                           (size_t)A.core_emax * (sizeof(VT) + 4) + (size_t)B * sizeof(VT) +
-                           (size_t)(B + 1) * 4 + 15) / 16 * 16;
-        if (A.core_B == B && gb <= 64 * 1024) {
+        // a padded core-block matrix of this block size whose blocks fit in LDS: staged sweeps
+        const size_t gb = hsgs_core_bytes(B, NV, A.core_emax, sizeof(VT));
+        if (A.core_B == B && gb <= kHsgsLds) {
             // blocks per wave: as many as the wave's lanes and 64 KB of LDS hold, but fewer
             // while there are not 2048 waves (2 per SIMD): a wave's time is its row chain,
             // the same for one block as for several
-            const int64_t fit = std::min<int64_t>(G, 64 * 1024 / (int64_t)gb);
+            const int64_t fit = std::min<int64_t>(G, kHsgsLds / gb);
             const int gw = (int)std::max<int64_t>(1, std::min<int64_t>(fit, nblk / 2048));
             switch (A.core_kb) {
             case 3:

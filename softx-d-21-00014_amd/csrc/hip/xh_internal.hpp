@@ -497,6 +497,14 @@ void jacobi_update(int64_t n, int nv, int prec, void *x, const void *b, const vo
 void hsgs_sweeps(const Mat &A, int nv, const void *t, void *x, int x_zero, double relax,
                  int64_t blk_rows, const int *done, hipStream_t s);
 int64_t hsgs_block_rows(int64_t n, int nblocks);
+// LDS of one core block in k_hsgs_core: x with its zero row, values and inverse diagonal (sv
+// bytes each), columns and row pointers (u32); emax: entries of the largest block.  The
+// kernel runs where that is at most kHsgsLds.
+constexpr size_t kHsgsLds = 64 * 1024;
+inline size_t hsgs_core_bytes(int64_t B, int nv, int64_t emax, int sv) {
+    return ((size_t)(B + 1) * nv * sv + (size_t)emax * (sv + 4) + (size_t)B * sv +
+            (size_t)(B + 1) * 4 + 15) / 16 * 16;
+}
 // y = D x; prec: precision of D and of the sums, xprec: of x and y (F64, or prec)
 void dense_matvec(int64_t n, int nv, int prec, int xprec, const void *D, const void *x, void *y,
                   const int *done, hipStream_t s);

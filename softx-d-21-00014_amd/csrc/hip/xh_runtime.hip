@@ -461,7 +461,7 @@ HostCsr off_block_csr(const HostCsr &h, int64_t B) {
     return o;
 }
 
-int upload_core(const HostCsr &h, int64_t B, int prec, const Mat &A, Mat &M) {
+int upload_core(const HostCsr &h, int64_t B, int nv, int prec, const Mat &A, Mat &M) {
     M = Mat();
     const int64_t n = h.nrows;
     std::vector<int64_t> cnt(n, 0);
@@ -474,14 +474,23 @@ int upload_core(const HostCsr &h, int64_t B, int prec, const Mat &A, Mat &M) {
     }
     auto padded = [](int64_t c, int kb) { return std::max<int64_t>(kb, (c + kb - 1) / kb * kb); };
     // KB: the width whose rows take the least time in the sweep's serial chain, a batch
-    // costing one LDS round trip (about as long as 12 subtractions) and its KB subtractions
+    // costing one LDS round trip (about as long as 12 subtractions) and its KB subtractions,
+    // among the widths whose pads leave the largest block in LDS (with 64 RHS the pads of 6
+    // or 8 can be what does not fit; 20^3 27-point, blocks of 104 rows, fp64, us for two sweeps:
+    // 370 by the kernel without staging, 69 with batches of 3)
     int KB = 3;
     int64_t best = -1;
     for (int kb : {3, 4, 6, 8}) {
-        int64_t cost = 0;
-        for (int64_t i = 0; i < n; ++i)
-            cost += padded(cnt[i], kb) / kb * (12 + kb);
-        if (best < 0 || cost < best) {
+        int64_t cost = 0, emax = 0;
+        for (int64_t lo = 0; lo < n; lo += B) {
+            int64_t e = 0;
+            for (int64_t i = lo; i < std::min(n, lo + B); ++i)
+                e += padded(cnt[i], kb);
+            cost += e / kb * (12 + kb);
+            emax = std::max(emax, e);
+        }
+        const bool fits = hsgs_core_bytes(B, nv, emax, prec == F64 ? 8 : 4) <= kHsgsLds;
+        if (fits && (best < 0 || cost < best)) {
             best = cost;
             KB = kb;
         }
@@ -1632,7 +1641,7 @@ int xh_solver_create(xh_hier H, const xh_params *prm, int nv, xh_solver *out) {
                 return bail(fail(XH_EINVAL, "Chebyshev order out of range"));
         if (roles[0]->method == XH_HSGS || roles[1]->method == XH_HSGS ||
             roles[2]->method == XH_HSGS) {
-            if ((rc = upload_core(H->A[l], L.hsgs_B, L.prec, L.A, L.core)))
+            if ((rc = upload_core(H->A[l], L.hsgs_B, nv, L.prec, L.A, L.core)))
                 return bail(rc);
             S->bytes += L.core.bytes;
             if (g_tune.hsgs_off_csr) {

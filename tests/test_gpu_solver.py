@@ -261,6 +261,26 @@ def test_hsgs_blocks_per_wave_bit_exact(gpu, O, N, nv, mg_prec, block_rows):
     assert f"k_hsgs_core<{'double' if mg_prec == 0 else 'float'},{nv}>" in names, names
 
 
+@pytest.mark.parametrize("block_rows,mg_prec", [(104, 0), (192, 2)])
+def test_hsgs_batch_width_leaves_the_block_in_lds(gpu, O, block_rows, mg_prec):
+    # 64 RHS, blocks of 27-point rows near the LDS limit: batches of 6 entries would cost a row
+    # less, but only those of 3 leave the block in LDS, and so the staged sweep
+    X = gpu
+    nv, (row, col, val) = 64, X.q1fem27(20, 20, 20)[:3]
+    levels = X.Amg(row, col, val, agg_num_levels=1, num_paths=2, coarse_size=100).export()
+    prm = X.default_params(method="MergedPBiCGStab", smoother="HSGS", sweeps=1, mg_prec=mg_prec)
+    prm.hsgs_block_rows = block_rows
+    S = X.Solver(X.Hier(levels), prm, nv)
+    n = len(row) - 1
+    b = X.rhs_uniform(12, n, nv)
+    db, dx = X.DeviceArray.from_host(b), X.DeviceArray(n * nv)
+    S.precond_apply(db, dx)
+    assert np.array_equal(dx.to_host(), O.mg_apply(O.Hier(levels), O.params_from(prm), nv, b))
+    dx.zero()
+    names = {k["kernel"] for k in S.profile(db, dx, 1) if k["level"] == 0}
+    assert any(k.startswith("k_hsgs_core<") for k in names), names
+
+
 def test_graph_and_eager_are_identical(gpu):
     X = gpu
     N, nv = 24, 8
