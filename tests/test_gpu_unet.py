@@ -192,7 +192,7 @@ def test_tiled_convolution_is_identical(gpu):
 
 
 def test_narrow_tiles_are_identical(gpu):
-    # 32-voxel lines (w % 64 != 0): tiles against the per-tap gathers, one and many z steps
+    # 32-voxel lines (w % 64 != 0): tiles against the per-tap gathers, one z step per workgroup
     X = gpu
     net = X.UNet((16, 32), seed=5)
     try:
@@ -208,6 +208,64 @@ def test_narrow_tiles_are_identical(gpu):
             assert np.array_equal(outs[0], outs[1]), (nx, ny, nz)
     finally:
         X.set_option("unet_conv_tile", 1)
+
+
+def net16(X, seed):
+    """one level of 16 channels (1 -> 16 and 16 -> 16) with non-zero biases"""
+    net = X.UNet((16,), seed=seed)
+    p = net.get_params()
+    rng = np.random.default_rng(seed)
+    for sl in layer_slices((16,))[1::2]:
+        p[sl] = rng.standard_normal(sl.stop - sl.start).astype(np.float32) * 0.1
+    net.set_params(p)
+    return net
+
+
+@pytest.mark.parametrize("nx,ny,nz,nv,mz", [
+    # lines of 64 voxels, 512 voxels per tile
+    (128, 128, 128, 1, 2), (128, 128, 64, 4, 4), (128, 128, 64, 8, 8),
+    (64, 64, 12, 64, 2), (64, 64, 20, 64, 2), (64, 64, 24, 64, 4),
+    # lines of 32, 256 voxels per tile
+    (32, 64, 12, 64, 2), (96, 32, 16, 64, 4), (32, 64, 32, 64, 8), (32, 64, 24, 64, 4)])
+def test_marching_tile_is_identical(gpu, nx, ny, nz, nv, mz):
+    # the 16 -> 16 convolution walks mz z steps of 2 planes over its ring of 4 planes: mz
+    # doubles up to 8 while it divides nz / 2 and at least 2048 workgroups are left
+    X = gpu
+    tiles, m = nx * ny * nz * nv // (512 if nx % 64 == 0 else 256), 1
+    while m < 8 and (nz // 2) % (2 * m) == 0 and tiles // (2 * m) >= 2048:
+        m *= 2
+    assert m == mz
+    net, V = net16(X, 7), nx * ny * nz
+    b = X.DeviceArray.from_host(np.random.default_rng(nx + nz).standard_normal(V * nv))
+    outs = []
+    try:
+        for tile in (0, 1):
+            X.set_option("unet_conv_tile", tile)
+            x = X.DeviceArray(V * nv)
+            net.infer(nx, ny, nz, nv, b, x)
+            outs.append(x.to_host())
+    finally:
+        X.set_option("unet_conv_tile", 1)
+    assert np.isfinite(outs[0]).all() and np.abs(outs[0]).max() > 0
+    assert np.array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("n,d,h,w", [(64, 24, 32, 32), (64, 16, 32, 64), (64, 32, 32, 32)])
+def test_marching_tile_gradients_are_identical(gpu, n, d, h, w):
+    # the same kernel on a data gradient, through the relu's mask (2, 2 and 4 z steps)
+    X = gpu
+    net, rng = net16(X, 8), np.random.default_rng(d)
+    x, t = (rng.standard_normal((n, d, h, w)).astype(np.float32) for _ in range(2))
+    outs = []
+    try:
+        for tile in (0, 1):
+            X.set_option("unet_conv_tile", tile)
+            outs.append(net.loss_grad(x, t))
+    finally:
+        X.set_option("unet_conv_tile", 1)
+    assert outs[0][0] == outs[1][0]
+    assert np.abs(outs[0][1]).max() > 0 and np.array_equal(outs[0][1], outs[1][1])
+    assert np.array_equal(outs[0][2], outs[1][2])
 
 
 @pytest.mark.parametrize("nv", [2, 3])
