@@ -67,8 +67,9 @@ def test_spmv_irregular_rows_bit_exact(gpu, O, nv):
 @pytest.mark.parametrize("prec", [0, 1])
 def test_spmv_wide_batches_bit_exact(gpu, O, nv, prec):
     # few rows of many entries (the coarse levels of an aggressively coarsened hierarchy)
-    # take the 16-wide batches: the same sums in the same order as the 8-wide kernel and,
-    # in fp64, as the oracle; y = A x and y += A x, u16 and u32 columns, empty rows
+    # take the 16-wide batches (with the long-row kernel off, which is faster on fewer rows):
+    # the same sums in the same order as the 8-wide kernel and, in fp64, as the oracle;
+    # y = A x and y += A x, u16 and u32 columns, empty rows
     X = gpu
     rng = np.random.default_rng(nv * 7 + prec)
     n = 2000
@@ -83,6 +84,7 @@ def test_spmv_wide_batches_bit_exact(gpu, O, nv, prec):
     x = rng.standard_normal(n * nv)
     y0 = np.linspace(-1, 1, n * nv)
     try:
+        X.set_option("spmv_wave_enable", 0)
         for index_mode in (1, 2):
             A = X.Matrix(row, col, val, prec=prec, index_mode=index_mode)
             out = []
@@ -100,18 +102,20 @@ def test_spmv_wide_batches_bit_exact(gpu, O, nv, prec):
                 assert np.array_equal(out[1][0], O.spmv(row, col, val, x, nv))
     finally:
         X.set_option("spmv_wide_batches", 1)
+        X.set_option("spmv_wave_enable", 2)
 
 
 def test_wide_batches_in_the_coarse_levels(gpu):
     # the coarse levels of the aggressively coarsened 64^3 cube (levels 2 and 3: 2295 and
-    # 587 rows of 34 and 45 entries) take the 16-wide SpMVs; the preconditioner is
-    # bit-identical with them off
+    # 587 rows of 34 and 45 entries) take the 16-wide SpMVs with the long-row kernel off; the
+    # preconditioner is bit-identical with them off
     X = gpu
     row, col, val = X.cube(64)
     levels = X.Amg(row, col, val, agg_num_levels=2, num_paths=2, coarse_size=500).export()
     n = len(row) - 1
     prm = X.default_params(method="MergedPBiCGStab", smoother="Chebyshev", poly_order=4)
     try:
+        X.set_option("spmv_wave_enable", 0)
         for nv in (8, 32):
             b = X.rhs_uniform(nv, n, nv)
             out, names = [], []
@@ -124,11 +128,35 @@ def test_wide_batches_in_the_coarse_levels(gpu):
                 dx.zero()
                 names.append({(k["kernel"], k["level"]) for k in S.profile(db, dx, 1)})
             assert np.array_equal(out[0], out[1]), nv
-            assert not any(k.endswith(",16>") for k, _ in names[0])
-            assert any(k.endswith(",16>") and lv >= 2 for k, lv in names[1]), names[1]
-            assert not any(k.endswith(",16>") and lv == 0 for k, lv in names[1])
+            wide = [{lv for k, lv in q if k.startswith("k_spmv<") and k.endswith(",16>")}
+                    for q in names]
+            assert not wide[0]
+            assert max(wide[1]) >= 2 and 0 not in wide[1], names[1]
+            assert not any(k.startswith("k_spmv_wave<") for q in names for k, _ in q)
     finally:
         X.set_option("spmv_wide_batches", 1)
+        X.set_option("spmv_wave_enable", 2)
+
+
+@pytest.mark.parametrize("nv", [8, 32])
+def test_long_row_kernel_in_the_coarse_levels(gpu, nv):
+    # by default the same levels take the long-row kernel: at nv = 8 both, at nv = 32 (a cap of
+    # 1536 rows) the 587 rows, the 2295 rows the 16-wide SpMVs
+    X = gpu
+    row, col, val = X.cube(64)
+    levels = X.Amg(row, col, val, agg_num_levels=2, num_paths=2, coarse_size=500).export()
+    prm = X.default_params(method="MergedPBiCGStab", smoother="Chebyshev", poly_order=4)
+    S = X.Solver(X.Hier(levels), prm, nv)
+    n = len(row) - 1
+    db, dx = X.DeviceArray.from_host(X.rhs_uniform(nv, n, nv)), X.DeviceArray(n * nv)
+    dx.zero()
+    names = {(k["kernel"], k["level"]) for k in S.profile(db, dx, 1) if "OP_CHEB" in k["kernel"]}
+    for lv, wave in ((2, nv == 8), (3, True)):
+        if not any(q == lv for _, q in names):
+            continue  # the coarsest level is solved directly
+        want = "k_spmv_wave<" if wave else "k_spmv<"
+        assert all(k.startswith(want) and k.endswith(",16>") for k, q in names if q == lv), names
+    assert any(q == 2 for _, q in names)
 
 
 def test_spmv_order_sensitive_row(gpu):
