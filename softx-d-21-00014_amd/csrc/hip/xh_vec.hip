@@ -281,6 +281,29 @@ __global__ __launch_bounds__(kBlock) void k_jacobi(int64_t count, int nv, VT *__
     }
 }
 
+// y = D x with one output per thread, which walks its n columns in memory: the small products,
+// whose whole D is a few tiles, and those with many outputs per row of D (dense_tiled)
+template <typename VT, typename XT>
+__global__ __launch_bounds__(kBlock) void k_dense_direct(int64_t n, int nv,
+                                                         const VT *__restrict__ D,
+                                                         const XT *__restrict__ x,
+                                                         XT *__restrict__ y,
+                                                         const int *__restrict__ done) {
+    if (done != nullptr && *done)
+        return;
+    const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (e >= n * nv)
+        return;
+    const int64_t i = e / nv;
+    const int k = (int)(e % nv);
+    VT acc = VT(0);
+    // j order as dense_Ax_y; unrolled so that many loads are in flight
+#pragma unroll 16
+    for (int64_t j = 0; j < n; ++j)
+        acc = acc + D[i * n + j] * (VT)x[j * nv + k];
+    y[e] = (XT)acc;
+}
+
 // y = D x, D dense n x n (the coarsest level's inverse, n of a few hundred): every output is
 // a sum of n terms added one by one in column order (the rounding of dense_Ax_y), so the
 // time cannot go below n dependent adds; what is left to hide is memory.  A workgroup owns
@@ -565,14 +588,34 @@ void jacobi_update(int64_t n, int nv, int prec, void *x, const void *b, const vo
                            (const float *)inv_diag, (float)relax, x_zero, done);
 }
 
+// Whether the product runs in tiles (k_dense).  A tile's barriers and the four tiles loaded
+// ahead cost a small product more than they hide; with 64 right-hand sides, and 16 or 32 in
+// fp32, a row of D is read by a whole wave at once already, so the direct kernel waits
+// less per term.  us per call, direct / tiled: fp64 nv = 8, n = 48 14.6 / 14.7, 100 17.1 / 16.3,
+// 500 33.6 / 26.1; nv = 64, n = 100 17.4 / 20.0, 1000 57.1 / 63.2, 1200 114 / 64 (D leaves the
+// L2 caches); fp32 nv = 8, n = 160 15.6 / 15.7, 200 17.0 / 16.2; nv = 16, n = 500 22.9 / 24.8, 2500
+// 65 / 77, 3000 110 / 89; nv = 32, n = 257 17.9 / 18.8, 500 23.0 / 22.3; nv = 64, n = 1000 34.4 /
+// 41.7, 1200 50.5 / 41.0.
+bool dense_tiled(int64_t n, int nv, int prec) {
+    if (nv == 64)
+        return n >= 1100;
+    if (prec == F64)
+        return n >= 96;
+    return n >= (nv <= 8 ? 180 : nv == 16 ? 2800 : 450);
+}
+
 template <typename VT, typename XT, int NV>
 void dense_t(int64_t n, const void *D, const void *x, void *y, const int *done, hipStream_t s) {
-    // two waves per workgroup while that gives at most 2 workgroups per CU
+    // two waves per workgroup while that gives at most 2 workgroups per CU (never with 64
+    // right-hand sides, whose small products are direct)
     constexpr int R1 = DenseShape<NV, 2>::RB, R4 = DenseShape<NV, 4>::RB;
-    if (R1 == R4 || (n + R1 - 1) / R1 <= 512)
-        hipLaunchKernelGGL((k_dense<VT, XT, NV, 2>), dim3((unsigned)((n + R1 - 1) / R1)), dim3(128),
-                           0, s, n, (const VT *)D, (const XT *)x, (XT *)y, done);
-    else
+    if constexpr (NV < 64)
+        if (R1 == R4 || (n + R1 - 1) / R1 <= 512) {
+            hipLaunchKernelGGL((k_dense<VT, XT, NV, 2>), dim3((unsigned)((n + R1 - 1) / R1)),
+                               dim3(128), 0, s, n, (const VT *)D, (const XT *)x, (XT *)y, done);
+            return;
+        }
+    if constexpr (NV == 64 || R1 != R4)
         hipLaunchKernelGGL((k_dense<VT, XT, NV, 4>), dim3((unsigned)((n + R4 - 1) / R4)), dim3(256),
                            0, s, n, (const VT *)D, (const XT *)x, (XT *)y, done);
 }
@@ -580,6 +623,12 @@ void dense_t(int64_t n, const void *D, const void *x, void *y, const int *done, 
 template <typename VT, typename XT>
 void dense_nv(int64_t n, int nv, const void *D, const void *x, void *y, const int *done,
               hipStream_t s) {
+    if (!dense_tiled(n, nv, sizeof(VT) == 8 ? F64 : F32)) {
+        const dim3 grid((unsigned)((n * nv + kBlock - 1) / kBlock));
+        hipLaunchKernelGGL((k_dense_direct<VT, XT>), grid, dim3(kBlock), 0, s, n, nv, (const VT *)D,
+                           (const XT *)x, (XT *)y, done);
+        return;
+    }
     switch (nv) {
     case 1:
         return dense_t<VT, XT, 1>(n, D, x, y, done, s);
@@ -603,7 +652,8 @@ void dense_matvec(int64_t n, int nv, int prec, int xprec, const void *D, const v
     LedgerScope led(s);
     if (led.on) {
         const double sv = prec == F64 ? 8.0 : 4.0, sx = xprec == F64 ? 8.0 : 4.0;
-        led.kernel = std::string("k_dense<") + prec_name(prec) + "," + prec_name(xprec) + ">";
+        led.kernel = std::string(dense_tiled(n, nv, prec) ? "k_dense<" : "k_dense_direct<") +
+                     prec_name(prec) + "," + prec_name(xprec) + ">";
         led.bytes = sv * (double)(n * n) + 2.0 * sx * (double)(n * nv); // D, x, y
     }
     if (prec == F64 && xprec == F64)

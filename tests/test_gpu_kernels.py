@@ -190,12 +190,18 @@ def test_dense_matvec_bit_exact(gpu, O):
 
 @pytest.mark.parametrize("n,nv", [(1, 1), (33, 1), (63, 2), (64, 4), (65, 8), (129, 16),
                                   (200, 32), (7, 64), (191, 64),
-                                  (1100, 32), (530, 64), (700, 1)])
+                                  (1100, 32), (530, 64), (700, 1),
+                                  # the first sizes in tiles and the last without, by nv
+                                  (95, 1), (96, 1), (96, 2), (127, 4), (128, 8), (193, 32),
+                                  (179, 8), (180, 8), (192, 2), (449, 32), (450, 32), (1099, 64),
+                                  (2799, 16), (2800, 16),
+                                  # four waves per workgroup
+                                  (1100, 64), (1153, 64), (2049, 32), (4097, 16)])
 @pytest.mark.parametrize("prec", [0, 1])
 def test_dense_matvec_tile_edges_bit_exact(gpu, n, nv, prec):
     # sums in column order with separate multiply and add, at the edges of the row blocks
-    # (1 to 32 rows), of the 64-column tiles (one, even and odd tile counts) and of the
-    # two-wave and four-wave variants
+    # (1 to 32 rows), of the 64-column tiles (one, even and odd tile counts), of the direct
+    # and the tiled kernel, and of the two-wave and four-wave variants
     X = gpu
     rng = np.random.default_rng(n + nv)
     dt = np.float64 if prec == 0 else np.float32
@@ -296,6 +302,26 @@ def test_long_row_kernel_in_a_vcycle_is_identical(gpu, smoother, nv, mg_prec):
     finally:
         X.set_option("spmv_wave_enable", 2)
     assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
+
+
+@pytest.mark.parametrize("coarse_size,nv,mg_prec", [(60, 8, 0), (60, 4, 2), (600, 8, 0),
+                                                    (600, 1, 2), (600, 64, 0), (600, 16, 1)])
+def test_dense_kernel_by_size(gpu, coarse_size, nv, mg_prec):
+    # small coarse levels, and those with 64 RHS or 16 in fp32, are solved by one thread per
+    # output, the others in tiles; the fp64 solve of an fp32 hierarchy reads its vectors as
+    # they are
+    X = gpu
+    row, col, val = X.cube(16)
+    levels = X.Amg(row, col, val, agg_num_levels=1, num_paths=2, coarse_size=coarse_size).export()
+    nc, n = levels[-1]["A"][0], len(row) - 1
+    assert (nc < 96) == (coarse_size == 60) and nc < 1100
+    S = X.Solver(X.Hier(levels), X.default_params(mg_prec=mg_prec), nv)
+    db, dx = X.DeviceArray.from_host(X.rhs_uniform(2, n, nv)), X.DeviceArray(n * nv)
+    dx.zero()
+    names = {k["kernel"] for k in S.profile(db, dx, 1)}
+    tiled = coarse_size == 600 and not (nv == 64 or (mg_prec == 1 and nv == 16))
+    types = {0: "double,double", 1: "float,float", 2: "double,float"}[mg_prec]
+    assert f"k_dense{'' if tiled else '_direct'}<{types}>" in names, (nc, names)
 
 
 def test_spmv_full_size_cube_128(gpu, O):
