@@ -87,7 +87,7 @@ __device__ __forceinline__ int64_t neigh(const Dims &g, int64_t m, int t) {
 // tiles, so every B fragment feeds MT MFMAs.  UP: `in` is the coarse volume of a nearest
 // x2 upsampling (d/2 x h/2 x w/2) and the fine neighbour (z, y, x) reads coarse voxel
 // (z/2, y/2, x/2): the upsampled tensor is never written.
-template <int CT, int MT, bool UP>
+template <int CT, int MT, bool UP, int PF>
 __global__ __launch_bounds__(256) void k_conv(Dims g, const bf16_t *__restrict__ in, int cin,
                                               const bf16_t *__restrict__ wt, int kpad,
                                               const float *__restrict__ bias,
@@ -121,10 +121,8 @@ __global__ __launch_bounds__(256) void k_conv(Dims g, const bf16_t *__restrict__
 #pragma unroll
         for (int c = 0; c < CT; ++c)
             acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // The operands of the next PF k steps are in flight while a step computes: on the deep
-    // levels (a few hundred waves, 54 steps of 64 channels) a step otherwise waits a memory
-    // round trip (16 volumes of 4^3, 64 channels: 77 -> 29 us).
-    constexpr int PF = 3;
+    // PF > 1: the operands of the next PF k steps are in flight while a step computes; 1: a
+    // step loads its own (launch_conv)
     bf16x8 a[PF][MT];
     uint4 qb[PF][CT];
     // tap and channel of the lane's k in the step being loaded, advanced by 32 per step
@@ -185,22 +183,26 @@ __global__ __launch_bounds__(256) void k_conv(Dims g, const bf16_t *__restrict__
         for (int c = 0; c < CT; ++c)
             bv[c] = *reinterpret_cast<const uint4 *>(wt + (size_t)(c * 16 + r) * kpad + k0);
     };
+    if constexpr (PF > 1) {
 #pragma unroll
-    for (int q = 0; q < PF; ++q)
-        if (32 * q < kpad)
-            load(32 * q, a[q], qb[q]);
+        for (int q = 0; q < PF; ++q)
+            if (32 * q < kpad)
+                load(32 * q, a[q], qb[q]);
+    }
     for (int kb = 0; kb < kpad; kb += 32 * PF) {
 #pragma unroll
         for (int q = 0; q < PF; ++q) {
             const int ks = kb + 32 * q;
             if (ks < kpad) { // uniform
+                if constexpr (PF == 1)
+                    load(ks, a[q], qb[q]);
 #pragma unroll
                 for (int c = 0; c < CT; ++c)
 #pragma unroll
                     for (int t = 0; t < MT; ++t)
                         acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                             a[q][t], __builtin_bit_cast(bf16x8, qb[q][c]), acc[t][c], 0, 0, 0);
-                if (ks + 32 * PF < kpad)
+                if (PF > 1 && ks + 32 * PF < kpad)
                     load(ks + 32 * PF, a[q], qb[q]);
             }
         }
@@ -1418,8 +1420,23 @@ void launch_conv(const Dims &g, const bf16_t *in, int cin, const bf16_t *wt, int
                  const float *bias, const bf16_t *add, const bf16_t *mask, int relu, bf16_t *out,
                  hipStream_t s) {
     constexpr int MT = CT >= 3 ? 1 : 4 / CT;
-    const dim3 grid((unsigned)((g.vox() + 64 * MT - 1) / (64 * MT))), blk(256);
-    hipLaunchKernelGGL((k_conv<CT, MT, UP>), grid, blk, 0, s, g, in, cin, wt, kpad, bias, add,
+    const int64_t wgs = (g.vox() + 64 * MT - 1) / (64 * MT);
+    const dim3 grid((unsigned)wgs), blk(256);
+    // Operands of three k steps in flight: pays where a wave has many steps and few other
+    // waves beside it, and costs registers, so waves per SIMD, where there are enough.  us, own
+    // loads / three ahead: 48 -> 48 channels, 8192 voxels (128 workgroups) 38 / 20, 32768 41 / 26,
+    // 1M 1363 / 1364; 64 -> 64, 8192 voxels 42 / 34; 32 -> 32, 65536 voxels (512 workgroups) 25.2 /
+    // 22.4, 524288 (4096) 112 / 117.  With 16 output channels it loses at every size (16 -> 16,
+    // 262144 voxels 28 / 37, 8.4M 673 / 820; upsampled 32 -> 16 8.4M 1065 / 1271), and with one
+    // k step, the single-channel input, there is nothing to load ahead (1 -> 64, 8.4M 623 /
+    // 913).
+    if constexpr (CT > 1)
+        if (cin > 1 && (CT >= 3 || wgs <= 512)) {
+            hipLaunchKernelGGL((k_conv<CT, MT, UP, 3>), grid, blk, 0, s, g, in, cin, wt, kpad,
+                               bias, add, mask, relu, out);
+            return;
+        }
+    hipLaunchKernelGGL((k_conv<CT, MT, UP, 1>), grid, blk, 0, s, g, in, cin, wt, kpad, bias, add,
                        mask, relu, out);
 }
 

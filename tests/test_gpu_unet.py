@@ -210,6 +210,28 @@ def test_narrow_tiles_are_identical(gpu):
         X.set_option("unet_conv_tile", 1)
 
 
+@pytest.mark.parametrize("channels,nx,ny,nz,nv", [
+    ((32,), 64, 32, 32, 1),      # 512 workgroups of 128 voxels: three k steps ahead
+    ((32,), 64, 32, 36, 1),      # more: own loads
+    ((48,), 32, 8, 8, 1), ((48,), 32, 32, 36, 2), ((16, 32), 128, 64, 24, 1)])
+def test_gather_convolution_by_size_is_identical(gpu, channels, nx, ny, nz, nv):
+    # the per-tap gathers that load k steps ahead and those that do not, against the tiles
+    X = gpu
+    net, V = X.UNet(channels, seed=11), nx * ny * nz
+    b = X.DeviceArray.from_host(np.random.default_rng(nz).standard_normal(V * nv))
+    outs = []
+    try:
+        for tile in (0, 1):
+            X.set_option("unet_conv_tile", tile)
+            x = X.DeviceArray(V * nv)
+            net.infer(nx, ny, nz, nv, b, x)
+            outs.append(x.to_host())
+    finally:
+        X.set_option("unet_conv_tile", 1)
+    assert np.isfinite(outs[0]).all() and np.abs(outs[0]).max() > 0
+    assert np.array_equal(outs[0], outs[1])
+
+
 def net16(X, seed):
     """one level of 16 channels (1 -> 16 and 16 -> 16) with non-zero biases"""
     net = X.UNet((16,), seed=seed)
