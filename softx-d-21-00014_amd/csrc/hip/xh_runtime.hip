@@ -475,11 +475,14 @@ int upload_core(const HostCsr &h, int64_t B, int nv, int prec, const Mat &A, Mat
     auto padded = [](int64_t c, int kb) { return std::max<int64_t>(kb, (c + kb - 1) / kb * kb); };
     // KB: the width whose rows take the least time in the sweep's serial chain, a batch
     // costing one LDS round trip (about as long as 12 subtractions) and its KB subtractions,
-    // among the widths whose pads leave the largest block in LDS (with 64 RHS the pads of 6
-    // or 8 can be what does not fit; 20^3 27-point, blocks of 104 rows, fp64, us for two sweeps:
-    // 370 by the kernel without staging, 69 with batches of 3)
+    // among the widths whose pads leave the largest block in LDS if any does (with 64 RHS the
+    // pads of 6 or 8 can be what does not fit; 20^3 27-point, blocks of 104 rows, fp64, us for
+    // two sweeps: 370 by the kernel without staging, 69 with batches of 3).  Where none does,
+    // wide batches suit the unrolled loop of that kernel too (blocks of 300 rows: 22.0 / 23.2
+    // ms per V-cycle of the 40^3 cube with 8 / 3)
     int KB = 3;
     int64_t best = -1;
+    bool best_fits = false;
     for (int kb : {3, 4, 6, 8}) {
         int64_t cost = 0, emax = 0;
         for (int64_t lo = 0; lo < n; lo += B) {
@@ -490,8 +493,9 @@ int upload_core(const HostCsr &h, int64_t B, int nv, int prec, const Mat &A, Mat
             emax = std::max(emax, e);
         }
         const bool fits = hsgs_core_bytes(B, nv, emax, prec == F64 ? 8 : 4) <= kHsgsLds;
-        if (fits && (best < 0 || cost < best)) {
+        if (best < 0 || fits > best_fits || (fits == best_fits && cost < best)) {
             best = cost;
+            best_fits = fits;
             KB = kb;
         }
     }
