@@ -505,9 +505,10 @@ inline size_t hsgs_core_bytes(int64_t B, int nv, int64_t emax, int sv) {
     return ((size_t)(B + 1) * nv * sv + (size_t)emax * (sv + 4) + (size_t)B * sv +
             (size_t)(B + 1) * 4 + 15) / 16 * 16;
 }
-// y = D x; prec: precision of D and of the sums, xprec: of x and y (F64, or prec)
+// y = D x; prec: precision of D and of the sums, xprec: of x and y (F64, or prec); warm: not
+// between the other levels of a solve
 void dense_matvec(int64_t n, int nv, int prec, int xprec, const void *D, const void *x, void *y,
-                  const int *done, hipStream_t s);
+                  bool warm, const int *done, hipStream_t s);
 void convert(int64_t count, int from_prec, const void *src, void *dst, const int *done,
              hipStream_t s);
 void copy_vec(int64_t count, int prec, const void *src, void *dst, const int *done,

@@ -850,7 +850,7 @@ void smooth(xh_solver_s *S, const xh_role &role, Level &L, const std::vector<dou
         return;
     }
     case XH_DIRECT: {
-        dense_matvec(L.n, nv, L.dinv_prec, L.prec, L.dinv, b, x, S->dflag, st);
+        dense_matvec(L.n, nv, L.dinv_prec, L.prec, L.dinv, b, x, false, S->dflag, st);
         return;
     }
     case XH_IDENTITY:
@@ -1461,7 +1461,7 @@ int xh_spmv_timed(xh_matrix A, int nv, const void *dx, void *dy, int accumulate,
 int xh_dense_matvec(int64_t n, int nv, int prec, const void *dD, const void *dx, void *dy) {
     if (n <= 0 || !nv_ok(nv) || !dD || !dx || !dy)
         return fail(XH_EINVAL, "xh_dense_matvec: bad arguments");
-    dense_matvec(n, nv, prec, prec, dD, dx, dy, nullptr, g_stream);
+    dense_matvec(n, nv, prec, prec, dD, dx, dy, true, nullptr, g_stream);
     XH_HIP(hipGetLastError());
     XH_HIP(hipStreamSynchronize(g_stream));
     return 0;

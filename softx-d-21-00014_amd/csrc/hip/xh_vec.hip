@@ -282,7 +282,7 @@ __global__ __launch_bounds__(kBlock) void k_jacobi(int64_t count, int nv, VT *__
 }
 
 // y = D x with one output per thread, which walks its n columns in memory: the small products,
-// whose whole D is a few tiles, and those with many outputs per row of D (dense_tiled)
+// whose whole D is a tile or less, and products called on their own (dense_tiled)
 template <typename VT, typename XT>
 __global__ __launch_bounds__(kBlock) void k_dense_direct(int64_t n, int nv,
                                                          const VT *__restrict__ D,
@@ -588,15 +588,20 @@ void jacobi_update(int64_t n, int nv, int prec, void *x, const void *b, const vo
                            (const float *)inv_diag, (float)relax, x_zero, done);
 }
 
-// Whether the product runs in tiles (k_dense).  A tile's barriers and the four tiles loaded
-// ahead cost a small product more than they hide; with 64 right-hand sides, and 16 or 32 in
-// fp32, a row of D is read by a whole wave at once already, so the direct kernel waits
-// less per term.  us per call, direct / tiled: fp64 nv = 8, n = 48 14.6 / 14.7, 100 17.1 / 16.3,
-// 500 33.6 / 26.1; nv = 64, n = 100 17.4 / 20.0, 1000 57.1 / 63.2, 1200 114 / 64 (D leaves the
-// L2 caches); fp32 nv = 8, n = 160 15.6 / 15.7, 200 17.0 / 16.2; nv = 16, n = 500 22.9 / 24.8, 2500
-// 65 / 77, 3000 110 / 89; nv = 32, n = 257 17.9 / 18.8, 500 23.0 / 22.3; nv = 64, n = 1000 34.4 /
-// 41.7, 1200 50.5 / 41.0.
-bool dense_tiled(int64_t n, int nv, int prec) {
+// Whether the product runs in tiles (k_dense).  Inside a solve D has left the L2 caches since
+// its last use, and the tiles, loaded four ahead, hide that: event-timed launches in us,
+// direct / tiled: fp64 nv = 8, n = 45 7.7 / 6.4, nv = 64, n = 512 33 / 26, 1000 70 / 55; fp32 nv =
+// 16, n = 512 18.6 / 16.7, 1728 64 / 46.  Only 64 right-hand sides and a D of less than a tile
+// are better without (n = 33 6.4 / 9.2, 45 9.9 / 9.7).
+// Called on its own, again on the same D (warm), a small product pays for the tiles'
+// barriers, and with 64 right-hand sides, or 16 and 32 in fp32, a whole wave reads a row of D
+// at once already.  us per call, direct / tiled: fp64 nv = 8, n = 48 14.6 / 14.7, 100 17.1 / 16.3,
+// 500 33.6 / 26.1; nv = 64, n = 100 17.4 / 20.0, 1000 57.1 / 63.2, 1200 114 / 64; fp32 nv = 8, n = 160
+// 15.6 / 15.7, 200 17.0 / 16.2; nv = 16, n = 500 22.9 / 24.8, 2500 65 / 77, 3000 110 / 89; nv = 32, n =
+// 257 17.9 / 18.8, 500 23.0 / 22.3; nv = 64, n = 1000 34.4 / 41.7, 1200 50.5 / 41.0.
+bool dense_tiled(int64_t n, int nv, int prec, bool warm) {
+    if (!warm)
+        return nv < 64 || n >= 40;
     if (nv == 64)
         return n >= 1100;
     if (prec == F64)
@@ -606,24 +611,20 @@ bool dense_tiled(int64_t n, int nv, int prec) {
 
 template <typename VT, typename XT, int NV>
 void dense_t(int64_t n, const void *D, const void *x, void *y, const int *done, hipStream_t s) {
-    // two waves per workgroup while that gives at most 2 workgroups per CU (never with 64
-    // right-hand sides, whose small products are direct)
+    // two waves per workgroup while that gives at most 2 workgroups per CU
     constexpr int R1 = DenseShape<NV, 2>::RB, R4 = DenseShape<NV, 4>::RB;
-    if constexpr (NV < 64)
-        if (R1 == R4 || (n + R1 - 1) / R1 <= 512) {
-            hipLaunchKernelGGL((k_dense<VT, XT, NV, 2>), dim3((unsigned)((n + R1 - 1) / R1)),
-                               dim3(128), 0, s, n, (const VT *)D, (const XT *)x, (XT *)y, done);
-            return;
-        }
-    if constexpr (NV == 64 || R1 != R4)
+    if (R1 == R4 || (n + R1 - 1) / R1 <= 512)
+        hipLaunchKernelGGL((k_dense<VT, XT, NV, 2>), dim3((unsigned)((n + R1 - 1) / R1)), dim3(128),
+                           0, s, n, (const VT *)D, (const XT *)x, (XT *)y, done);
+    else
         hipLaunchKernelGGL((k_dense<VT, XT, NV, 4>), dim3((unsigned)((n + R4 - 1) / R4)), dim3(256),
                            0, s, n, (const VT *)D, (const XT *)x, (XT *)y, done);
 }
 
 template <typename VT, typename XT>
-void dense_nv(int64_t n, int nv, const void *D, const void *x, void *y, const int *done,
-              hipStream_t s) {
-    if (!dense_tiled(n, nv, sizeof(VT) == 8 ? F64 : F32)) {
+void dense_nv(int64_t n, int nv, const void *D, const void *x, void *y, bool tiled,
+              const int *done, hipStream_t s) {
+    if (!tiled) {
         const dim3 grid((unsigned)((n * nv + kBlock - 1) / kBlock));
         hipLaunchKernelGGL((k_dense_direct<VT, XT>), grid, dim3(kBlock), 0, s, n, nv, (const VT *)D,
                            (const XT *)x, (XT *)y, done);
@@ -648,20 +649,21 @@ void dense_nv(int64_t n, int nv, const void *D, const void *x, void *y, const in
 }
 
 void dense_matvec(int64_t n, int nv, int prec, int xprec, const void *D, const void *x, void *y,
-                  const int *done, hipStream_t s) {
+                  bool warm, const int *done, hipStream_t s) {
     LedgerScope led(s);
+    const bool tiled = dense_tiled(n, nv, prec, warm);
     if (led.on) {
         const double sv = prec == F64 ? 8.0 : 4.0, sx = xprec == F64 ? 8.0 : 4.0;
-        led.kernel = std::string(dense_tiled(n, nv, prec) ? "k_dense<" : "k_dense_direct<") +
+        led.kernel = std::string(tiled ? "k_dense<" : "k_dense_direct<") +
                      prec_name(prec) + "," + prec_name(xprec) + ">";
         led.bytes = sv * (double)(n * n) + 2.0 * sx * (double)(n * nv); // D, x, y
     }
     if (prec == F64 && xprec == F64)
-        dense_nv<double, double>(n, nv, D, x, y, done, s);
+        dense_nv<double, double>(n, nv, D, x, y, tiled, done, s);
     else if (prec == F64)
-        dense_nv<double, float>(n, nv, D, x, y, done, s);
+        dense_nv<double, float>(n, nv, D, x, y, tiled, done, s);
     else
-        dense_nv<float, float>(n, nv, D, x, y, done, s);
+        dense_nv<float, float>(n, nv, D, x, y, tiled, done, s);
 }
 
 void convert(int64_t count, int from_prec, const void *src, void *dst, const int *done,

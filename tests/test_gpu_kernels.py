@@ -191,7 +191,8 @@ def test_dense_matvec_bit_exact(gpu, O):
 @pytest.mark.parametrize("n,nv", [(1, 1), (33, 1), (63, 2), (64, 4), (65, 8), (129, 16),
                                   (200, 32), (7, 64), (191, 64),
                                   (1100, 32), (530, 64), (700, 1),
-                                  # the first sizes in tiles and the last without, by nv
+                                  # called on its own: the last sizes without tiles and the
+                                  # first with, by nv
                                   (95, 1), (96, 1), (96, 2), (127, 4), (128, 8), (193, 32),
                                   (179, 8), (180, 8), (192, 2), (449, 32), (450, 32), (1099, 64),
                                   (2799, 16), (2800, 16),
@@ -304,24 +305,27 @@ def test_long_row_kernel_in_a_vcycle_is_identical(gpu, smoother, nv, mg_prec):
     assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
 
 
-@pytest.mark.parametrize("coarse_size,nv,mg_prec", [(60, 8, 0), (60, 4, 2), (600, 8, 0),
-                                                    (600, 1, 2), (600, 64, 0), (600, 16, 1)])
-def test_dense_kernel_by_size(gpu, coarse_size, nv, mg_prec):
-    # small coarse levels, and those with 64 RHS or 16 in fp32, are solved by one thread per
-    # output, the others in tiles; the fp64 solve of an fp32 hierarchy reads its vectors as
-    # they are
+@pytest.mark.parametrize("N,coarse_size,nv,mg_prec", [
+    (10, 70, 8, 0), (10, 70, 32, 2), (10, 70, 64, 0), (10, 70, 64, 1), (16, 60, 64, 2),
+    (16, 600, 16, 1), (16, 600, 64, 0), (16, 600, 1, 2)])
+def test_dense_kernel_of_the_coarse_solve(gpu, O, N, coarse_size, nv, mg_prec):
+    # coarse solves run in tiles, but for 64 RHS on less than 40 unknowns (33 here, then 45 and
+    # 512); the fp64 solve of an fp32 hierarchy reads its vectors as they are
     X = gpu
-    row, col, val = X.cube(16)
+    row, col, val = X.cube(N)
     levels = X.Amg(row, col, val, agg_num_levels=1, num_paths=2, coarse_size=coarse_size).export()
     nc, n = levels[-1]["A"][0], len(row) - 1
-    assert (nc < 96) == (coarse_size == 60) and nc < 1100
-    S = X.Solver(X.Hier(levels), X.default_params(mg_prec=mg_prec), nv)
-    db, dx = X.DeviceArray.from_host(X.rhs_uniform(2, n, nv)), X.DeviceArray(n * nv)
+    assert nc == {70: 33, 60: 45, 600: 512}[coarse_size]
+    prm = X.default_params(method="MergedPBiCGStab", mg_prec=mg_prec)
+    S = X.Solver(X.Hier(levels), prm, nv)
+    b = X.rhs_uniform(2, n, nv)
+    db, dx = X.DeviceArray.from_host(b), X.DeviceArray(n * nv)
+    S.precond_apply(db, dx)
+    assert np.array_equal(dx.to_host(), O.mg_apply(O.Hier(levels), O.params_from(prm), nv, b))
     dx.zero()
     names = {k["kernel"] for k in S.profile(db, dx, 1)}
-    tiled = coarse_size == 600 and not (nv == 64 or (mg_prec == 1 and nv == 16))
     types = {0: "double,double", 1: "float,float", 2: "double,float"}[mg_prec]
-    assert f"k_dense{'' if tiled else '_direct'}<{types}>" in names, (nc, names)
+    assert f"k_dense{'_direct' if nv == 64 and nc < 40 else ''}<{types}>" in names, (nc, names)
 
 
 def test_spmv_full_size_cube_128(gpu, O):
