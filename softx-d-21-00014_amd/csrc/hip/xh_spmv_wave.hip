@@ -221,13 +221,16 @@ void by_nv(const Mat &A, int nv, const void *x, void *y, SpmvOp op, const SpmvAr
 } // namespace
 
 // Where this kernel is the faster one.  A wave here costs the instructions of a whole row
-// (the sum runs in L of its 64 lanes), so it pays while the launch has few waves: the caps
-// below are where the two kernels' times crossed on hierarchy levels of 261 to 262144 rows
-// (us, row-parallel / this): L = 2 (nv = 4, fp64), 38 entries: 17391 rows 8.6 / 7.6, and at
-// 24 entries 27366 rows 7.5 / 9.8; L = 4 (nv = 8): 5663 rows 9.3 / 6.6, 17391 rows 7.3 / 12.0;
-// L = 8 (nv = 16): 1259 rows 10.7 / 5.6, 4375 rows 9.5 / 9.6; L = 16 (nv = 32): 440 rows
-// 14.2 / 10.8, 1596 rows 11.8 / 11.7, 4375 rows 8.8 / 15.5.  Short rows (restrictions, 6 to
-// 11 entries) leave less to gain: half the waves.  Below 4 entries a row is one batch there.
+// (the sum runs in L of its 64 lanes) and saves the row-parallel kernel's wait per 8 entries,
+// so it pays while the launch has few rows, and fewer the shorter they are.  The caps are
+// where the two kernels' times crossed on 4080 matrices of hierarchies (all operators,
+// prolongations and restrictions of 7- and 27-point grids of 20^3 to 128^3), time of the
+// row-parallel kernel over this one's: L = 1 32768 rows of 7 0.78, 32768 of 25 1.4, 21952 of 7
+// 1.3; L = 2 (nv = 4, fp64) 9910 of 9 0.95, 7500 of 6 1.2, 17391 of 38 1.14, 27366 of 24 0.7; L = 4
+// (nv = 8) 3470 of 8 0.95, 2500 of 7 1.2, 6912 of 17 0.86, 5700 of 22 1.2, 7000 of 30 1.25, 8500 of
+// 30 0.9; L = 8 (nv = 16) 3470 of 12 0.88, 2500 of 13 1.35, 4375 of 56 1.0; L = 16 (nv = 32) 400 of
+// 6 0.93, 400 of 10 1.05, 440 of 38 1.3, 2200 of 25 0.8.  Below 4 entries a row is one batch
+// there.
 // One right-hand side, and two in fp32, win at every size with long rows (262144 rows of 26:
 // fp64 nv = 1 52.9 / 24.8, fp32 nv = 2 41.1 / 21.8; 163868 rows of 14: 15.0 / 13.0, 12.6 /
 // 11.7), as the row-parallel kernel then has each lane load its own entries.  Two in fp64
@@ -252,10 +255,15 @@ bool takes_wave(const Mat &A, SpmvOp op, int nv) {
     const int L = nv / std::min(nv, A.prec == F64 ? 2 : 4);
     if (A.gcode != nullptr && L > 1)
         return false;
-    const int64_t waves = L >= 4 ? A.nrows : A.nrows * L / 4;
-    const int64_t cap = L == 1 ? 8192 : L == 2 ? 10240 : L == 4 ? 8192 : L == 8 ? 4096
-                        : L == 16 ? 1536 : 0;
-    return waves <= (longrows || L == 1 ? cap : cap / 2);
+    // most rows by entries per row: 4 to 12, 12 to 26, more
+    static const int64_t cap[5][3] = {{24576, 32768, 32768}, // L = 1
+                                      {8192, 20480, 20480},  // 2
+                                      {3072, 6144, 7680},    // 4
+                                      {2048, 3072, 4096},    // 8
+                                      {768, 1536, 1536}};    // 16
+    if (L > 16 || (L == 16 && A.nnz < 9 * A.nrows))
+        return false;
+    return A.nrows <= cap[__builtin_ctz(L)][!longrows ? 0 : A.nnz < 26 * A.nrows ? 1 : 2];
 }
 
 int wave_entries(const Mat &A, int nv) {

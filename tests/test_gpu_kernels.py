@@ -280,6 +280,23 @@ def test_long_row_kernel_by_size_on_codes(gpu, nv, mg_prec, dims, want):
     assert bool(took) == want, names
 
 
+@pytest.mark.parametrize("N,nv,want", [(28, 1, True), (32, 1, False), (28, 2, True),
+                                       (32, 2, False), (12, 4, False)])
+def test_long_row_kernel_by_size_on_short_rows(gpu, N, nv, want):
+    # 7-point operators (4 to 12 entries per row) in the default mode: the long-row kernel up
+    # to 24576 rows with one lane per entry, with more lanes none of a matrix with a grid view
+    X = gpu
+    row, col, val = X.varcoef7(N, sigma=1.0, seed=3)[:3]
+    levels = X.Amg(row, col, val, agg_num_levels=1, coarse_size=60).export()
+    prm = X.default_params(method="MergedPBiCGStab", smoother="Jacobi", sweeps=2)
+    S = X.Solver(X.Hier(levels), prm, nv)
+    db, dx = X.DeviceArray.from_host(X.rhs_uniform(1, N ** 3, nv)), X.DeviceArray(N ** 3 * nv)
+    dx.zero()
+    names = {k["kernel"] for k in S.profile(db, dx, 1)
+             if k["level"] == 0 and "OP_RESID" in k["kernel"] and "RESID0" not in k["kernel"]}
+    assert any(k.startswith("k_spmv_wave<") for k in names) == want, names
+
+
 @pytest.mark.parametrize("smoother,nv,mg_prec", [("Chebyshev", 1, 0), ("Chebyshev", 8, 2),
                                                  ("Chebyshev", 32, 1), ("Jacobi", 4, 0),
                                                  ("HSGS", 2, 2), ("Chebyshev", 64, 0)])
