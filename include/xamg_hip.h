@@ -117,8 +117,8 @@ int xh_matrix_fold(xh_matrix A, int64_t set, int64_t *fold);
  * entry couples grid neighbours (|dx|, |dy|, |dz| <= 1; 7- and 27-point operators).  Such
  * a matrix can run the SpMV on 1-byte neighbour codes instead of column indices, or as a
  * sweep along x over tiles of grid lines with the x rows of the tile and its halo lines
- * staged in LDS ("spmv_grid_enable").  No reference counterpart (the reference's csr_Ax_y is row-parallel, src/blas2/
- * detail/csr_matvec.inl:149-260); the arithmetic is that of the row-parallel kernel.
+ * staged in LDS ("spmv_grid_enable").  No reference counterpart (the reference's csr_Ax_y is
+ * row-parallel, src/blas2/detail/csr_matvec.inl:149-260); the arithmetic is that of the row-parallel kernel.
  * xh_matrix_grid: dims = {nx, ny, nz}, zeros when the matrix has no grid view.
  * xh_csr_grid: the same detection on a host CSR; code
  * (nullable, nnz bytes) receives 9(dz+1) + 3(dy+1) + (dx+1) per entry or 255, coded the
@@ -161,7 +161,8 @@ int xh_spmv_schedule(int64_t nrows, int64_t nnz, int64_t fold, int prec, int nv,
  * neighbour codes instead of columns where they are the faster ones, for more than 4
  * right-hand sides when the launch's matrix, x and y are at least "spmv_codes_min_bytes"
  * together (default 200 MB), and the fp64 SpMMs with dot partials for 16 or 32
- * right-hand sides run the sweep where its work items fill the chip; 0 neither), "spmv_grid_items" (default 2048),
+ * right-hand sides run the sweep where its work items fill the chip; 0 neither),
+ * "spmv_grid_items" (default 2048),
  * "cheb_fuse_zero" (0/1, default 1: a Chebyshev smoother from a zero x runs its first two
  * steps as one SpMV that gathers b and forms the first step's values per entry,
  * bit-identical to two launches), "hsgs_offblock_csr" (0/1, default 1, read at solver
@@ -178,9 +179,9 @@ int xh_spmv_schedule(int64_t nrows, int64_t nnz, int64_t fold, int prec, int nv,
  * order unchanged),
  * "spmv_grid_min_seg" (default 32), "unet_fuse_up" (0/1, default 1: the U-Net reads
  * the decoder's upsampled inputs through the convolution instead of writing them),
- * "unet_conv_tile" (0/1, default 1: convolutions with 16 output channels on volumes of
- * w % 32 == h % 4 == d % 2 == 0, with 32 on w % 64 == 0 and with 48 on w % 32 == 0 read their
- * input from LDS-staged tiles). */
+ * "unet_conv_tile" (0/1, default 1: on volumes of h % 4 == d % 2 == 0, convolutions with 16 or
+ * 48 output channels on w % 32 == 0, and with 32 on w % 64 == 0 or, from 16 channels, w % 32 ==
+ * 0, read their input from LDS-staged tiles). */
 int xh_set_option(const char *key, int64_t value);
 
 /* Compressed block: the reference's compact-index CSR block, as csr_matrix::compress

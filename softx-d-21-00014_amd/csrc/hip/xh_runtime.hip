@@ -1123,7 +1123,7 @@ void enqueue_iteration(xh_solver_s *S, double *x, bool replace) {
         finalize(FIN_OMEGA_MERGED, S->st, S->partials, np, nv, st);
         VecArgs vx;
         vx.st = S->st;
-            vx.p_ = S->p;
+        vx.p_ = S->p;
         vx.s_ = S->s;
         vx.gate = 1;
         vec_op(V_X_UPDATE, S->n, nv, vx, st);
@@ -1138,7 +1138,7 @@ void enqueue_iteration(xh_solver_s *S, double *x, bool replace) {
         finalize(FIN_BETA, S->st, S->partials, np, nv, st);
         VecArgs v5;
         v5.st = S->st;
-            v5.p = S->p;
+        v5.p = S->p;
         v5.s = S->s;
         v5.r = S->r;
         v5.v = S->v;

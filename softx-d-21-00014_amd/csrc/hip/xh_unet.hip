@@ -1462,9 +1462,9 @@ bool launch_conv_tile(const Dims &g, const bf16_t *in, const bf16_t *wt, int kpa
 
 // The convolution cin -> cout over LDS-staged tiles, if it has a tile kernel and the tiles
 // divide the volume (false: nothing launched).  16 output channels on lines of 64 or 32
-// voxels, 32 on lines of 64, 48 on lines of 32 (the widths those layers have at 128^3 and on
-// 32^3 crops); the staged input is at most 68 KB: 32 plain input channels take tiles of 2
-// lines.  16 crops of 32^3, 16 -> 16: 26 us, 59 by k_conv.
+// voxels, 32 on lines of 64 (from 16 also of 32), 48 on lines of 32 (the widths those layers
+// have at 128^3 and on 32^3 crops); the staged input is at most 68 KB: 32 plain input channels
+// take tiles of 2 lines.  16 crops of 32^3, 16 -> 16: 26 us, 59 by k_conv.
 bool conv_tiled(const Dims &g, const bf16_t *in, int cin, int cout, const bf16_t *wt, int kpad,
                 const float *bias, const bf16_t *add, const bf16_t *mask, int relu, bf16_t *out,
                 bool up, hipStream_t st) {

@@ -53,7 +53,8 @@ __device__ __forceinline__ void block_partials(double (&p)[ND], double *__restri
 enum Gate : int { GATE_NOT_DONE = 0, GATE_CONV_ALL = 1 };
 
 template <int NV, int OP>
-__global__ __launch_bounds__(kBlock) void k_vec(int64_t n, int64_t chunk, double *__restrict__ p, double *__restrict__ s,
+__global__ __launch_bounds__(kBlock) void k_vec(int64_t n, int64_t chunk, double *__restrict__ p,
+                                                double *__restrict__ s,
                                                 double *__restrict__ r,
                                                 const double *__restrict__ r0,
                                                 const double *__restrict__ v,
