@@ -1353,11 +1353,23 @@ int level_dims_ok(const xh_unet_s *U, int d, int h, int w) {
     return d > 0 && h > 0 && w > 0 && d % f == 0 && h % f == 0 && w % f == 0;
 }
 
+// 0: the upsampled decoder inputs are written out for the forward pass
+int g_fuse_up = 1;
+
+// the upsampled decoder inputs, which only a forward pass without the fused upsampling writes
+int ensure_up(xh_unet_s *U, Work &W) {
+    for (int l = 0; l + 1 < U->L && !g_fuse_up; ++l)
+        if (W.u[l] == nullptr)
+            if (const int rc = dalloc_t(U, &W.u[l], W.g[l].vox() * U->ch[l + 1], W.owned))
+                return rc;
+    return 0;
+}
+
 int get_work(xh_unet_s *U, int n, int d, int h, int w, bool grads, Work **out) {
     for (auto &p : U->work)
         if (p->n == n && p->d == d && p->h == h && p->w == w && (p->grads || !grads)) {
             *out = p.get();
-            return 0;
+            return ensure_up(U, *p);
         }
     auto W = std::make_unique<Work>();
     W->n = n;
@@ -1373,18 +1385,17 @@ int get_work(xh_unet_s *U, int n, int d, int h, int w, bool grads, Work **out) {
         const int64_t V = g.vox();
         const int cl = U->ch[l], cinl = l == 0 ? 1 : U->ch[l - 1];
         const int cup = l + 1 < L ? U->ch[l + 1] : 0;
-        bf16_t *p_in, *p_a, *p_s, *p_u = nullptr, *p_d = nullptr, *p_h = nullptr;
+        bf16_t *p_in, *p_a, *p_s, *p_d = nullptr, *p_h = nullptr;
         if ((rc = dalloc_t(U, &p_in, V * cinl, W->owned)) || (rc = dalloc_t(U, &p_a, V * cl, W->owned)) ||
             (rc = dalloc_t(U, &p_s, V * cl, W->owned)))
             return rc;
         if (l + 1 < L)
-            if ((rc = dalloc_t(U, &p_u, V * cup, W->owned)) || (rc = dalloc_t(U, &p_d, V * cl, W->owned)) ||
-                (rc = dalloc_t(U, &p_h, V * cl, W->owned)))
+            if ((rc = dalloc_t(U, &p_d, V * cl, W->owned)) || (rc = dalloc_t(U, &p_h, V * cl, W->owned)))
                 return rc;
         W->in.push_back(p_in);
         W->a.push_back(p_a);
         W->s.push_back(p_s);
-        W->u.push_back(p_u);
+        W->u.push_back(nullptr);
         W->dd.push_back(p_d);
         W->hh.push_back(p_h);
         bf16_t *g_in = nullptr, *g_a = nullptr, *g_s = nullptr, *g_u = nullptr, *g_d = nullptr,
@@ -1411,7 +1422,7 @@ int get_work(xh_unet_s *U, int n, int d, int h, int w, bool grads, Work **out) {
         return rc;
     *out = W.get();
     U->work.push_back(std::move(W));
-    return 0;
+    return ensure_up(U, **out);
 }
 
 // MT tiles of 16 voxels per wave: CT * MT = 4 accumulator tiles
@@ -1616,9 +1627,6 @@ void conv_wgrad(xh_unet_s *U, const Conv &c, const Dims &g, const bf16_t *in, co
 #undef XH_WG
     reduce_parts(U, nchunk, len, len, c.gw);
 }
-
-// 0: the upsampled decoder inputs are written out for the forward pass
-int g_fuse_up = 1;
 
 // the decoder's first convolution reads the coarse tensor through the fused upsampling
 void forward(xh_unet_s *U, Work &W, bool infer = false) {

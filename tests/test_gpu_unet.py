@@ -160,6 +160,29 @@ def test_fused_upsampling_inference_is_identical(gpu):
         assert np.array_equal(outs[0], outs[1])
 
 
+def test_upsampled_inputs_are_made_on_demand(gpu):
+    # buffers of one shape first used with the fused upsampling, which needs no upsampled
+    # tensors, then without it: inference and gradients are the same
+    X = gpu
+    net, n, nv = X.UNet((16, 32, 48), seed=4), 16, 2
+    rng = np.random.default_rng(1)
+    b = X.DeviceArray.from_host(rng.standard_normal(n ** 3 * nv))
+    x, t = (rng.standard_normal((nv, n, n, n)).astype(np.float32) for _ in range(2))
+    outs = []
+    try:
+        for fuse in (1, 0, 1):
+            X.set_option("unet_fuse_up", fuse)
+            o = X.DeviceArray(n ** 3 * nv)
+            net.infer(n, n, n, nv, b, o)
+            outs.append((o.to_host(),) + net.loss_grad(x, t)[1:])
+    finally:
+        X.set_option("unet_fuse_up", 1)
+    assert np.abs(outs[0][0]).max() > 0
+    for q in outs[1:]:
+        for u, v in zip(outs[0], q):
+            assert np.array_equal(u, v)
+
+
 def test_tiled_convolution_is_identical(gpu):
     # forward convolutions with 16 or 32 output channels on volumes with w % 64 == h % 4 ==
     # d % 2 == 0 (48 channels: w % 32 == 0) read their input from LDS-staged tiles (plain,
