@@ -2278,7 +2278,7 @@ struct xh_batch_s {
     unsigned long long *d_t0 = nullptr;
     BatchBarrier *d_bar = nullptr; // grid barriers of the single-launch solve
     // Work lists: of the operations without dots, by the layout that xh_batch_autotune or the
-    // caller picks, and of the operations with dots, by kDotPasses and kDotRhsPerLane.  The
+    // caller picks, and of the operations with dots, by each system's size (dot_passes).  The
     // active items are rebuilt after every iteration.
     BatchList vec, dot;
     int nvec = 0, ndot = 0;
@@ -2301,34 +2301,42 @@ namespace {
 
 int nv_class(int nv) { return nv == 1 ? 0 : nv == 2 ? 1 : nv == 4 ? 2 : nv == 8 ? 3 : 4; }
 
-// Layout of the operations with dots, per nv class 1, 2, 4, 8, 16.  An item's rows and their
-// split over lanes are the grouping of its dot partials, so this layout is a constant: the
-// same systems give the same bits whatever layout the other operations run with, and
-// whatever a tuning run measured.
+// Layout of the operations with dots.  An item's rows and their split over lanes are the
+// grouping of its dot partials, so this layout depends on the system's rows and nv only: the
+// same system gives the same bits whatever layout the other operations run with, whatever a
+// tuning run measured and whichever systems it is solved with.  Passes per item, by nv class
+// 1, 2, 4, 8, 16: the most, as tuning runs picked for large systems, but at least 64 items
+// per system while it has the rows (17 systems of 8^3 to 25^3: 5.4 ms per solve with the
+// most passes, 5.07 so).
 constexpr int kDotPasses[5] = {4, 4, 8, 4, 8};
-constexpr int kDotRhsPerLane[5] = {1, 2, 2, 2, 2};
+int dot_rhs_per_lane(int nv) { return nv >= 2 ? 2 : 1; }
+int dot_passes(int64_t n, int nv) {
+    const int64_t rows = kBlock * dot_rhs_per_lane(nv) / nv; // per pass
+    return (int)std::max<int64_t>(1, std::min<int64_t>(kDotPasses[nv_class(nv)],
+                                                       (n + rows - 1) / rows / 64));
+}
 
-// work items of the systems whose nv class is in `mask`, passes[class] passes of
-// 256 * w[class] / nv rows each; start/count (nullable): of each system
-void build_items(const xh_batch_s *B, unsigned mask, const int *passes, const int *w,
-                 std::vector<BatchItem> &items, std::vector<int> *start,
-                 std::vector<int> *count) {
+// work items of the systems whose nv class is in `mask`: passes of 256 * w / nv rows each, by
+// the batch's layout (tile_passes, tile_w) or that of the operations with dots; start/count
+// (nullable): of each system
+void build_items(const xh_batch_s *B, unsigned mask, bool dots, std::vector<BatchItem> &items,
+                 std::vector<int> *start, std::vector<int> *count) {
     items.clear();
     if (start) {
         start->assign(B->nsys, 0);
         count->assign(B->nsys, 0);
     }
     for (int s = 0; s < B->nsys; ++s) {
-        const int c = nv_class(B->nv[s]);
+        const int nv = B->nv[s], c = nv_class(nv);
         if (!(mask & (1u << c)))
             continue;
-        const int wpl = B->nv[s] >= 2 ? w[c] : 1;
-        const int64_t tile = (int64_t)passes[c] * (kBlock * wpl / B->nv[s]);
+        const int wpl = dots ? dot_rhs_per_lane(nv) : nv >= 2 ? B->tile_w[c] : 1;
+        const int64_t tile = (int64_t)(dots ? dot_passes(B->n[s], nv) : B->tile_passes[c]) *
+                             (kBlock * wpl / nv);
         if (start)
             (*start)[s] = (int)items.size();
         for (int64_t r0 = 0; r0 < B->n[s]; r0 += tile)
-            items.push_back({s, B->nv[s], r0, std::min(B->n[s], r0 + tile), wpl,
-                             (int32_t)items.size()});
+            items.push_back({s, nv, r0, std::min(B->n[s], r0 + tile), wpl, (int32_t)items.size()});
         if (count)
             (*count)[s] = (int)items.size() - (*start)[s];
     }
@@ -2342,11 +2350,11 @@ void free_list(BatchList &l) {
     l = BatchList();
 }
 
-// builds a list of all systems with the given layout and uploads it; on failure `out` stays
-int upload_list(xh_batch_s *B, const int *passes, const int *w, BatchList &out, int &n) {
+// builds one of the lists over all systems and uploads it; on failure `out` stays
+int upload_list(xh_batch_s *B, bool dots, BatchList &out, int &n) {
     std::vector<BatchItem> items;
     std::vector<int> start, count;
-    build_items(B, 0x1f, passes, w, items, &start, &count);
+    build_items(B, 0x1f, dots, items, &start, &count);
     BatchList l;
     auto up = [&]() -> int {
         size_t acc = 0;
@@ -2372,7 +2380,7 @@ int upload_list(xh_batch_s *B, const int *passes, const int *w, BatchList &out, 
 
 // the list of the operations without dots, after a change of its layout
 int upload_items(xh_batch_s *B) {
-    const int rc = upload_list(B, B->tile_passes, B->tile_w, B->vec, B->nvec);
+    const int rc = upload_list(B, false, B->vec, B->nvec);
     if (B->gexec) {
         (void)hipGraphExecDestroy(B->gexec);
         (void)hipGraphDestroy(B->graph);
@@ -2658,7 +2666,7 @@ extern "C" int xh_batch_create(int nsys, const int64_t *nrows, const int32_t *nv
     if (e != hipSuccess)
         return bail(fail(XH_EHIP, std::string("xh_batch_create: ") + hipGetErrorString(e)));
     B->wall_khz = khz;
-    if ((rc = upload_list(B, kDotPasses, kDotRhsPerLane, B->dot, B->ndot)) ||
+    if ((rc = upload_list(B, true, B->dot, B->ndot)) ||
         (rc = dmalloc(&B->partials, (size_t)B->ndot * kBatchPart, acc)) || (rc = upload_items(B)))
         return bail(rc);
     *out = B;
@@ -2846,7 +2854,7 @@ extern "C" int xh_batch_autotune(xh_batch B, int reps, int32_t *tile_passes) {
             const int p = cand[cw % 6], wl = 1 + cw / 6;
             B->tile_passes[c] = p;
             B->tile_w[c] = wl;
-            build_items(B, 1u << c, B->tile_passes, B->tile_w, items, nullptr, nullptr);
+            build_items(B, 1u << c, false, items, nullptr, nullptr);
             (void)hipFree(d_items);
             size_t acc = 0;
             if ((rc = dmalloc(&d_items, items.size(), acc)))

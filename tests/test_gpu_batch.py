@@ -181,10 +181,10 @@ def test_batch_two_rhs_per_lane_layout(gpu, O, persistent):
 def test_batch_bits_do_not_depend_on_the_layout(gpu, method, precond):
     # the operations with dots walk a list fixed by each system's size and RHS count, so the
     # iterates are the same bits in every layout, set or tuned (two tunings may pick two
-    # layouts).  Every system has several items of several passes in each layout, or is
-    # smaller than one item.
+    # layouts).  The systems have one to several passes per item in that list, several items
+    # or one in the others.
     X = gpu
-    sizes, nvs = (17, 14, 13, 12, 11, 5), (1, 2, 4, 8, 16, 4)
+    sizes, nvs = (40, 26, 27, 12, 11, 5), (1, 2, 4, 8, 16, 4)
     sy = systems(X, sizes, seed=90, sigma=1.0 if precond else 0.0)
     B, _ = run_batch(X, sy, nvs, params(X, method, precond))
     ref = [(B.x(s), B.stats(s)["iters"]) for s in range(len(sizes))]
