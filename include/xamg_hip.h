@@ -160,8 +160,9 @@ int xh_spmv_schedule(int64_t nrows, int64_t nnz, int64_t fold, int prec, int nv,
  * 12 or more entries, e.g. 27-point operators, the row-parallel kernel reads 1-byte
  * neighbour codes instead of columns where they are the faster ones, for more than 4
  * right-hand sides when the launch's matrix, x and y are at least "spmv_codes_min_bytes"
- * together (default 200 MB), and the fp64 SpMMs with dot partials for 16 or 32
- * right-hand sides run the sweep where its work items fill the chip; 0 neither),
+ * together (default 200 MB), and large SpMMs run the sweep where its work items fill the
+ * chip: with dot partials in fp64 for 16 or 32 right-hand sides, products and residuals for
+ * 32 in fp64 and 64 in fp32; 0 neither),
  * "spmv_grid_items" (default 2048),
  * "cheb_fuse_zero" (0/1, default 1: a Chebyshev smoother from a zero x runs its first two
  * steps as one SpMV that gathers b and forms the first step's values per entry,

@@ -992,30 +992,39 @@ bool takes_codes(const Mat &A, SpmvOp op, int nv) {
            A.nnz * (sv + si) + 2 * A.nrows * nv * sv >= g_tune.codes_min_bytes;
 }
 
-// Whether op on A runs as the LDS-window line sweep (k_spmv_sweep).  By default only the fp64
-// SpMMs with dot partials of a long-row operator, with 16 or 32 right-hand sides, and only
-// when the launch's work items (tile of lines x segment) fill at least 4/5 of the 2048
-// workgroups the chip holds: a workgroup stages its own window, so with fewer items the
-// chip idles and with a few more than 2048 half of it waits for second items.  27-point
-// operators, DOT1 + DOT3 in us, sweep / row-parallel (columns), by that share:
+// Whether op on A runs as the LDS-window line sweep (k_spmv_sweep).  By default only for
+// long-row operators, and of those first the fp64 SpMMs with dot partials, with 16 or 32
+// right-hand sides, when the launch's work items (tile of lines x segment) fill at least 4/5
+// of the 2048 workgroups the chip holds: a workgroup stages its own window, so with fewer
+// items the chip idles and with a few more than 2048 half of it waits for second items.
+// 27-point operators, DOT1 + DOT3 in us, sweep / row-parallel (columns), by that share:
 // 32 right-hand sides 0.52 (92^3) 728 / 641, 0.57 (112^3) 1171 / 1123, 0.73 (151x190x122)
 // 2791 / 2774, 0.81 (86x101x125) 903 / 879, 0.84 (96^3) 692 / 714, 0.97 (164x87x72) 802 / 850,
 // 1.0 (128^3) 1504 / 1642; 16: 0.60 (152x110x87) 714 / 724, 0.81 (156x137x92) 960 / 973,
 // 0.86 (131x79x174) 845 / 886, 0.97 (184x163x74) 1027 / 1089, 1.0 (128^3) 908 / 1004.  With 8
 // the row-parallel kernel is the faster one or even at every share (0.92 and 0.99: 1183 /
-// 1099, 1235 / 1238), with 64 it is by 10 to 20 % (tiles of 8 rows, so more halo); y = A x at
-// 96^3 in fp32: 194 against 128.
+// 1099, 1235 / 1238), with 64 it is by 10 to 20 % (tiles of 8 rows, so more halo).
+// Second, products and residuals where 16 lanes own a row (tiles of 16 lines): in fp64, 32
+// right-hand sides, from 9/10 of the workgroups on (y = A x, 0.63 (150x110x90) 529 / 501, 0.84
+// (96^3) 296 / 295, 0.97 (164x87x72) 347 / 353, 0.99 (104^3) 365 / 386, 1.0 (128^3) 667 / 733); in
+// fp32, 64, with at least 1700 items (968 (88^3) 219 / 170, 1664 (86x101x125) 353 / 352, 1728
+// (96^3) 265 / 276, 2352 (112^3) 431 / 455, 2048 (128^3) 596 / 690).  Others are even at best
+// (128^3, nv = 16, fp64 412 / 431, fp32 233 / 237; 120^3 388 / 348, 202 / 190).
 bool takes_sweep(const Mat &A, SpmvOp op, int nv) {
     if (A.idx == IDX_U8 || op == OP_OFFBLOCK || op == OP_PROLONG32 || op == OP_CHEBZ ||
         op == OP_CHEBR || A.gcode == nullptr || A.row_ind != nullptr || g_tune.grid_enable == 0)
         return false;
     if (g_tune.grid_enable == 1)
         return true;
-    if (A.prec != F64 || (nv != 16 && nv != 32) || A.nnz < kGridMinRowNnz * A.nrows ||
-        !(op == OP_DOT1 || op == OP_DOT3 || op == OP_RDOT4 || op == OP_RESID0))
+    const bool dots = op == OP_DOT1 || op == OP_DOT3 || op == OP_RDOT4 || op == OP_RESID0;
+    const int W = A.prec == F64 ? 2 : 4;
+    if (A.nnz < kGridMinRowNnz * A.nrows ||
+        !(dots || op == OP_SET || op == OP_ADD || op == OP_RESID) ||
+        !(nv == 16 * W || (dots && A.prec == F64 && nv == 16)))
         return false;
-    const GridLaunch G = grid_plan(A.gx, A.gy, A.gz, kBlock / (nv / 2), g_tune.grid_dot_groups);
-    return 5 * (int64_t)G.g.nitems >= 4 * (int64_t)G.g.ipw * 2048;
+    const GridLaunch G = grid_plan(A.gx, A.gy, A.gz, kBlock / (nv / W), g_tune.grid_dot_groups);
+    const int64_t items = G.g.nitems, places = (int64_t)G.g.ipw * 2048;
+    return dots ? 5 * items >= 4 * places : A.prec == F64 ? 10 * items >= 9 * places : items >= 1700;
 }
 
 namespace {

@@ -169,6 +169,39 @@ def test_sweep_by_filled_workgroups(gpu, dims, nv, want):
     assert (np.abs(x - x0).reshape(n, nv).max(0) / np.abs(x0).reshape(n, nv).max(0)).max() <= 1e-6
 
 
+@pytest.mark.parametrize("mg_prec,nv,dims,want", [
+    (0, 32, (64, 48, 40), True),   # 1920 of 2048 workgroups
+    (0, 32, (64, 40, 44), False),  # 1760
+    (0, 32, (64, 44, 48), False),  # 2112: two for some
+    (2, 64, (64, 40, 44), True), (2, 64, (64, 40, 36), False),
+    (0, 64, (64, 48, 40), False), (0, 16, (64, 48, 40), False), (2, 32, (64, 48, 40), False)])
+def test_sweep_residuals_by_filled_workgroups(gpu, mg_prec, nv, dims, want):
+    # residuals of a V-cycle in the default mode (segments of 4 rows, as above): the sweep for
+    # 16 lanes per row where its work items fill the chip, with the bits of the row kernel
+    X = gpu
+    row, col, val = X.q1fem27(*dims)[:3]
+    n = len(row) - 1
+    levels = X.Amg(row, col, val, agg_num_levels=2, num_paths=2, coarse_size=500).export()
+    prm = X.default_params(method="MergedPBiCGStab", smoother="Jacobi", sweeps=2, mg_prec=mg_prec)
+    S = X.Solver(X.Hier(levels), prm, nv)
+    db, dx = X.DeviceArray.from_host(X.rhs_uniform(5, n, nv)), X.DeviceArray(n * nv)
+    out = []
+    try:
+        X.set_option("spmv_grid_min_seg", 4)
+        dx.zero()
+        names = {k["kernel"] for k in S.profile(db, dx, 1) if k["level"] == 0}
+        for ge in (2, 0):
+            X.set_option("spmv_grid_enable", ge)
+            S.precond_apply(db, dx)
+            out.append(dx.to_host())
+    finally:
+        X.set_option("spmv_grid_enable", 2)
+        X.set_option("spmv_grid_min_seg", 32)
+    t = "float" if mg_prec else "double"
+    assert (f"k_spmv_sweep<{t},{nv},OP_RESID>" in names) == want, names
+    assert np.array_equal(*out)
+
+
 def test_no_grid_view_for_partial_grids(gpu):
     X = gpu
     row, col, val = X.cube(8, 6, 5)
